@@ -205,6 +205,40 @@ __device__ __forceinline__ double spherical_cap(double h, double r) {
     return PI_D * h * h / 3.0 * (3.0 * r - h);
 }
 
+// The terms particle xi takes from the void of the slice [lo, hi), in the
+// reference's order: at most two (the lower and the upper boundary).
+// Returns how many.
+__device__ __forceinline__ int slice_terms(const double4 xi, double lo, double hi, double& t0,
+                                           double& t1) {
+    const double zc = xi.z, r = xi.w;
+    const double zl = zc - r, zh = zc + r;
+    // Entirely above or below the slice: no condition holds (at zl == hi the
+    // cap is zero).
+    if (r >= 0.0 && (zl >= hi || zh < lo)) return 0;
+    const double V_sphere = 4.0 / 3.0 * PI_D * r * r * r;
+    if (lo <= zl && zh <= hi) {
+        t0 = V_sphere;
+        return 1;
+    }
+    double t[2] = {0.0, 0.0};
+    bool low = true, up = true;
+    if (lo >= zc && lo <= zh)
+        t[0] = spherical_cap(zh - lo, r);
+    else if (lo < zc && lo > zl)
+        t[0] = V_sphere + spherical_cap(lo - zl, r);
+    else
+        low = false;
+    if (hi <= zc && hi >= zl)
+        t[1] = spherical_cap(hi - zl, r);
+    else if (hi > zc && hi < zh)
+        t[1] = V_sphere + spherical_cap(zh - hi, r);
+    else
+        up = false;
+    t0 = low ? t[0] : t[1];
+    t1 = t[1];
+    return (low ? 1 : 0) + (up ? 1 : 0);
+}
+
 // One work-item per slice, the particles in index order (the reference's
 // serial subtraction per slice).
 __global__ __launch_bounds__(64) void k_porosity(const double4* __restrict__ x, uint32_t np,
@@ -217,25 +251,97 @@ __global__ __launch_bounds__(64) void k_porosity(const double4* __restrict__ x, 
     const double lo = iz * h_slice;
     const double hi = lo + h_slice;
     for (uint32_t i = 0; i < np; ++i) {
-        const double4 xi = x[i];
-        const double zc = xi.z, r = xi.w;
-        const double zl = zc - r, zh = zc + r;
-        const double V_sphere = 4.0 / 3.0 * PI_D * r * r * r;
-        if (lo <= zl && zh <= hi) {
-            V_void -= V_sphere;
-        } else {
-            if (lo >= zc && lo <= zh)
-                V_void -= spherical_cap(zh - lo, r);
-            else if (lo < zc && lo > zl)
-                V_void -= V_sphere + spherical_cap(lo - zl, r);
-            if (hi <= zc && hi >= zl)
-                V_void -= spherical_cap(hi - zl, r);
-            else if (hi > zc && hi < zh)
-                V_void -= V_sphere + spherical_cap(zh - hi, r);
-        }
+        double t0, t1;
+        const int n = slice_terms(x[i], lo, hi, t0, t1);
+        if (n > 0) V_void -= t0;
+        if (n > 1) V_void -= t1;
     }
     z_pos[iz] = lo + 0.5 * h_slice;
     porosity[iz] = V_void / V_slice;
+}
+
+// One workgroup per slice.  The subtraction is a serial chain in particle
+// order (each slice's result is rounded term by term), so the terms are
+// formed apart from it: the wavefronts after the first evaluate a tile of
+// particles each round and leave the terms in LDS, compacted in particle
+// order, while the first work-item subtracts the tile before, sixteen terms
+// read ahead of the adds.  Bound by the rounds (about 1.8 us for 960
+// particles) and, where a slice holds many particles, by the chain of adds.
+// One work-item per slice took 0.23 us a particle for any number of slices:
+// 100,003 particles in 10 slices 23.6 ms there, 0.20 ms here; 5,000 in 10
+// slices 1.19 ms and 0.02 ms.
+constexpr uint32_t PW = 16;                // wavefronts
+constexpr uint32_t PTILE = 64 * (PW - 1);  // particles per round
+__global__ __launch_bounds__(64 * PW) void k_porosity_slice(const double4* __restrict__ x,
+                                                            uint32_t np, double h_slice,
+                                                            double V_slice,
+                                                            double* __restrict__ z_pos,
+                                                            double* __restrict__ porosity) {
+    __shared__ __align__(16) double term[2 * PTILE + 32];
+    __shared__ uint32_t cnt[2][PW];
+    const int iz = (int)blockIdx.x;
+    const double lo = iz * h_slice;
+    const double hi = lo + h_slice;
+    const uint32_t wave = threadIdx.x / 64u, lane = threadIdx.x % 64u;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t rounds = (np + PTILE - 1) / PTILE;
+    double V_void = V_slice;
+    uint32_t i = threadIdx.x - 64u;  // the particle of this round (wave > 0)
+    double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (wave > 0 && i < np) xi = x[i];
+    // Round r evaluates tile r and subtracts tile r - 1.
+    for (uint32_t r = 0; r <= rounds; ++r) {
+        const uint32_t h = r & 1u;
+        double t0 = 0.0, t1 = 0.0;
+        int n = 0;
+        uint64_t b0 = 0, b1 = 0;
+        if (wave > 0) {
+            if (i < np) n = slice_terms(xi, lo, hi, t0, t1);
+            b0 = __ballot(n > 0);
+            b1 = __ballot(n > 1);
+            if (lane == 0) cnt[h][wave] = (uint32_t)(__popcll(b0) + __popcll(b1));
+            i += PTILE;
+            if (i < np) xi = x[i];
+        } else if (threadIdx.x == 0 && r > 0) {
+            uint32_t m = 0;
+            for (uint32_t w = 1; w < PW; ++w) m += cnt[h ^ 1u][w];
+            double a[16], b[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) a[k] = term[k];
+            uint32_t j = 0;
+            for (; j + 32 <= m; j += 32) {
+#pragma unroll
+                for (int k = 0; k < 16; ++k) b[k] = term[j + 16 + k];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) V_void -= a[k];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) a[k] = term[j + 32 + k];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) V_void -= b[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) b[k] = term[j + 16 + k];
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+                if (j + k < m) V_void -= a[k];
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+                if (j + 16 + k < m) V_void -= b[k];
+        }
+        __syncthreads();
+        if (n > 0) {
+            uint32_t off = 0;
+            for (uint32_t w = 1; w < wave; ++w) off += cnt[h][w];
+            off += (uint32_t)(__popcll(b0 & below) + __popcll(b1 & below));
+            term[off] = t0;
+            if (n > 1) term[off + 1] = t1;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        z_pos[iz] = lo + 0.5 * h_slice;
+        porosity[iz] = V_void / V_slice;
+    }
 }
 
 }  // namespace
@@ -281,8 +387,16 @@ hipError_t launch_overlaps_grid(const double4* x, const double4* vel, uint32_t n
 
 hipError_t launch_porosity(const double4* x, uint32_t np, int z_slices, double h_slice,
                            double V_slice, double* z_pos, double* porosity, hipStream_t s) {
-    hipLaunchKernelGGL(k_porosity, dim3((z_slices + 63) / 64), dim3(64), 0, s, x, np, z_slices,
-                       h_slice, V_slice, z_pos, porosity);
+    // A workgroup per slice pays while the chip holds them in few rounds (512
+    // at a time).  5,000 particles: 0.36 ms against 1.11 at 8,192 slices, the
+    // same at 32,768; 500 particles: 0.14 against 0.16 at 8,192; 50 particles:
+    // equal at 1,000, 0.09 against 0.06 at 8,192.
+    if (z_slices <= 1024 || (z_slices <= 8192 && (uint32_t)z_slices / 16u <= np))
+        hipLaunchKernelGGL(k_porosity_slice, dim3(z_slices), dim3(64 * PW), 0, s, x, np, h_slice,
+                           V_slice, z_pos, porosity);
+    else
+        hipLaunchKernelGGL(k_porosity, dim3((z_slices + 63) / 64), dim3(64), 0, s, x, np,
+                           z_slices, h_slice, V_slice, z_pos, porosity);
     return hipGetLastError();
 }
 

@@ -1,0 +1,46 @@
+"""The readers' and contact kernels at the sizes where their tiling can go
+wrong (tile edges, remainders, dispatch lines), bit for bit against the
+oracle."""
+
+import numpy
+import pytest
+
+import oracle
+from sphere_amd import engine, scenes
+from sphere_amd.sim import sim
+
+pytestmark = pytest.mark.gpu
+
+
+def _cloud(n, seed, r=(0.008, 0.012), last=None, L=(0.5, 0.5, 0.5)):
+    """n spheres at random places of a box (they may overlap)."""
+    rng = numpy.random.default_rng(seed)
+    s = sim(np=n, sid="cloud-%d" % n)
+    s.radius = rng.uniform(r[0], r[1], n)
+    if last is not None:
+        s.radius[-1] = last
+    s.x = rng.uniform(0.02, 0.48, (n, 3))
+    s.defaultParams(rho=2600.0, k_n=1.0e6, k_t=1.0e6)
+    s.normalBoundariesXY()
+    s.defineWorldBoundaries(L=list(L))
+    dt = scenes.dt_rule(float(s.radius.min()), 2600.0, 1.0e6)
+    s.time_dt[0] = dt
+    s.time_current[0] = 0.0
+    s.time_total[0] = dt * 1000
+    s.time_file_dt[0] = dt * 1000
+    return s
+
+
+# A round of the slice kernel takes 960 particles; a thin slice takes two
+# terms from most of them; beyond 8,192 slices (1,024 in a small simulation)
+# each work-item takes a slice.
+@pytest.mark.parametrize("n,slices,last", [
+    (1, 1, None), (64, 3, None), (959, 7, None), (960, 7, None), (961, 20, None),
+    (2881, 1, None), (1920, 60, 1.0e-4), (700, 8192, 1.0e-5), (700, 8193, 1.0e-5),
+    (20, 1024, 1.0e-5), (20, 1025, 1.0e-5)])
+def test_porosity_tile_edges(n, slices, last):
+    image = _cloud(n, 7 + n, last=last).tobytes()
+    with engine.Context(image) as ctx:
+        za, pa = ctx.porosity(slices)
+    zb, pb = oracle.Oracle(image).porosity(slices)
+    assert numpy.array_equal(za, zb) and numpy.array_equal(pa, pb)
