@@ -82,7 +82,8 @@ struct AdjState {
     const double4* Ldt_in;   // ntot x NC: of the displacements the step writes
     double4* Ldt_out;        // ntot x NC: of the displacements the step read, at the
                              //   slots occupied in prev_rows
-    double* part;            // per adjoint workgroup: ADJ_NPART partial sums
+    double* part;            // ADJ_NPART partial sums of every adjoint workgroup,
+                             //   quantity by quantity
     double* gparam;          // nsim x ADJ_NPARAM, accumulated over the steps
     double* wall;            // total walls x ADJ_WALL reverse state
     uint32_t* asym;          // contacts missing from their partner's row

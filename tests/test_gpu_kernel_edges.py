@@ -9,6 +9,8 @@ import oracle
 from sphere_amd import engine, scenes
 from sphere_amd.sim import sim
 
+from . import cases
+
 pytestmark = pytest.mark.gpu
 
 
@@ -44,3 +46,23 @@ def test_porosity_tile_edges(n, slices, last):
         za, pa = ctx.porosity(slices)
     zb, pb = oracle.Oracle(image).porosity(slices)
     assert numpy.array_equal(za, zb) and numpy.array_equal(pa, pb)
+
+
+# The reverse pass's sums run over 64-particle workgroups in 256 shares:
+# 256 workgroups exactly, one more (np rounds up to 256), and a bonded bed.
+@pytest.mark.parametrize("n,bond_frac", [(16384, 0.0), (16385, 0.0), (17000, 0.05)])
+def test_adjoint_sums_over_many_workgroups(n, bond_frac):
+    s = cases.lattice_bed(n, 5, 0.01, 0.1, bond_frac=bond_frac)
+    image, steps = s.tobytes(), 3
+    rng = numpy.random.default_rng(n)
+    c = rng.standard_normal((n, 3))
+    with engine.Context(image) as ctx:
+        g = ctx.adjoint(steps, None, c, None)
+    for name in ("k_n", "gamma_n", "gamma_wn"):
+        t = oracle.TangentOracle(image)
+        t.seed_param(name, 1.0)
+        t.step(steps)
+        want = float(numpy.sum(c * t.tangent("vel")))
+        # Forward and reverse mode agree to rounding of sums over n terms of
+        # either sign: 1e-6 of the result, as the other tangent checks.
+        assert abs(g[name] - want) <= 1e-6 * abs(want), (name, g[name], want)
