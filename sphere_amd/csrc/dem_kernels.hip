@@ -886,8 +886,8 @@ __device__ __forceinline__ void tape_start(const DevArrays& a, CParams& p, uint3
         }
 }
 
-// CM is the contact model (1, 2 or 3); one instantiation per model keeps
-// only that model's registers live.
+// CM is the contact model (2 or 3, or 0 for no particle contacts); one
+// instantiation per model keeps only that model's registers live.
 template <int CM>
 __global__ __launch_bounds__(BLOCK, CONTACT_MIN_BLOCKS) void k_contact(const DevArrays a) {
     __shared__ uint32_t srow[BLOCK * ROW_STRIDE];
@@ -904,7 +904,7 @@ __global__ __launch_bounds__(BLOCK, CONTACT_MIN_BLOCKS) void k_contact(const Dev
     const double Lz = grid_Lz(p, a);
     const double4 vel_a = S.v[S.at(ia)];
     const double4 av_a = S.w[S.at(ia)];
-    const d3 angvel_a = xyz(av_a);
+    [[maybe_unused]] const d3 angvel_a = xyz(av_a);
     tape_start(a, p, ia, ia_orig, xa, vel_a, av_a, true);
     Acc A;
     A.F = mk3(0.0, 0.0, 0.0);
@@ -1065,40 +1065,6 @@ __global__ __launch_bounds__(BLOCK, CONTACT_MIN_BLOCKS) void k_contact(const Dev
         if (a.tape_rows)
             for (int i = 0; i < NC; ++i)
                 a.tape_rows[(size_t)ia_orig * NC + i] = word_to_orig(a, row[i]);
-    } else if constexpr (CM == 1) {
-        // findAndProcessContactsInCell, src/contactsearch.cuh:91-186.
-        for (int dz = -1; dz < 2; ++dz)
-            for (int dy = -1; dy < 2; ++dy)
-                for (int dx = -1; dx < 2; ++dx) {
-                    int tx = gx + dx, ty = gy + dy;
-                    const int tz = gz + dz;
-                    const int code = find_dist_mod(p, tx, ty, tz);
-                    if (code < 0) continue;
-                    const uint32_t cell = p.cell_base + (uint32_t)tx + (uint32_t)ty * p.num[0] +
-                                          (p.num[0] * p.num[1]) * (uint32_t)tz;
-                    const uint32_t start = a.cell_start[cell];
-                    if (start == 0xffffffffu) continue;
-                    const uint32_t end = a.cell_end[cell];
-                    const d3 dm = shift_of(p, (uint32_t)code);
-                    for (uint32_t ib = start; ib < end; ++ib) {
-                        if (ib == ia) continue;
-                        const uint32_t jb = S.at(ib);
-                        const double4 xb = S.x[jb];
-                        const double rb = xb.w;
-                        const double kappa = p.kappa;
-                        d3 xab = mk3(xa.x - xb.x, xa.y - xb.y, xa.z - xb.z);
-                        xab += dm;
-                        const double len = length(xab);
-                        const double delta = len - (ra + rb);
-                        if (delta < 0.0) {
-                            contact_linear_viscous(p, A, vel_a, angvel_a, S.v[jb],
-                                                   xyz(S.w[jb]), ra, rb, xab, len,
-                                                   delta, kappa);
-                        } else if (delta < p.db) {
-                            capillary_cohesion_exp(p, A, ra, rb, delta, xab, len, kappa);
-                        }
-                    }
-                }
     }
     walls_and_outputs(p, a, A, xa, vel_a, av_a, Lz, ia_orig, 4);
 }
@@ -2004,6 +1970,162 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
 }
 
 // ---------------------------------------------------------------------------
+// Contact model 1 (no contact history): findAndProcessContactsInCell,
+// src/contactsearch.cuh:91-186, with four lanes per particle.  The overlapping
+// candidates are collected in scan order (in LDS, NC at a time) from the
+// candidate list, or from the 27 cells while the list is rebuilt, has
+// overflowed, or cannot serve (a capillary debonding distance reaches beyond
+// the lists).  Each lane then evaluates one of them and the group adds the
+// contributions in scan order.
+//
+// Bound by the latency of the gather chain.  One lane per particle scanning
+// 27 cells every step took 153 us a launch on a sheared bed of 16,096; this
+// takes 10.
+template <int WG>
+__global__ __launch_bounds__(WG) void k_contact_v(const DevArrays a) {
+    constexpr int LPP = 4;
+    constexpr int PPB = WG / LPP;  // particles per workgroup
+    constexpr int RMAX = NV / LPP;
+    static_assert(NV <= NC, "a list fits the hit buffer");
+    __shared__ uint32_t s_hit[PPB * NC];
+    const LaneGroup<LPP> g;
+    const uint32_t blk = xcd_block(a, blockIdx.x, gridDim.x);
+    const uint32_t ia = blk * PPB + threadIdx.x / LPP;
+    CParams& p = chunk_params(a, blk * PPB / BLOCK);
+    if (ia - p.base >= p.np) return;  // whole groups leave together
+    DevLoop* lp = a.loop + p.sim;
+    const uint32_t ia_orig = a.perm[ia];
+    const SortedReader S(a, lp);
+    const bool lists = p.vl_enabled && !(p.db > 0.0);
+    const bool rebuild = !lists || lp->rebuild[step_slot(lp)] != 0u || lp->force_rebuild != 0u;
+    const uint32_t vcnt = rebuild ? VL_OVERFLOW : a.vcount[ia].x;
+    const uint32_t self = S.stale ? ia_orig : ia;
+    const double4 xa = S.x[self];
+    const double4 vel_a = S.v[self];
+    const double4 av_a = S.w[self];
+    uint2 ev[RMAX];
+    uint2* vrow = a.vlist + (size_t)ia * NV;
+#pragma unroll
+    for (int i = 0; i < RMAX; ++i) {
+        ev[i] = make_uint2(0u, 0u);
+        if (vcnt != VL_OVERFLOW && g.q + LPP * i < vcnt) ev[i] = vrow[g.q + LPP * i];
+    }
+    const double ra = xa.w;
+    const double Lz = grid_Lz(p, a);
+    uint32_t* hit_words = s_hit + (threadIdx.x / LPP) * NC;
+    const uint32_t below = (1u << g.q) - 1u;
+    uint32_t nh = 0;
+    Acc A;
+    A.F = mk3(0.0, 0.0, 0.0);
+    A.T = mk3(0.0, 0.0, 0.0);
+    A.es_dot = 0.0;
+    A.ev_dot = 0.0;
+    A.p = 0.0;
+    // Adds the collected contacts in order and empties the buffer.
+    auto process = [&]() {
+        wave_sync();
+        for (uint32_t r = 0; r < nh; r += LPP) {
+            Acc C;
+            C.F = mk3(0.0, 0.0, 0.0);
+            C.T = mk3(0.0, 0.0, 0.0);
+            C.p = 0.0;
+            if (r + g.q < nh) {
+                const uint32_t wrd = hit_words[r + g.q];
+                const uint32_t jb = S.at(wrd & CW_IDX_MASK);
+                const double4 xb = S.x[jb];
+                const double4 vel_b = S.v[jb];
+                const double4 av_b = S.w[jb];
+                const double rb = xb.w;
+                d3 xab = mk3(xa.x - xb.x, xa.y - xb.y, xa.z - xb.z);
+                xab += shift_of(p, word_code(wrd));
+                const double len = length(xab);
+                const double delta = len - (ra + rb);
+                if (delta < 0.0)
+                    contact_linear_viscous(p, C, vel_a, xyz(av_a), vel_b, xyz(av_b), ra, rb, xab,
+                                           len, delta, p.kappa);
+                else
+                    capillary_cohesion_exp(p, C, ra, rb, delta, xab, len, p.kappa);
+            }
+            // A lane without a contact adds +0.0: the sums start at +0.0
+            // and so are never -0.0, and x + 0.0 = x for every other x.
+            A.F += g.template bc<0>(C.F); A.T += g.template bc<0>(C.T); A.p += g.template bc<0>(C.p);
+            A.F += g.template bc<1>(C.F); A.T += g.template bc<1>(C.T); A.p += g.template bc<1>(C.p);
+            A.F += g.template bc<2>(C.F); A.T += g.template bc<2>(C.T); A.p += g.template bc<2>(C.p);
+            A.F += g.template bc<3>(C.F); A.T += g.template bc<3>(C.T); A.p += g.template bc<3>(C.p);
+        }
+        wave_sync();
+        nh = 0;
+    };
+    auto collect = [&](bool hit, uint32_t word) {
+        const uint32_t hm = g.bits(hit);
+        if (nh + __popc(hm) > (uint32_t)NC) process();
+        if (hit) hit_words[nh + __popc(hm & below)] = word;
+        nh += __popc(hm);
+    };
+    if (vcnt != VL_OVERFLOW) {
+        const uint32_t listed =
+            vcnt > g.q ? ((1u << ((vcnt - g.q + LPP - 1) / LPP)) - 1u) & ((1u << RMAX) - 1u) : 0u;
+        const bool tail = __ballot(listed >> TCHUNK) != 0ull;
+        const uint32_t hits = test_entries<LPP>(p, S, xa, ia, ev, listed, tail);
+#pragma unroll
+        for (int i = 0; i < RMAX; ++i) collect((hits >> i) & 1u, ev[i].y);
+    } else {
+        const bool build = lists && rebuild;
+        uint32_t nl = 0;
+        const int gx = (int)floor((xa.x - p.origo[0]) / (p.L[0] / p.num[0]));
+        const int gy = (int)floor((xa.y - p.origo[1]) / (p.L[1] / p.num[1]));
+        const int gz = (int)floor((xa.z - p.origo[2]) / (Lz / p.num[2]));
+        for (int dz = -1; dz < 2; ++dz)
+            for (int dy = -1; dy < 2; ++dy)
+                for (int dx = -1; dx < 2; ++dx) {
+                    int tx = gx + dx, ty = gy + dy;
+                    const int tz = gz + dz;
+                    const int code = find_dist_mod(p, tx, ty, tz);
+                    if (code < 0) continue;
+                    const uint32_t cell = p.cell_base + (uint32_t)tx + (uint32_t)ty * p.num[0] +
+                                          (p.num[0] * p.num[1]) * (uint32_t)tz;
+                    const uint32_t start = a.cell_start[cell];
+                    if (start == 0xffffffffu) continue;
+                    const uint32_t end = a.cell_end[cell];
+                    const d3 dm = shift_of(p, (uint32_t)code);
+                    const uint32_t celloff = (uint32_t)((dz + 1) * 9 + (dy + 1) * 3 + (dx + 1));
+                    for (uint32_t r = start; r < end; r += LPP) {
+                        const uint32_t ib = r + g.q;
+                        bool hit = false, near = false;
+                        if (ib < end && ib != ia) {
+                            const double4 xb = S.x[S.at(ib)];
+                            d3 xab = mk3(xa.x - xb.x, xa.y - xb.y, xa.z - xb.z);
+                            xab += dm;
+                            const double dd = dot(xab, xab);
+                            const double Sab = ra + xb.w;
+                            if (build) {
+                                const double Sv = Sab + p.vl_skin;
+                                near = dd < Sv * Sv;
+                            }
+                            const double delta = sqrt32(dd) - Sab;
+                            hit = delta < 0.0 || delta < p.db;
+                        }
+                        const uint32_t word = pack_word(ib, (uint32_t)code);
+                        if (build) {
+                            const uint32_t nm = g.bits(near);
+                            const uint32_t pos = nl + __popc(nm & below);
+                            if (near && pos < (uint32_t)NV)
+                                vrow[pos] = make_uint2(ib | (celloff << VL_CELL_SHIFT), word);
+                            nl += __popc(nm);
+                        }
+                        collect(hit, word);
+                    }
+                }
+        if (build && g.q == 0) {
+            a.vcount[ia] = make_uint2(nl <= p.vl_cap ? nl : VL_OVERFLOW, 0u);
+            a.x_build[ia_orig] = xa;
+        }
+    }
+    process();
+    walls_and_outputs(p, a, A, xa, vel_a, av_a, Lz, ia_orig, (int)g.q);
+}
+
+// ---------------------------------------------------------------------------
 // Block tree sum of the reference's `summation` kernel (one element per
 // work-item, then the halving tree, src/integration.cuh:309-341).
 
@@ -2679,7 +2801,7 @@ hipError_t launch_contact(const DevArrays& a, int contactmodel, int lanes, int w
     }
     const dim3 g(a.nchunk);
     if (contactmodel == 1)
-        hipLaunchKernelGGL(k_contact<1>, g, b, 0, s, a);
+        hipLaunchKernelGGL(k_contact_v<BLOCK>, dim3(a.nchunk * 4u), b, 0, s, a);
     else if (contactmodel == 3)
         hipLaunchKernelGGL(k_contact<3>, g, b, 0, s, a);
     else if (contactmodel == 2)

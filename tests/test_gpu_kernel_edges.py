@@ -66,3 +66,34 @@ def test_adjoint_sums_over_many_workgroups(n, bond_frac):
         # Forward and reverse mode agree to rounding of sums over n terms of
         # either sign: 1e-6 of the result, as the other tangent checks.
         assert abs(g[name] - want) <= 1e-6 * abs(want), (name, g[name], want)
+
+
+def _model1(case):
+    if case == "crowded":  # 44 overlaps: more than a list or the hit buffer holds
+        s = cases.crowded_case()
+    elif case == "fcc":
+        s = cases.fcc_case()
+    elif case == "one":
+        s = _cloud(1, 3)
+        s.vel[:, 2] = -1.0
+    else:
+        s = scenes.lattice_box(int(case), seed=4)
+    s.contactmodel[0] = 1
+    return s
+
+
+# Lists, list overflow, a list rebuilt every step (no lists), particles that
+# change cell, one particle, a last wavefront with few groups.
+@pytest.mark.parametrize("case,steps,skin", [
+    ("crowded", 20, None), ("crowded", 5, 0.0), ("fcc", 100, None), ("one", 10, None),
+    ("66", 400, None), ("1025", 300, None), ("1025", 50, 0.0)])
+def test_model1_matches_oracle(case, steps, skin):
+    image = _model1(case).tobytes()
+    ref = oracle.Oracle(image)
+    ref.step(steps)
+    with engine.Context(image) as ctx:
+        if skin is not None:
+            ctx.set_scalar("vl_skin", skin)
+        ctx.step(steps)
+        for f in ("perm", "x", "vel", "angvel", "force", "torque", "p", "es", "ev"):
+            assert numpy.array_equal(ctx.get(f), ref.get(f)), f
