@@ -71,12 +71,14 @@ struct DevArrays {
     double4* ws[2];
     uint32_t* rank;      // original index -> sorted index (inverse of perm)
     uint32_t* movers;    // per simulation, MV_CAP indices whose key changed (unordered)
-    // The order a step used, kept when the step's end already re-sorted for
-    // the next one (what the reference's arrays hold after that step).
+    // The order a step used, when the step's end already re-sorted for the
+    // next one (what the reference's arrays hold after that step): kept whole
+    // (RESORTED_FULL), or told by the movers of the merge, per simulation
+    // MV_CAP records {index, old key, old place, new place} in ascending new
+    // place (RESORTED_MERGE).  Its cell ranges follow from its keys.
     uint32_t* skey_bk;
     uint32_t* perm_bk;
-    uint32_t* cs_bk;
-    uint32_t* ce_bk;
+    uint4* mv_last;
     // candidate lists (sorted-index rows of NV entries)
     uint2* vlist;
     uint2* vcount;       // {entries per row | flags, or VL_OVERFLOW; hit mask}

@@ -249,7 +249,8 @@ __global__ __launch_bounds__(BLOCK) void k_hash(const DevArrays a) {
 // element order inside a tile is (round, thread), which is the global
 // index order, so ranking each round after all earlier rounds keeps the
 // sort stable.  The stages are written per tile so that the same code runs
-// as one launch per stage or inside the one-workgroup re-sort.
+// as one launch per stage or inside the one-workgroup re-sort, whose
+// work-items beyond BLOCK only keep the barriers.
 
 __device__ __forceinline__ void radix_hist_tile(const uint32_t* __restrict__ kin, uint32_t n,
                                                 int shift, int bits,
@@ -257,13 +258,14 @@ __device__ __forceinline__ void radix_hist_tile(const uint32_t* __restrict__ kin
                                                 uint32_t tile) {
     __shared__ uint32_t h[256];
     const uint32_t bins = 1u << bits, mask = bins - 1u;
-    h[threadIdx.x] = 0;
+    const bool act = threadIdx.x < BLOCK;
+    if (act) h[threadIdx.x] = 0;
     __syncthreads();
     const uint32_t base = tile * RADIX_TILE;
 #pragma unroll
     for (int j = 0; j < RADIX_ITEMS; ++j) {
         const uint32_t e = base + j * BLOCK + threadIdx.x;
-        if (e < n) atomicAdd(&h[(kin[e] >> shift) & mask], 1u);
+        if (act && e < n) atomicAdd(&h[(kin[e] >> shift) & mask], 1u);
     }
     __syncthreads();
     if (threadIdx.x < bins) hist[threadIdx.x * ntiles + tile] = h[threadIdx.x];
@@ -317,15 +319,18 @@ __device__ __forceinline__ void radix_scatter_tile(const uint32_t* __restrict__ 
     const uint32_t t = threadIdx.x;
     const uint32_t w = t >> 6;
     const uint32_t lane = t & 63u;
-    running[t] = t < bins ? hist[t * ntiles + tile] : 0u;
+    const bool act = t < BLOCK;
+    if (act) running[t] = t < bins ? hist[t * ntiles + tile] : 0u;
     const uint32_t base = tile * RADIX_TILE;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     for (int j = 0; j < RADIX_ITEMS; ++j) {
+        if (act) {
 #pragma unroll
-        for (int q = 0; q < BLOCK / 64; ++q) whist[q][t] = 0u;
+            for (int q = 0; q < BLOCK / 64; ++q) whist[q][t] = 0u;
+        }
         __syncthreads();
         const uint32_t e = base + j * BLOCK + t;
-        const bool valid = e < n;
+        const bool valid = act && e < n;
         const uint32_t k = valid ? kin[e] : 0u;
         const uint32_t v = valid ? (vin ? vin[e] : vbase + e) : 0u;
         const uint32_t d = (k >> shift) & mask;
@@ -345,10 +350,12 @@ __device__ __forceinline__ void radix_scatter_tile(const uint32_t* __restrict__ 
             vout[off] = v;
         }
         __syncthreads();
-        uint32_t add = 0;
+        if (act) {
+            uint32_t add = 0;
 #pragma unroll
-        for (int q = 0; q < BLOCK / 64; ++q) add += whist[q][t];
-        running[t] += add;
+            for (int q = 0; q < BLOCK / 64; ++q) add += whist[q][t];
+            running[t] += add;
+        }
         __syncthreads();
     }
 }
@@ -2249,7 +2256,7 @@ __device__ __forceinline__ double serial_sum(const double* __restrict__ part, ui
     double sum = 0.0;
     for (uint32_t base = 0; base < n; base += CH) {
         const uint32_t cnt = (n - base) < CH ? (n - base) : CH;
-        for (uint32_t j = threadIdx.x; j < cnt; j += BLOCK) stage[j] = part[base + j];
+        for (uint32_t j = threadIdx.x; j < cnt; j += blockDim.x) stage[j] = part[base + j];
         __syncthreads();
         if (threadIdx.x == 0) {
             // Sixteen LDS reads in flight, then the dependent adds in order:
@@ -2426,7 +2433,7 @@ template <typename T>
 __device__ __forceinline__ void bitonic_sort_lds(T* v, uint32_t n) {
     for (uint32_t k = 2; k <= n; k <<= 1)
         for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = threadIdx.x; i < n; i += BLOCK) {
+            for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
                 const uint32_t ixj = i ^ j;
                 if (ixj > i) {
                     const T x = v[i], y = v[ixj];
@@ -2457,51 +2464,141 @@ __device__ __forceinline__ unsigned long long composite(uint32_t key, uint32_t k
     return ((unsigned long long)(key & kmask) << 32) | idx;
 }
 
+// The number of entries of the old order [B, B + N) below composite c, found
+// by a whole wavefront: each round probes 64 places at once (three rounds
+// for 1e5 particles, where a binary search waits for 17 loads in turn).
+__device__ __forceinline__ uint32_t wave_lower_bound(const DevArrays& a, uint32_t B, uint32_t N,
+                                                     uint32_t kmask, unsigned long long c) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t lo = 0, hi = N;
+    while (hi > lo) {
+        const uint32_t len = hi - lo;
+        const uint32_t stride = (len + 63u) / 64u;
+        const uint32_t at = lo + lane * stride;
+        bool less = false;
+        if (at < hi) less = composite(a.skey[B + at], kmask, a.perm[B + at]) < c;
+        const uint32_t n = (uint32_t)__popcll(__ballot(less));
+        if (n == 0) break;
+        hi = min(hi, lo + n * stride);
+        lo = lo + (n - 1u) * stride + 1u;
+    }
+    return lo;
+}
+
+constexpr uint32_t WALLS_WG = 1024;  // work-items of k_walls
+constexpr uint32_t MV_FEW = 256;     // movers up to which the runs are listed
+constexpr uint32_t MV_WAVE = 64;     // movers up to which each search takes a wavefront
+
 // Re-sort simulation p's segment [B, B + N) of the sorted order (N = npad:
-// its particles, then its padding, whose keys never change).
-__device__ void resort_one_block(CParams& p, const DevArrays& a, int passes, int bits,
-                                 int sorted_bits) {
+// its particles, then its padding, whose keys never change).  A merge
+// rewrites only the places whose content changes: those a mover leaves or
+// takes, and the runs between them that shift.  With few movers the runs are
+// listed; with more, the whole span between the first and the last such
+// place is rewritten.  Each mover is recorded with its old and new place, so
+// that the finished step's order can be told afterwards.  Returns
+// DevLoop::resorted_last.
+//
+// Copying and rebuilding all places and cells in 256 work-items took 55-78 us
+// on a column of 4,096 in a wide grid and 300 us on 20,000 particles; this
+// takes 6 and 9.
+__device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp, int passes,
+                                     int bits, int sorted_bits) {
     __shared__ unsigned long long comp[MV_CAP];  // movers' (new key, index), ascending
     __shared__ uint32_t rk[MV_CAP];              // movers' old positions, ascending
     __shared__ uint32_t npos[MV_CAP];            // movers' new positions
+    __shared__ uint32_t okey[MV_CAP];            // movers' old keys
+    __shared__ uint32_t place[2 * MV_FEW];       // places left or taken, ascending
+    __shared__ uint32_t run0[2 * MV_FEW];        // first place of each run to rewrite
+    __shared__ uint32_t rlen[2 * MV_FEW];        // its length
+    __shared__ uint32_t roff[2 * MV_FEW + 1];    // places in the runs before it
     const uint32_t tid = threadIdx.x;
     const uint32_t B = p.base, N = p.npad;
-    const DevLoop* lp = a.loop + p.sim;
     const uint32_t* mv = a.movers + (size_t)p.sim * MV_CAP;
+    uint4* rec = a.mv_last + (size_t)p.sim * MV_CAP;
     const uint32_t M = lp->nmovers;
     // The radix sort orders by the low bits * passes bits of the key.
     const uint32_t kmask = bits * passes >= 32 ? 0xffffffffu : ((1u << (bits * passes)) - 1u);
-    const bool merge = M <= p.mv_max && M <= MV_CAP;
-    // Keep the order and cell ranges the finished step used.
-    for (uint32_t j = tid; j < N; j += BLOCK) {
-        a.skey_bk[B + j] = a.skey[B + j];
-        a.perm_bk[B + j] = a.perm[B + j];
+    if (!(M > 0 && M <= p.mv_max && M <= MV_CAP)) {
+        // Sort anew, keeping the order the finished step used.
+        for (uint32_t j = tid; j < N; j += WALLS_WG) {
+            a.skey_bk[B + j] = a.skey[B + j];
+            a.perm_bk[B + j] = a.perm[B + j];
+        }
+        __syncthreads();
+        const uint32_t nt = n_tiles(N);
+        uint32_t* hist = a.rhist + p.rhist_base;
+        for (int pass = 0; pass < passes; ++pass) {
+            const RadixPass r = radix_pass(a, pass, passes, B);
+            const int shift = bits * pass;
+            for (uint32_t t = 0; t < nt; ++t)
+                radix_hist_tile(r.kin, N, shift, bits, hist, nt, t);
+            __syncthreads();
+            radix_scan_block<WALLS_WG>(hist, (1u << bits) * nt);
+            for (uint32_t t = 0; t < nt; ++t)
+                radix_scatter_tile(r.kin, r.vin, r.kout, r.vout, N, shift, bits, hist, nt, t, B);
+            __syncthreads();
+        }
+        for (uint32_t c = tid; c < p.ncells; c += WALLS_WG)
+            a.cell_start[p.cell_base + c] = 0xffffffffu;
+        __syncthreads();
+        // (The sorted copies are left in the previous order: the next step
+        // reads the original-index arrays through perm, copies_stale, and
+        // its integration pass writes them in the new order.)
+        for (uint32_t j = tid; j < N; j += WALLS_WG)
+            cells_one(p, a, B + j, sorted_bits, 0u, false);
+        __syncthreads();
+        return RESORTED_FULL;
     }
-    for (uint32_t c = tid; c < p.ncells; c += BLOCK) {
-        a.cs_bk[p.cell_base + c] = a.cell_start[p.cell_base + c];
-        a.ce_bk[p.cell_base + c] = a.cell_end[p.cell_base + c];
+    const bool few = M <= MV_FEW;
+    uint32_t n2 = 1;
+    while (n2 < M) n2 <<= 1;
+    for (uint32_t m = tid; m < n2; m += WALLS_WG) {
+        comp[m] = ~0ull;
+        rk[m] = 0xffffffffu;
+        if (m < M) {
+            const uint32_t o = mv[m];
+            const uint32_t key = a.key[o], r = a.rank[o] - B;
+            comp[m] = composite(key, kmask, o);
+            rk[m] = r;
+            okey[m] = a.skey[B + r];
+            a.key_prev[o] = key;
+            if (sorted_bits < 32 && (key >> sorted_bits) != 0u)
+                atomicOr(&lp->error_bits, (uint32_t)DFLAG_KEY_RANGE);
+        }
     }
     __syncthreads();
-    if (merge) {
-        uint32_t n2 = 1;
-        while (n2 < M) n2 <<= 1;
-        for (uint32_t m = tid; m < n2; m += BLOCK) {
-            if (m < M) {
-                const uint32_t o = mv[m];
-                comp[m] = composite(a.key[o], kmask, o);
-                rk[m] = a.rank[o] - B;
-            } else {
-                comp[m] = ~0ull;
-                rk[m] = 0xffffffffu;
+    if (few) {
+        // Each mover's place by counting.
+        unsigned long long c = 0;
+        uint32_t r = 0, pc = 0, pr = 0;
+        if (tid < M) {
+            c = comp[tid];
+            r = rk[tid];
+            for (uint32_t k = 0; k < M; ++k) {
+                pc += comp[k] < c ? 1u : 0u;
+                pr += rk[k] < r ? 1u : 0u;
             }
         }
         __syncthreads();
+        if (tid < M) {
+            comp[pc] = c;
+            rk[pr] = r;
+        }
+        __syncthreads();
+    } else {
         bitonic_sort_lds(comp, n2);
         bitonic_sort_lds(rk, n2);
-        // A mover's new position: the unchanged particles before it (old
-        // elements below its composite, minus the movers among them) plus
-        // the movers before it.
-        for (uint32_t m = tid; m < M; m += BLOCK) {
+    }
+    // A mover's new position: the unchanged particles before it (old
+    // elements below its composite, minus the movers among them) plus
+    // the movers before it.
+    if (M <= MV_WAVE) {
+        for (uint32_t m = tid / 64u; m < M; m += WALLS_WG / 64u) {
+            const uint32_t lo = wave_lower_bound(a, B, N, kmask, comp[m]);
+            if ((tid & 63u) == 0) npos[m] = lo - count_below(rk, M, lo) + m;
+        }
+    } else {
+        for (uint32_t m = tid; m < M; m += WALLS_WG) {
             const unsigned long long c = comp[m];
             uint32_t lo = 0, hi = N;
             while (lo < hi) {
@@ -2511,67 +2608,110 @@ __device__ void resort_one_block(CParams& p, const DevArrays& a, int passes, int
             }
             npos[m] = lo - count_below(rk, M, lo) + m;
         }
+    }
+    __syncthreads();
+    for (uint32_t m = tid; m < M; m += WALLS_WG) {
+        const uint32_t o = (uint32_t)(comp[m] & 0xffffffffull);
+        const uint32_t r = a.rank[o] - B;
+        rec[m] = make_uint4(o, a.skey[B + r], r, npos[m]);
+    }
+    // The runs to rewrite.
+    uint32_t nrun = 1;
+    if (few) {
+        nrun = 2 * M;
+        if (tid < M) {
+            place[tid + count_below(npos, M, rk[tid])] = rk[tid];
+            place[tid + count_below(rk, M, npos[tid] + 1u)] = npos[tid];
+        }
         __syncthreads();
-        // New positions, a contiguous chunk per work-item.  The n-th
-        // unchanged particle sits at old position n + d, d = the number of
-        // movers with rk[d'] - d' <= n.
-        const uint32_t chunk = (N + BLOCK - 1) / BLOCK;
-        const uint32_t j0 = tid * chunk;
-        const uint32_t j1 = j0 + chunk < N ? j0 + chunk : N;
-        if (j0 < j1) {
-            uint32_t e = count_below(npos, M, j0);
-            uint32_t n = j0 - e;
+        if (tid < nrun) {
+            // After place x, until the next one, the content shifts by the
+            // movers that left up to x less those that arrived.
+            const uint32_t x = place[tid];
+            const uint32_t next = tid + 1 < nrun ? place[tid + 1] : x + 1;
+            const bool shifts = count_below(rk, M, x + 1u) != count_below(npos, M, x + 1u);
+            run0[tid] = x;
+            rlen[tid] = shifts ? next - x : (next != x ? 1u : 0u);
+        }
+        __syncthreads();
+        if (tid <= nrun) {
+            uint32_t off = 0;
+            for (uint32_t k = 0; k < tid; ++k) off += rlen[k];
+            roff[tid] = off;
+        }
+    } else if (tid == 0) {
+        const uint32_t s0 = min(rk[0], npos[0]);
+        run0[0] = s0;
+        roff[0] = 0;
+        roff[1] = max(rk[M - 1], npos[M - 1]) + 1u - s0;
+    }
+    __syncthreads();
+    const uint32_t total = roff[nrun];
+    // Place t of the runs; `last` where it ends its run.
+    auto place_of = [&](uint32_t t, bool& last) {
+        const uint32_t k = nrun == 1 ? 0u : count_below(roff, nrun, t + 1u) - 1u;
+        last = t + 1u == roff[k + 1];
+        return run0[k] + (t - roff[k]);
+    };
+    bool last;
+    // The n-th unchanged particle sits at old position n + d, d = the number
+    // of movers with rk[d'] - d' <= n.
+    for (uint32_t t = tid; t < total; t += WALLS_WG) {
+        const uint32_t j = place_of(t, last);
+        const uint32_t e = count_below(npos, M, j);
+        uint32_t key, o;
+        if (e < M && npos[e] == j) {
+            o = (uint32_t)(comp[e] & 0xffffffffull);
+            key = a.key[o];
+        } else {
+            const uint32_t n = j - e;
             uint32_t lo = 0, hi = M;
             while (lo < hi) {
                 const uint32_t mid = (lo + hi) >> 1;
                 if (rk[mid] - mid <= n) lo = mid + 1; else hi = mid;
             }
-            uint32_t d = lo;
-            for (uint32_t j = j0; j < j1; ++j) {
-                if (e < M && npos[e] == j) {
-                    const uint32_t o = (uint32_t)(comp[e] & 0xffffffffull);
-                    a.key_tmp[B + j] = a.key[o];
-                    a.val_tmp[B + j] = o;
-                    ++e;
-                } else {
-                    while (d < M && rk[d] - d <= n) ++d;
-                    const uint32_t i = n + d;
-                    a.key_tmp[B + j] = a.skey[B + i];
-                    a.val_tmp[B + j] = a.perm[B + i];
-                    ++n;
-                }
-            }
+            key = a.skey[B + n + lo];
+            o = a.perm[B + n + lo];
         }
-        __syncthreads();
-        for (uint32_t j = tid; j < N; j += BLOCK) {
-            a.skey[B + j] = a.key_tmp[B + j];
-            a.perm[B + j] = a.val_tmp[B + j];
-        }
-    } else {
-        const uint32_t nt = n_tiles(N);
-        uint32_t* hist = a.rhist + p.rhist_base;
-        for (int pass = 0; pass < passes; ++pass) {
-            const RadixPass r = radix_pass(a, pass, passes, B);
-            const int shift = bits * pass;
-            for (uint32_t t = 0; t < nt; ++t)
-                radix_hist_tile(r.kin, N, shift, bits, hist, nt, t);
-            __syncthreads();
-            radix_scan_block<BLOCK>(hist, (1u << bits) * nt);
-            for (uint32_t t = 0; t < nt; ++t)
-                radix_scatter_tile(r.kin, r.vin, r.kout, r.vout, N, shift, bits, hist, nt, t, B);
-            __syncthreads();
-        }
+        a.key_tmp[B + j] = key;
+        a.val_tmp[B + j] = o;
     }
-    for (uint32_t c = tid; c < p.ncells; c += BLOCK) a.cell_start[p.cell_base + c] = 0xffffffffu;
     __syncthreads();
-    // For the next step (the loop counter advances after this re-sort).  The
-    // sorted copies are left in the previous order: gathering them here, in
-    // one workgroup, would cost far more than the next step's contact pass
-    // reading the original-index arrays through perm (copies_stale), after
-    // which the integration pass writes them in the new order.
-    const uint32_t nxt = cur_set(a.loop + p.sim) ^ 1u;
-    for (uint32_t j = tid; j < N; j += BLOCK) cells_one(p, a, B + j, sorted_bits, nxt, false);
+    for (uint32_t t = tid; t < total; t += WALLS_WG) {
+        const uint32_t j = place_of(t, last);
+        const uint32_t o = a.val_tmp[B + j];
+        a.skey[B + j] = a.key_tmp[B + j];
+        a.perm[B + j] = o;
+        a.rank[o] = B + j;
+    }
     __syncthreads();
+    // Cell boundaries at the rewritten places and right behind each run
+    // (cells_one's rules).
+    auto boundary = [&](uint32_t j) {
+        const uint32_t pk = j > 0 ? a.skey[B + j - 1] : 0xffffffffu;
+        const uint32_t key = j < N ? a.skey[B + j] : 0xffffffffu;
+        if (j < N && (j == 0 || key != pk) && key - p.cell_base < p.ncells)
+            a.cell_start[key] = B + j;
+        if (j > 0 && (j == N || key != pk) && pk - p.cell_base < p.ncells)
+            a.cell_end[pk] = B + j;
+    };
+    for (uint32_t t = tid; t < total; t += WALLS_WG) {
+        const uint32_t j = place_of(t, last);
+        boundary(j);
+        if (last) boundary(j + 1u);
+    }
+    __syncthreads();
+    // A cell a mover left is empty when its range no longer starts with a
+    // particle of it.
+    for (uint32_t m = tid; m < M; m += WALLS_WG) {
+        const uint32_t k = okey[m];
+        if (k - p.cell_base >= p.ncells) continue;
+        const uint32_t s = a.cell_start[k];
+        if (s == 0xffffffffu) continue;
+        if (a.skey[s] != k || (s > B && a.skey[s - 1] == k)) a.cell_start[k] = 0xffffffffu;
+    }
+    __syncthreads();
+    return RESORTED_MERGE;
 }
 
 // integrateWalls + the loop advance (src/integration.cuh:344-450,
@@ -2579,8 +2719,8 @@ __device__ void resort_one_block(CParams& p, const DevArrays& a, int passes, int
 // integrates wall 0's force sum (src/device.cu:2504-2505).  With `resort`
 // set it first re-sorts for the next step when the integration pass found
 // particles that changed cell (the next step then launches no sort).
-__global__ __launch_bounds__(BLOCK) void k_walls(const DevArrays a, int resort, int passes,
-                                                 int bits, int sorted_bits) {
+__global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resort, int passes,
+                                                    int bits, int sorted_bits) {
     __shared__ double stage[2048];
     __shared__ uint32_t do_sort;
     touch_args();
@@ -2624,7 +2764,9 @@ __global__ __launch_bounds__(BLOCK) void k_walls(const DevArrays a, int resort, 
         if (threadIdx.x == 0) s_fsum[k] = fs;
     }
     __syncthreads();
-    if (do_sort) resort_one_block(p, a, passes, bits, sorted_bits);
+    const uint32_t movers = lp->nmovers;
+    uint32_t resorted = 0;
+    if (do_sort) resorted = resort_one_block(p, a, lp, passes, bits, sorted_bits);
     if (mine) {
         const uint32_t wi = p.wall_base + w;
         w_mvfd.z = s_fsum[p.wall_sums ? w : 0u];  // 0.0 + partial[0] + partial[1] + ...
@@ -2639,7 +2781,9 @@ __global__ __launch_bounds__(BLOCK) void k_walls(const DevArrays a, int resort, 
     }
     if (threadIdx.x != 0) return;
     if (do_sort) lp->sorts = sorts + 1u;
-    lp->resorted_last = do_sort;
+    lp->resorted_last = resorted;
+    if (resorted == RESORTED_MERGE) lp->nmv_last = movers;
+    if (movers) lp->moved += movers;
     // The next step's contact pass maps its rows to the new order and reads
     // the state through perm.
     lp->order_changed = do_sort;
@@ -2943,7 +3087,7 @@ hipError_t launch_integrate_q(const DevArrays& a, hipStream_t s) {
 
 hipError_t launch_walls(const DevArrays& a, int resort, int passes, int bits, int sorted_bits,
                         hipStream_t s) {
-    hipLaunchKernelGGL(k_walls, dim3(a.nsim), dim3(BLOCK), 0, s, a, resort, passes, bits,
+    hipLaunchKernelGGL(k_walls, dim3(a.nsim), dim3(WALLS_WG), 0, s, a, resort, passes, bits,
                        sorted_bits);
     return hipGetLastError();
 }

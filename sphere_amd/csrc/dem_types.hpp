@@ -135,11 +135,18 @@ struct DevLoop {
     uint32_t sorts;             // number of re-sorts so far (diagnostic)
     uint32_t nmovers;           // particles whose key changed for the next step
     uint32_t resorted_last;     // the last step ended with the next step's re-sort
+                                // (RESORTED_*), or 0
     uint32_t order_changed;     // the order changed since the contact rows were written
     uint32_t copies_stale;      // the sorted copies are in the previous order (read
                                 // the original-index arrays through perm instead)
+    uint32_t nmv_last;          // records of the last merge (DevArrays::mv_last)
+    uint32_t moved;             // particles that changed cell so far (diagnostic)
     uint32_t pad1;
 };
+
+// DevLoop::resorted_last: how the previous order is kept.
+constexpr uint32_t RESORTED_FULL = 1u;
+constexpr uint32_t RESORTED_MERGE = 2u;
 
 // Batch-wide state.
 struct DevGlobal {

@@ -165,6 +165,7 @@ struct sph_ctx {
     bool sample_pending = false;
     int64_t sample_iter0 = 0;
     uint64_t sample_sorts0 = 0;
+    uint32_t sample_moved0 = 0;
     // Steady-state step chunks replayed from captured HIP graphs (0 = off):
     // one graph per (chunk length, re-sort placement, contact lanes).
     int graph_steps = 0;
@@ -536,7 +537,7 @@ int allocate(sph_ctx* c) {
     ALLOC(A.x_build, np);
     ALLOC(A.movers, ns * MV_CAP);
     ALLOC(A.skey_bk, np); ALLOC(A.perm_bk, np);
-    ALLOC(A.cs_bk, nkeys); ALLOC(A.ce_bk, nkeys);
+    ALLOC(A.mv_last, ns * MV_CAP);
     ALLOC(A.crow, np * NC);
     ALLOC(A.perm_rows, np);
     ALLOC(A.delta_t, np * NC);
@@ -940,9 +941,21 @@ void prof_collect(sph_ctx* c) {
 }
 
 // Re-sort placement for the steps about to be enqueued.  In automatic mode
-// the choice follows the re-sort rate seen over the previous sph_step call,
-// read from an asynchronous copy of the loop counters (no synchronisation):
-// the end-of-step workgroup wins while fewer than one step in ten re-sorts.
+// the choice follows the particles that changed cell per re-sort over the
+// previous sph_step call, read from an asynchronous copy of the loop counters
+// (no synchronisation).  The end-of-step workgroup rewrites only what the
+// movers shift; the sort launches cost 16-20 us a step even when they return
+// at once and sort everything when they do not.  Collapsing gases, us a step,
+// end of step / launches: 5,000 particles 40 / 70 (83% of the steps re-sort),
+// 100,000 112 / 186 (98%), 1,000,000 940 / 1,651 (100%, a few movers each).
+// With more movers what they shift grows, the sooner against a whole sort the
+// smaller the simulation: 133 / 191 at 25 movers and 275 / 191 at 125 of
+// 100,000, 390 / 488 at 75 of 300,000, 1,356 / 1,652 at 250 of 1,000,000.  Up
+// to SMALL_NP particles rewriting everything in one workgroup still costs
+// less than the launches (20,000: 75 / 88).
+constexpr double MOVERS_PER_SQRT_NP = 0.27, MOVERS_SMALL = 1024.0;
+constexpr uint32_t SMALL_NP = 32768;
+
 void choose_sort_placement(sph_ctx* c) {
     if (c->sort_mode != 2) {
         c->resort_at_end = c->sort_mode == 1;
@@ -958,11 +971,15 @@ void choose_sort_placement(sph_ctx* c) {
     if (hipEventQuery(c->sample_ev) != hipSuccess) return;
     c->sample_pending = false;
     const DevLoop& L = c->loop_sample[0];
-    const int64_t steps = L.iter - c->sample_iter0;
-    const uint64_t sorts = L.sorts - c->sample_sorts0;
-    if (steps >= 20) c->resort_at_end = (double)sorts < 0.1 * (double)steps;
+    const uint32_t sorts = L.sorts - (uint32_t)c->sample_sorts0;
+    const uint32_t moved = L.moved - c->sample_moved0;
+    const uint32_t np = c->sims[0].h.np;
+    const double limit = np > SMALL_NP ? MOVERS_PER_SQRT_NP * sqrt((double)np) : MOVERS_SMALL;
+    if (L.iter - c->sample_iter0 >= 20)
+        c->resort_at_end = (double)moved <= limit * (double)std::max(sorts, 1u);
     c->sample_iter0 = L.iter;
     c->sample_sorts0 = L.sorts;
+    c->sample_moved0 = L.moved;
 }
 
 void sample_loop(sph_ctx* c) {
@@ -1635,6 +1652,51 @@ int sph_run(sph_ctx* c, const char* out_dir, const char* sid) {
     return SPH_OK;
 }
 
+// The order (global keys, batch indices) the last step of simulation `sim`
+// used, when that step ended by re-sorting for the next one.
+static int previous_order(sph_ctx* c, int sim, const DevLoop& L, std::vector<uint32_t>& key,
+                          std::vector<uint32_t>& perm) {
+    const Sim& S = c->sims[sim];
+    const size_t np = S.h.np, b0 = S.P.base;
+    const bool full = L.resorted_last == RESORTED_FULL;
+    key.resize(np);
+    perm.resize(np);
+    int rc = d2h(c, key.data(), (full ? c->A.skey_bk : c->A.skey) + b0, np * 4);
+    if (!rc) rc = d2h(c, perm.data(), (full ? c->A.perm_bk : c->A.perm) + b0, np * 4);
+    if (rc || full) return rc;
+    // Undo the merge: take the movers out of their new places (ascending in
+    // the records) and put them back at their old ones.
+    std::vector<uint4> mv(L.nmv_last);
+    rc = d2h(c, mv.data(), c->A.mv_last + (size_t)sim * MV_CAP, mv.size() * sizeof(uint4));
+    if (rc) return rc;
+    std::vector<uint32_t> k0, p0;
+    k0.reserve(np);
+    p0.reserve(np);
+    size_t e = 0;
+    for (size_t j = 0; j < np; ++j) {
+        if (e < mv.size() && mv[e].w == j) {
+            ++e;
+            continue;
+        }
+        k0.push_back(key[j]);
+        p0.push_back(perm[j]);
+    }
+    std::sort(mv.begin(), mv.end(), [](const uint4& x, const uint4& y) { return x.z < y.z; });
+    size_t n = 0, d = 0;
+    for (size_t i = 0; i < np; ++i) {
+        if (d < mv.size() && mv[d].z == i) {
+            key[i] = mv[d].y;
+            perm[i] = mv[d].x;
+            ++d;
+        } else {
+            key[i] = k0[n];
+            perm[i] = p0[n];
+            ++n;
+        }
+    }
+    return SPH_OK;
+}
+
 int64_t sph_field_bytes_sim(sph_ctx* c, int sim, int field) {
     CHECK_SIM(c, sim);
     return field_bytes(c, sim, field);
@@ -1718,23 +1780,39 @@ int sph_get_field_sim(sph_ctx* c, int sim, int f, void* dst, size_t bytes) {
             DevLoop L;
             int rc = read_loop(c, sim, &L);
             if (rc) return rc;
-            const bool bk = L.resorted_last != 0u;
-            const uint32_t* src = nullptr;
-            size_t off = 0;
-            if (f == SPH_F_CELLID) { src = bk ? A.skey_bk : A.skey; off = b0; }
-            if (f == SPH_F_PERM) { src = bk ? A.perm_bk : A.perm; off = b0; }
-            if (f == SPH_F_CELLSTART) { src = bk ? A.cs_bk : A.cell_start; off = S.P.cell_base; }
-            if (f == SPH_F_CELLEND) { src = bk ? A.ce_bk : A.cell_end; off = S.P.cell_base; }
-            rc = d2h(c, dst, src + off, bytes);
             uint32_t* w = static_cast<uint32_t*>(dst);
+            if (L.resorted_last == 0u) {
+                const uint32_t* src = f == SPH_F_CELLID      ? A.skey + b0
+                                      : f == SPH_F_PERM      ? A.perm + b0
+                                      : f == SPH_F_CELLSTART ? A.cell_start + S.P.cell_base
+                                                             : A.cell_end + S.P.cell_base;
+                rc = d2h(c, dst, src, bytes);
+                if (rc) return rc;
+                const uint32_t base = f == SPH_F_CELLID ? S.P.cell_base : (uint32_t)b0;
+                const bool range = f == SPH_F_CELLSTART || f == SPH_F_CELLEND;
+                for (size_t i = 0; i < bytes / 4; ++i)
+                    if (!range || w[i] != 0xffffffffu) w[i] -= base;
+                return SPH_OK;
+            }
+            std::vector<uint32_t> key, perm;
+            rc = previous_order(c, sim, L, key, perm);
+            if (rc) return rc;
             if (f == SPH_F_CELLID)
-                for (size_t i = 0; !rc && i < np; ++i) w[i] -= S.P.cell_base;
+                for (size_t i = 0; i < np; ++i) w[i] = key[i] - S.P.cell_base;
             if (f == SPH_F_PERM)
-                for (size_t i = 0; !rc && i < np; ++i) w[i] -= (uint32_t)b0;
-            if (f == SPH_F_CELLSTART || f == SPH_F_CELLEND)
-                for (size_t i = 0; !rc && i < S.P.ncells; ++i)
-                    if (w[i] != 0xffffffffu) w[i] -= (uint32_t)b0;
-            return rc;
+                for (size_t i = 0; i < np; ++i) w[i] = perm[i] - (uint32_t)b0;
+            if (f == SPH_F_CELLSTART || f == SPH_F_CELLEND) {
+                // The ranges of the order's keys (the ends of empty cells
+                // are not meaningful).
+                for (size_t i = 0; i < S.P.ncells; ++i) w[i] = 0xffffffffu;
+                for (size_t i = 0; i < np; ++i) {
+                    const uint32_t k = key[i] - S.P.cell_base;
+                    if (k >= S.P.ncells) continue;
+                    if (f == SPH_F_CELLEND) w[k] = (uint32_t)i + 1u;
+                    else if (w[k] == 0xffffffffu) w[k] = (uint32_t)i;
+                }
+            }
+            return SPH_OK;
         }
         case SPH_F_WALLS_NX: return d2h(c, dst, A.w_nx + w0, bytes);
         case SPH_F_WALLS_MVFD: return d2h(c, dst, A.w_mvfd + w0, bytes);

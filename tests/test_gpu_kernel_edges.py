@@ -97,3 +97,34 @@ def test_model1_matches_oracle(case, steps, skin):
         ctx.step(steps)
         for f in ("perm", "x", "vel", "angvel", "force", "torque", "p", "es", "ev"):
             assert numpy.array_equal(ctx.get(f), ref.get(f)), f
+
+
+# The end-of-step re-sort: one mover, a few, more than get a wavefront for
+# their search (64), more than have their runs listed (256), more than it
+# merges (2,048), whole and partial last chunks; the finished step's order and
+# cells are told from the movers' records.
+@pytest.mark.parametrize("n,movers", [
+    (1, 1), (256, 1), (257, 3), (3000, 2), (3000, 64), (3000, 65), (3000, 256), (3000, 257),
+    (3000, 1900), (3000, 2600)])
+def test_resort_of_many_movers(n, movers):
+    rng = numpy.random.default_rng(n + movers)
+    s = _cloud(n, 11, r=(0.002, 0.003))
+    s.x = rng.uniform(0.1, 0.4, (n, 3))
+    cell = float(s.L[0]) / int(s.num[0])
+    pick = rng.choice(n, size=movers, replace=False)
+    step = rng.uniform(-1.3, 1.3, (movers, 3)) * cell
+    s.vel[pick, :3] = step / float(s.time_dt[0])
+    image = s.tobytes()
+    ref = oracle.Oracle(image)
+    with engine.Context(image) as ctx:
+        ctx.set_scalar("sort_mode", 1)
+        for k in range(5):
+            ctx.step(1)
+            ref.step(1)
+            cs, ce = ctx.get("cellstart"), ctx.get("cellend")
+            rs, re_ = ref.get("cellstart"), ref.get("cellend")
+            occ = rs != 0xffffffff
+            assert numpy.array_equal(cs, rs) and numpy.array_equal(ce[occ], re_[occ]), k
+            for f in ("perm", "cellid", "contacts", "x", "vel", "force", "delta_t"):
+                assert numpy.array_equal(ctx.get(f), ref.get(f)), (k, f)
+        assert ctx.scalar("sorts") >= 1
