@@ -39,6 +39,7 @@
 
 #include "adjoint.hpp"
 #include "dem_math.hpp"
+#include "dem_scalar.hpp"
 
 namespace sphx {
 
@@ -53,21 +54,23 @@ constexpr double PI = 3.14159265358979;  // src/constants.h:14
 __device__ __forceinline__ d3 zero3() { return mk3(0.0, 0.0, 0.0); }
 
 // Cotangents of the parameters, in the order of AdjParam: one work-item's
-// running sums, kept in LDS (stride 256 doubles between parameters) to
-// spare registers.
+// running sums (indexed by constants only: registers).
 struct PGrad {
-    double* s;
-    __device__ __forceinline__ void add(int k, double x) const { s[k * 256] += x; }
+    double s[ADJ_NPARAM];
+    __device__ __forceinline__ void add(int k, double x) { s[k] += x; }
+    __device__ __forceinline__ void add(bool own, int k, double x) { s[k] += own ? x : 0.0; }
 };
 
 // Reverse of contactLinear (src/contactmodels.cuh:244-411, kappa = 0,
 // E <= 0.001) for one contact of particle a with partner b.  Inputs are the
 // forward inputs; gF, gT are the cotangents of a's force and torque and gdt
-// that of the new tangential displacement.  Outputs are accumulated.
-template <bool PARAMS>
-__device__ void adj_contact_linear(CParams& p, d3 va, d3 wa, d3 vb, d3 wb, double ra,
-                                   double rb, d3 x, d3 dt0, d3 gF, d3 gT, d3 gdt, d3& gx,
-                                   d3& gva, d3& gwa, d3& gvb, d3& gwb, d3& gdt0, PGrad& gp) {
+// that of the new tangential displacement.  The outputs are what falls on
+// one of the two: with `own` on a (gx, gv, gw, the stored displacement's
+// cotangent gdt0, and the parameters added to gp), else on b (gx, gv, gw).
+__device__ __forceinline__ void adj_contact_linear(CParams& p, bool own, d3 va, d3 wa, d3 vb,
+                                                   d3 wb, double ra, double rb, d3 x, d3 dt0,
+                                                   d3 gF, d3 gT, d3 gdt, d3& gx, d3& gv, d3& gw,
+                                                   d3& gdt0, PGrad& gp) {
     // forward (same expressions and FP32 lengths, so the same branches)
     const double len = length(x);
     const double delta = len - (ra + rb);
@@ -122,15 +125,15 @@ __device__ void adj_contact_linear(CParams& p, d3 va, d3 wa, d3 vb, d3 wb, doubl
             // dt_new = -1/k_t (mu_d L t + gamma_t vel_t), f_t = mu_s L t
             const d3 A = p.mu_d * L * t + p.gamma_t * vel_t;
             const d3 gA = gdt * (-1.0 / p.k_t);
-            if constexpr (PARAMS) gp.add(ADJ_KT, dot(gdt, A) / (p.k_t * p.k_t));
-            if constexpr (PARAMS) gp.add(ADJ_MUD, L * dot(t, gA));
+            gp.add(own, ADJ_KT, dot(gdt, A) / (p.k_t * p.k_t));
+            gp.add(own, ADJ_MUD, L * dot(t, gA));
             gL += p.mu_d * dot(t, gA);
             d3 gt = (p.mu_d * L) * gA;
-            if constexpr (PARAMS) gp.add(ADJ_GT, dot(vel_t, gA));
+            gp.add(own, ADJ_GT, dot(vel_t, gA));
             gvel_t += p.gamma_t * gA;
             const double glim = dot(t, gft);
             gt += limit * gft;
-            if constexpr (PARAMS) gp.add(ADJ_MUS, L * glim);
+            gp.add(own, ADJ_MUS, L * glim);
             gL += p.mu_s * glim;
             gfraw = (gt - t * dot(t, gt)) / frl;
         } else {
@@ -139,8 +142,8 @@ __device__ void adj_contact_linear(CParams& p, d3 va, d3 wa, d3 vb, d3 wb, doubl
         }
         // f_raw = -k_t dtmp - gamma_t vel_t, dtmp = dtp + vel_t dt
         gdtmp += -p.k_t * gfraw;
-        if constexpr (PARAMS) gp.add(ADJ_KT, -dot(dtmp, gfraw));
-        if constexpr (PARAMS) gp.add(ADJ_GT, -dot(vel_t, gfraw));
+        gp.add(own, ADJ_KT, -dot(dtmp, gfraw));
+        gp.add(own, ADJ_GT, -dot(vel_t, gfraw));
         gvel_t += -p.gamma_t * gfraw;
         gdtp += gdtmp;
         gvel_t += p.dt * gdtmp;
@@ -152,13 +155,13 @@ __device__ void adj_contact_linear(CParams& p, d3 va, d3 wa, d3 vb, d3 wb, doubl
     gn += cn * gfn;
     double gvel_n = 0.0;
     if (cn_raw > 0.0) {
-        if constexpr (PARAMS) gp.add(ADJ_KN, -delta * gcn);
+        gp.add(own, ADJ_KN, -delta * gcn);
         gdelta += -p.k_n * gcn;
-        if constexpr (PARAMS) gp.add(ADJ_GN, vel_n * gcn);
+        gp.add(own, ADJ_GN, vel_n * gcn);
         gvel_n = p.gamma_n * gcn;
     }
     // dtp = dt0 - n (n . dt0)
-    gdt0 += gdtp - n * dot(n, gdtp);
+    gdt0 = gdtp - n * dot(n, gdtp);
     gn += -(nd0 * gdtp + dot(n, gdtp) * dt0);
     // vel_t = vel - n (n . vel)
     const d3 gvel = gvel_t - n * dot(n, gvel_t);
@@ -171,12 +174,11 @@ __device__ void adj_contact_linear(CParams& p, d3 va, d3 wa, d3 vb, d3 wb, doubl
     gdelta += 0.5 * dot(gvel, na) + 0.5 * dot(gvel, nb);
     const d3 gna = ca * gvel, gnb = cb * gvel;
     gn += cross(wa, gna) + cross(wb, gnb);
-    gwa += cross(gna, n);
-    gwb += cross(gnb, n);
-    gva += gvl;
-    gvb += -gvl;
+    gw = cross(own ? gna : gnb, n);
+    gv = own ? gvl : -gvl;
     // n = x / |x|, delta = |x| - (ra + rb)
-    gx += (gn - n * dot(n, gn)) / len + n * gdelta;
+    const d3 gxa = (gn - n * dot(n, gn)) / len + n * gdelta;
+    gx = own ? gxa : -gxa;
 }
 
 // Reverse of contactLinear_wall (src/contactmodels.cuh:10-117) for one wall
@@ -248,14 +250,10 @@ constexpr int ALPP = 4;               // work-items per particle
 constexpr int ASPL = NC / ALPP;       // contact slots per work-item
 static_assert(ADJ_PPB * ALPP == 256, "four work-items per particle");
 
-__device__ __forceinline__ double group_sum(double v) {
-#pragma unroll
-    for (int o = 1; o < ALPP; o <<= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-__device__ __forceinline__ d3 group_sum(d3 v) {
-    return mk3(group_sum(v.x), group_sum(v.y), group_sum(v.z));
+// Orders the wavefront's LDS accesses around it.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // Force and torque cotangents of one particle (reverse of TY3 for the
@@ -304,30 +302,6 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// One list wall's contact (walls 0..nw-1 of the simulation): the particle's
-// part, the wall's position and velocity cotangents (sign: how the contact
-// distance changes with the wall position), the force sum's cotangent gS.
-__device__ __forceinline__ void wall_contact(CParams& p, const AdjStep& st,
-                                             const AdjState& g, int w, d3 va, d3 wa, double ra,
-                                             d3 e, double sign, double dw, d3 wn, double wvel,
-                                             d3 gF, d3 gT, d3& gxa, d3& gva, d3& gwa,
-                                             double (&cwp)[MAXWALLS], double (&cwu)[MAXWALLS],
-                                             PGrad& gp) {
-    const bool listed = (uint32_t)w < p.nw;
-    const double gS = listed ? g.wall[(p.wall_base + w) * ADJ_WALL + 3] : 0.0;
-    double gdel = 0.0, gwv = 0.0;
-    adj_contact_wall(p, va, wa, ra, wn, dw, wvel, gF, gT, gS, gva, gwa, gdel, gwv, gp);
-    gxa += gdel * e;
-    if (listed) {
-#pragma unroll
-        for (int k = 0; k < MAXWALLS; ++k)
-            if (k == w) {
-                cwp[k] += sign * gdel;
-                cwu[k] += gwv;
-            }
-    }
-}
-
 // Reverse of one whole step, ALPP work-items per particle, in the step's
 // sorted order (partner gathers then stay near each other in the recorded
 // state).  Every particle's input cotangent is gathered by its own group,
@@ -336,51 +310,82 @@ __device__ __forceinline__ void wall_contact(CParams& p, const AdjStep& st,
 //     La/Laa out) the force and torque cotangents and the integrate part
 //     of the input cotangents; the acceleration cotangents of the step's
 //     inputs go to La/Laa in;
-//  2. contacts: each work-item takes slots q, q + ALPP, ... of the row the
-//     step left.  For contact a -> b it reverses a's contactLinear (a's
-//     part, the parameters, and the stored displacement's cotangent, handed
-//     to the step before where that slot held the same partner then), and
-//     finds a in b's row to reverse b's contactLinear against a for the
-//     part that falls on a (b's force cotangents recomputed from b's Lout).
-//     Contact rows are symmetric unless a row overflowed; a contact whose
-//     partner does not list it is counted in `asym` (the host then refuses
-//     the result);
+//  2. contacts.  A contact a -> b of the row the step left gives two
+//     evaluations: its own (a's contactLinear: a's part, the parameters, and
+//     the stored displacement's cotangent, handed to the step before where
+//     that slot held the same partner then), and its mirror (b's
+//     contactLinear against a, found in b's row: the part that falls on a,
+//     with b's force cotangents recomputed from b's Lout).  The wavefront's
+//     evaluations are numbered, all own ones first, then the mirrors, each
+//     particle's in slot order, and taken one per lane; each particle's lanes
+//     then add its contributions in that order (lane 0 x, lane 1 v, lane 2
+//     w), so that a particle's sums do not depend on its neighbours in the
+//     wavefront.  Contact rows are symmetric unless a row overflowed; a
+//     contact whose partner does not list it is counted in `asym` (the host
+//     then refuses the result);
 //  3. walls, on work-item 0, including the cotangent of each wall force
 //     the particle puts on a list wall (from the wall's equation of
 //     motion) and the cotangents of the walls' position and velocity;
 //  4. the group's sums are written to Lin; the workgroup's partial sums of
 //     the parameter and wall cotangents to part.
+// Bound by the latency of its load chain (order, row, partner and its row,
+// displacements) at two wavefronts per SIMD (202 VGPRs; three spill 59 and
+// took 102 us where two take 76).  Each work-item walking its own slots, both
+// evaluations of each one after the other, took 91 us a step on 1e5
+// particles and 25 on 2,000; this takes 76 and 17.
 __global__ __launch_bounds__(256) void k_adj_step(AdjStep st, AdjState g) {
+    constexpr int G = 64 / ALPP;  // particles per wavefront
+    struct Work {
+        double con[9][64];
+        uint16_t tab[G * NC];
+    };
+    __shared__ Work s_work[4];
+    __shared__ uint32_t s_row[4][G][NC];
+    __shared__ double4 s_state[4][3][G];
+    __shared__ double s_force[4][6][G];
+    __shared__ uint32_t s_orig[4][G];
+    __shared__ uint2 s_prev[4][G];
+    __shared__ __align__(16) uint8_t s_zc[4][G];
     __shared__ double red[ADJ_NPART][4];
-    __shared__ double psum[ADJ_NPARAM * 256];
-    CParams& p = *(CParams*)(st.ptab + st.chunk_sim[blockIdx.x / (256 / ADJ_PPB)]);
-    const uint32_t q = threadIdx.x % ALPP;
+    touch_lines<sizeof(AdjStep) + sizeof(AdjState)>((cvoid*)__builtin_amdgcn_kernarg_segment_ptr());
+    const uint32_t sim = st.nsim == 1u ? 0u : st.chunk_sim[blockIdx.x / (256 / ADJ_PPB)];
+    touch_lines<sizeof(DevParams)>((cvoid*)(st.ptab + sim));
+    CParams& p = *(CParams*)(st.ptab + sim);
+    const uint32_t lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+    const uint32_t q = threadIdx.x % ALPP, gw = lane / ALPP;
     const uint32_t ia = blockIdx.x * ADJ_PPB + threadIdx.x / ALPP;
+    const bool in = ia - p.base < p.np;
+    const double dt = p.dt;
     PGrad gp;
-    gp.s = psum + threadIdx.x;
-    for (int k = 0; k < ADJ_NPARAM; ++k) gp.s[k * 256] = 0.0;
-    double cwp[MAXWALLS], cwu[MAXWALLS];
 #pragma unroll
-    for (int k = 0; k < MAXWALLS; ++k) cwp[k] = cwu[k] = 0.0;
-    if (ia - p.base < p.np) {
-        const uint32_t a = st.perm[ia];
-        const double4 xa4 = st.x[ia], va4 = st.v[ia];
-        const d3 xa = xyz(xa4), va = xyz(va4), wa = xyz(st.w[ia]);
-        const double ra = xa4.w;
-        const double dt = p.dt;
+    for (int k = 0; k < ADJ_NPARAM; ++k) gp.s[k] = 0.0;
+    uint32_t a = 0, occ = 0;
+    d3 acc = zero3();
+    if (in) {
+        a = st.perm[ia];
+        // This work-item's row words (slots ASPL q, ...).
+        uint32_t word[ASPL];
+        const uint4* row = reinterpret_cast<const uint4*>(st.rows + (size_t)ia * NC + ASPL * q);
+#pragma unroll
+        for (int h = 0; h < ASPL / 4; ++h) {
+            const uint4 u = row[h];
+            word[4 * h] = u.x;
+            word[4 * h + 1] = u.y;
+            word[4 * h + 2] = u.z;
+            word[4 * h + 3] = u.w;
+        }
+        const uint2 prev = st.prev[ia];
+        const double4 xa4 = st.x[ia], va4 = st.v[ia], wa4 = st.w[ia];
         // 1. integrate
         const double4 Lx = g.Lout[0][a], Lv = g.Lout[1][a], Lw = g.Lout[2][a];
+        const double4 La = g.La_out[a], Laa = g.Laa_out[a];
         d3 gF, gT;
-        {
-            const double4 La = g.La_out[a], Laa = g.Laa_out[a];
-            force_cotangents(p, ra, va4.w, Lx, Lv, Lw, La, Laa, gF, gT);
-        }
-        d3 gxa = zero3(), gva = zero3(), gwa = zero3();
-        if (q == 0) {
-            // x' = x + ..., v' = v + ..., w' = w + ...
-            gxa = mk3(Lx.x, Lx.y, Lx.z);
-            gva = mk3(Lx.x * dt + Lv.x, Lx.y * dt + Lv.y, Lx.z * dt + Lv.z);
-            gwa = mk3(Lw.x, Lw.y, Lw.z);
+        force_cotangents(p, xa4.w, va4.w, Lx, Lv, Lw, La, Laa, gF, gT);
+        // x' = x + ..., v' = v + ..., w' = w + ...
+        if (q == 0) acc = mk3(Lx.x, Lx.y, Lx.z);
+        if (q == 1) acc = mk3(Lx.x * dt + Lv.x, Lx.y * dt + Lv.y, Lx.z * dt + Lv.z);
+        if (q == 2) acc = mk3(Lw.x, Lw.y, Lw.z);
+        if (q == 3) {
             const double c0 = st.first ? 0.0 : 1.0;  // acc0 is zero on a run's first step
             g.La_in[a] = make_double4(c0 * (-(dt * dt / 6.0) * Lx.x - 0.5 * dt * Lv.x),
                                       c0 * (-(dt * dt / 6.0) * Lx.y - 0.5 * dt * Lv.y),
@@ -388,182 +393,231 @@ __global__ __launch_bounds__(256) void k_adj_step(AdjStep st, AdjState g) {
             g.Laa_in[a] = make_double4(c0 * -0.5 * dt * Lw.x, c0 * -0.5 * dt * Lw.y,
                                        c0 * -0.5 * dt * Lw.z, 0.0);
         }
-        // 2. contacts.  This work-item's row words (and the previous step's)
-        // are loaded at once; the occupied slots go into a small queue held
-        // in registers (shifted, never indexed).
-        // (The previous rows' presence is tested once, not per word: a
-        // branch around each load would make the next load wait for it.)
-        uint32_t wv[ASPL], pv[ASPL];
-#pragma unroll
-        for (int j = 0; j < ASPL; ++j) {
-            wv[j] = st.rows[(size_t)a * NC + q + ALPP * j];
-            pv[j] = EMPTY;
+        if (q == 0) {
+            s_state[wv][0][gw] = make_double4(xa4.x, xa4.y, xa4.z, xa4.w);
+            s_orig[wv][gw] = a;
+            s_prev[wv][gw] = prev;
         }
-        if (st.prev_rows) {
-#pragma unroll
-            for (int j = 0; j < ASPL; ++j) pv[j] = st.prev_rows[(size_t)a * NC + q + ALPP * j];
-        }
-        // Queue entry: the row word, and j | previous slot occupied << 3 |
-        // same partner then << 4.
-        uint32_t qw[ASPL], qj[ASPL];
-        int nq = 0;
-#pragma unroll
-        for (int j = 0; j < ASPL; ++j) {
-            qw[j] = EMPTY;
-            qj[j] = 0;
+        if (q == 1) s_state[wv][1][gw] = make_double4(va4.x, va4.y, va4.z, va4.w);
+        if (q == 2) s_state[wv][2][gw] = make_double4(wa4.x, wa4.y, wa4.z, 0.0);
+        if (q == 3) {
+            s_force[wv][0][gw] = gF.x;
+            s_force[wv][1][gw] = gF.y;
+            s_force[wv][2][gw] = gF.z;
+            s_force[wv][3][gw] = gT.x;
+            s_force[wv][4][gw] = gT.y;
+            s_force[wv][5][gw] = gT.z;
         }
 #pragma unroll
         for (int j = 0; j < ASPL; ++j) {
-            const uint32_t wb = wv[j] & CW_IDX_MASK, pb = pv[j] & CW_IDX_MASK;
-            const bool occ = wb != EMPTY;
-            if (!occ && pb != EMPTY)
-                g.Ldt_out[(size_t)a * NC + q + ALPP * j] = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (occ) {
+            const uint32_t slot = ASPL * q + j;
+            const bool o = (word[j] & CW_IDX_MASK) != EMPTY;
+            s_row[wv][gw][slot] = word[j];
+            occ |= o ? 1u << slot : 0u;
+            // A slot that has lost its partner: no cotangent reaches the
+            // displacement it held.
+            if (!o && ((prev.x >> slot) & 1u))
+                g.Ldt_out[(size_t)a * NC + slot] = make_double4(0.0, 0.0, 0.0, 0.0);
+        }
+    }
 #pragma unroll
-                for (int k = ASPL - 1; k > 0; --k) {
-                    qw[k] = qw[k - 1];
-                    qj[k] = qj[k - 1];
+    for (int m = 1; m < ALPP; m <<= 1) occ |= (uint32_t)__shfl_xor((int)occ, m, 64);
+    const uint32_t zg = __popc(occ);
+    if (q == 0) s_zc[wv][gw] = (uint8_t)zg;
+    wave_sync();
+    // The group's first contact number and the wavefront's contact count
+    // (byte sums of the counts, each at most NC).
+    uint32_t first = 0, total = 0;
+    {
+        const uint32_t* zw = reinterpret_cast<const uint32_t*>(s_zc[wv]);
+#pragma unroll
+        for (int i = 0; i < G / 4; ++i) {
+            const uint32_t w = zw[i];
+            const int below_w = (int)gw - 4 * i;
+            const uint32_t m = below_w <= 0 ? 0u
+                               : below_w >= 4 ? 0xffffffffu
+                                              : (1u << (8 * below_w)) - 1u;
+            first += ((w & m) * 0x01010101u) >> 24;
+            total += (w * 0x01010101u) >> 24;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < ASPL; ++j) {
+        const uint32_t slot = ASPL * q + j;
+        if ((occ >> slot) & 1u)
+            s_work[wv].tab[first + __popc(occ & ((1u << slot) - 1u))] =
+                (uint16_t)((gw << 5) | slot);
+    }
+    wave_sync();
+    // 2. contacts
+    for (uint32_t r0 = 0; r0 < 2 * total; r0 += 64) {
+        const uint32_t it = r0 + lane;
+        d3 gx = zero3(), g1v = zero3(), g1w = zero3();
+        if (it < 2 * total) {
+            const bool own = it < total;
+            const uint32_t e = s_work[wv].tab[own ? it : it - total];
+            const uint32_t h = e >> 5, ih = ia - gw + h;
+            uint32_t slot = e & 31u, word = s_row[wv][h][slot];
+            const uint32_t bs = word & CW_IDX_MASK;
+            const double4 xb4 = st.x[bs], vb4 = st.v[bs], wb4 = st.w[bs];
+            uint32_t o1 = s_orig[wv][h], i1 = ih;  // whose contact it is
+            d3 gF, gT;
+            if (own) {
+                gF = mk3(s_force[wv][0][h], s_force[wv][1][h], s_force[wv][2][h]);
+                gT = mk3(s_force[wv][3][h], s_force[wv][4][h], s_force[wv][5][h]);
+            } else {
+                // The contact's mirror in b's row.  Every word is read (no
+                // branch between the loads, which would make each wait for
+                // the one before) and the first match kept.
+                const uint32_t b = st.perm[bs];
+                const uint4* brow = reinterpret_cast<const uint4*>(st.rows + (size_t)bs * NC);
+                slot = NC;
+#pragma unroll
+                for (int k = NC / 4 - 1; k >= 0; --k) {
+                    const uint4 u = brow[k];
+                    if ((u.w & CW_IDX_MASK) == ih) { slot = 4 * k + 3; word = u.w; }
+                    if ((u.z & CW_IDX_MASK) == ih) { slot = 4 * k + 2; word = u.z; }
+                    if ((u.y & CW_IDX_MASK) == ih) { slot = 4 * k + 1; word = u.y; }
+                    if ((u.x & CW_IDX_MASK) == ih) { slot = 4 * k; word = u.x; }
                 }
-                qw[0] = wv[j];
-                qj[0] = (uint32_t)j | (pb != EMPTY ? 8u : 0u) | (pb == wb ? 16u : 0u);
-                ++nq;
+                o1 = b;
+                i1 = bs;
+                force_cotangents(p, xb4.w, vb4.w, g.Lout[0][b], g.Lout[1][b], g.Lout[2][b],
+                                 g.La_out[b], g.Laa_out[b], gF, gT);
             }
-        }
-#pragma unroll 1
-        for (int k = 0; k < nq; ++k) {
-            const uint32_t wrd = qw[0], fl = qj[0];
-            const size_t mp = (size_t)a * NC + q + ALPP * (fl & 7u);
-#pragma unroll
-            for (int kk = 0; kk + 1 < ASPL; ++kk) {
-                qw[kk] = qw[kk + 1];
-                qj[kk] = qj[kk + 1];
-            }
-            const uint32_t b = wrd & CW_IDX_MASK;
-            const uint32_t bs = st.srt[mp];  // the partner's sorted index
-            const double4 xb4 = st.x[bs], vb4 = st.v[bs];
-            const d3 xb = xyz(xb4), vb = xyz(vb4), wb = xyz(st.w[bs]);
-            const double rb = xb4.w;
-            // a's contact with b: a's part, parameters, displacement.
-            {
-                const d3 dm = image_shift(p, wrd);
-                const d3 xab = mk3(xa.x - xb.x + dm.x, xa.y - xb.y + dm.y, xa.z - xb.z + dm.z);
-                const d3 gdt = st.last ? zero3() : xyz(g.Ldt_in[mp]);
-                d3 gx = zero3(), gvb = zero3(), gwb = zero3(), gdt0 = zero3();
-                adj_contact_linear<true>(p, va, wa, vb, wb, ra, rb, xab, xyz(st.dt0[mp]), gF, gT,
-                                         gdt, gx, gva, gwa, gvb, gwb, gdt0, gp);
-                gxa += gx;
-                if (fl & 8u)
-                    g.Ldt_out[mp] = (fl & 16u) ? make_double4(gdt0.x, gdt0.y, gdt0.z, 0.0)
-                                               : make_double4(0.0, 0.0, 0.0, 0.0);
-            }
-            // b's contact with a: the part that falls on a.
-            uint32_t t = NC;
-            const uint4* brow = reinterpret_cast<const uint4*>(st.rows + (size_t)b * NC);
-            // Every word is read (no branch between the loads, which would
-            // make each wait for the one before) and the first match kept.
-#pragma unroll
-            for (int h = NC / 4 - 1; h >= 0; --h) {
-                const uint4 u = brow[h];
-                t = (u.w & CW_IDX_MASK) == a ? 4 * h + 3 : t;
-                t = (u.z & CW_IDX_MASK) == a ? 4 * h + 2 : t;
-                t = (u.y & CW_IDX_MASK) == a ? 4 * h + 1 : t;
-                t = (u.x & CW_IDX_MASK) == a ? 4 * h : t;
-            }
-            if (t == NC) {
+            if (slot == NC) {
                 atomicAdd(g.asym, 1u);
-                continue;
-            }
-            const size_t mpb = (size_t)b * NC + t;
-            d3 gFb, gTb;
-            force_cotangents(p, rb, vb4.w, g.Lout[0][b], g.Lout[1][b], g.Lout[2][b],
-                             g.La_out[b], g.Laa_out[b], gFb, gTb);
-            const d3 dmb = image_shift(p, st.rows[mpb]);
-            const d3 xba = mk3(xb.x - xa.x + dmb.x, xb.y - xa.y + dmb.y, xb.z - xa.z + dmb.z);
-            const d3 gdtb = st.last ? zero3() : xyz(g.Ldt_in[mpb]);
-            d3 gx = zero3(), gvb_own = zero3(), gwb_own = zero3(), gva_part = zero3(),
-               gwa_part = zero3(), gdt0 = zero3();
-            adj_contact_linear<false>(p, vb, wb, va, wa, rb, ra, xba, xyz(st.dt0[mpb]), gFb, gTb,
-                                      gdtb, gx, gvb_own, gwb_own, gva_part, gwa_part, gdt0, gp);
-            gxa += -gx;
-            gva += gva_part;
-            gwa += gwa_part;
-        }
-        // 3. walls, as in the forward pass (src/contactsearch.cuh:602-701):
-        // top (wall 0, or the implicit wall at L_z), bottom, then the side
-        // walls by boundary mode; walls beyond nw are the implicit ones.
-        if (q == 0) {
-            const double4* wnx = st.wall_nx + p.wall_base;
-            const double4* wmv = st.wall_mvfd + p.wall_base;
-            {
-                double wpos = p.L[2], wvel = 0.0;
-                d3 wn = mk3(0.0, 0.0, -1.0);
-                if (p.nw >= 1) { wn = xyz(wnx[0]); wpos = wnx[0].w; wvel = wmv[0].y; }
-                const double dw = wpos - (xa.z + ra);
-                if (dw < 0.0)
-                    wall_contact(p, st, g, 0, va, wa, ra, mk3(0.0, 0.0, -1.0), 1.0, dw, wn, wvel,
-                                 gF, gT, gxa, gva, gwa, cwp, cwu, gp);
-            }
-            {
-                const double dw = xa.z - ra - p.origo[2];
-                if (dw < 0.0)
-                    wall_contact(p, st, g, -1, va, wa, ra, mk3(0.0, 0.0, 1.0), 0.0, dw,
-                                 mk3(0.0, 0.0, 1.0), 0.0, gF, gT, gxa, gva, gwa, cwp, cwu, gp);
-            }
-            if (p.periodic == 0) {
-                double wpos = p.L[0], wvel = 0.0;
-                d3 wn = mk3(-1.0, 0.0, 0.0);
-                if (p.nw >= 2) { wn = xyz(wnx[1]); wpos = wnx[1].w; wvel = wmv[1].y; }
-                double dw = wpos - (xa.x + ra);
-                if (dw < 0.0)
-                    wall_contact(p, st, g, 1, va, wa, ra, mk3(-1.0, 0.0, 0.0), 1.0, dw, wn, wvel,
-                                 gF, gT, gxa, gva, gwa, cwp, cwu, gp);
-                wpos = 0.0; wvel = 0.0; wn = mk3(1.0, 0.0, 0.0);
-                if (p.nw >= 3) { wn = xyz(wnx[2]); wpos = wnx[2].w; wvel = wmv[2].y; }
-                dw = xa.x - ra - wpos;
-                if (dw < 0.0)
-                    wall_contact(p, st, g, 2, va, wa, ra, mk3(1.0, 0.0, 0.0), -1.0, dw, wn, wvel,
-                                 gF, gT, gxa, gva, gwa, cwp, cwu, gp);
-            }
-            if (p.periodic == 0 || p.periodic == 2) {
-                double wpos = p.L[1], wvel = 0.0;
-                d3 wn = mk3(0.0, -1.0, 0.0);
-                if (p.nw >= 4) { wn = xyz(wnx[3]); wpos = wnx[3].w; wvel = wmv[3].y; }
-                double dw = wpos - (xa.y + ra);
-                if (dw < 0.0)
-                    wall_contact(p, st, g, 3, va, wa, ra, mk3(0.0, -1.0, 0.0), 1.0, dw, wn, wvel,
-                                 gF, gT, gxa, gva, gwa, cwp, cwu, gp);
-                wpos = 0.0; wvel = 0.0; wn = mk3(0.0, 1.0, 0.0);
-                if (p.nw >= 5) { wn = xyz(wnx[4]); wpos = wnx[4].w; wvel = wmv[4].y; }
-                dw = xa.y - ra - wpos;
-                if (dw < 0.0)
-                    wall_contact(p, st, g, 4, va, wa, ra, mk3(0.0, 1.0, 0.0), -1.0, dw, wn, wvel,
-                                 gF, gT, gxa, gva, gwa, cwp, cwu, gp);
+            } else {
+                const d3 dt0 = xyz(st.dt0[(size_t)i1 * NC + slot]);
+                const size_t mp = (size_t)o1 * NC + slot;
+                const d3 gdt = st.last ? zero3() : xyz(g.Ldt_in[mp]);
+                const double4 xh4 = s_state[wv][0][h], vh4 = s_state[wv][1][h],
+                              wh4 = s_state[wv][2][h];
+                // The contact's particle (1) and its partner (2).
+                const double4 x1 = own ? xh4 : xb4, x2 = own ? xb4 : xh4;
+                const double4 v1 = own ? vh4 : vb4, v2 = own ? vb4 : vh4;
+                const double4 w1 = own ? wh4 : wb4, w2 = own ? wb4 : wh4;
+                const d3 dm = image_shift(p, word);
+                const d3 x12 = mk3(x1.x - x2.x + dm.x, x1.y - x2.y + dm.y, x1.z - x2.z + dm.z);
+                d3 gdt0;
+                adj_contact_linear(p, own, xyz(v1), xyz(w1), xyz(v2), xyz(w2), x1.w, x2.w, x12,
+                                   dt0, gF, gT, gdt, gx, g1v, g1w, gdt0, gp);
+                const uint2 prev = s_prev[wv][h];
+                if (own && ((prev.x >> slot) & 1u))
+                    g.Ldt_out[mp] = ((prev.y >> slot) & 1u)
+                                        ? make_double4(gdt0.x, gdt0.y, gdt0.z, 0.0)
+                                        : make_double4(0.0, 0.0, 0.0, 0.0);
             }
         }
-        // 4. the particle's input cotangents
-        gxa = group_sum(gxa);
-        gva = group_sum(gva);
-        gwa = group_sum(gwa);
-        if (q == 0) {
-            g.Lin[0][a] = make_double4(gxa.x, gxa.y, gxa.z, 0.0);
-            g.Lin[1][a] = make_double4(gva.x, gva.y, gva.z, 0.0);
-            g.Lin[2][a] = make_double4(gwa.x, gwa.y, gwa.z, 0.0);
-        }
-    }
-    // Partial sums of the workgroup: wavefront butterflies, then the four
-    // wavefronts in order (a fixed order: reproducible bit for bit).
-    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    for (int k = 0; k < ADJ_NPARAM; ++k) {
-        const double v = wave_sum(gp.s[k * 256]);
-        if (lane == 0) red[k][wave] = v;
-    }
+        s_work[wv].con[0][lane] = gx.x;
+        s_work[wv].con[1][lane] = gx.y;
+        s_work[wv].con[2][lane] = gx.z;
+        s_work[wv].con[3][lane] = g1v.x;
+        s_work[wv].con[4][lane] = g1v.y;
+        s_work[wv].con[5][lane] = g1v.z;
+        s_work[wv].con[6][lane] = g1w.x;
+        s_work[wv].con[7][lane] = g1w.y;
+        s_work[wv].con[8][lane] = g1w.z;
+        wave_sync();
+        if (q < 3) {
 #pragma unroll
-    for (int k = 0; k < MAXWALLS; ++k) {
-        const double vp = wave_sum(cwp[k]), vu = wave_sum(cwu[k]);
-        if (lane == 0) {
-            red[ADJ_NPARAM + 2 * k][wave] = vp;
-            red[ADJ_NPARAM + 2 * k + 1][wave] = vu;
+            for (int part = 0; part < 2; ++part) {
+                const uint32_t f = first + (part ? total : 0u);
+                const uint32_t lo = f > r0 ? f : r0;
+                const uint32_t hi = f + zg < r0 + 64 ? f + zg : r0 + 64;
+                for (uint32_t c = lo; c < hi; ++c) {
+                    acc.x += s_work[wv].con[3 * q][c - r0];
+                    acc.y += s_work[wv].con[3 * q + 1][c - r0];
+                    acc.z += s_work[wv].con[3 * q + 2][c - r0];
+                }
+            }
         }
+        wave_sync();
+    }
+    // 3. walls, as in the forward pass (src/contactsearch.cuh:602-701):
+    // top (wall 0, or the implicit wall at L_z), bottom, then the side
+    // walls by boundary mode; walls beyond nw are the implicit ones.
+    if (lane < 2 * MAXWALLS) red[ADJ_NPARAM + lane][wv] = 0.0;
+    bool any_wall = false;
+    d3 gxw = zero3(), gvw = zero3(), gww = zero3();
+    {
+        const double4 xa4 = s_state[wv][0][gw];
+        // Side s: top, bottom, then x high and low, y high and low.  The
+        // contact distance changes with the position along e.
+#pragma unroll 1
+        for (int s = 0; s < 6; ++s) {
+            if ((s == 2 || s == 3) && p.periodic != 0) continue;
+            if ((s == 4 || s == 5) && p.periodic != 0 && p.periodic != 2) continue;
+            const int w = s == 0 ? 0 : s == 1 ? -1 : s - 1;  // its list wall
+            const bool listed = w >= 0 && (uint32_t)w < p.nw;
+            const double side = (s == 1 || s == 3 || s == 5) ? 1.0 : -1.0;
+            const d3 e = s < 2 ? mk3(0.0, 0.0, side)
+                               : s < 4 ? mk3(side, 0.0, 0.0) : mk3(0.0, side, 0.0);
+            d3 wn = e;
+            double wpos = s == 0 ? p.L[2] : s == 1 ? p.origo[2] : s == 2 ? p.L[0]
+                          : s == 4 ? p.L[1] : 0.0;
+            double wvel = 0.0;
+            if (listed) {
+                const auto* nx = (const __attribute__((address_space(4))) double*)(
+                    st.wall_nx + p.wall_base + w);
+                const auto* mv = (const __attribute__((address_space(4))) double*)(
+                    st.wall_mvfd + p.wall_base + w);
+                wn = mk3(nx[0], nx[1], nx[2]);
+                wpos = nx[3];
+                wvel = mv[1];
+            }
+            const double xc = s < 2 ? xa4.z : s < 4 ? xa4.x : xa4.y;
+            const double dw = side < 0.0 ? wpos - (xc + xa4.w) : xc - xa4.w - wpos;
+            const bool touch = in && q == 0 && dw < 0.0;
+            if (__ballot(touch) == 0ull) continue;
+            any_wall = true;
+            double gdel = 0.0, gwv = 0.0;
+            if (touch) {
+                const d3 va = xyz(s_state[wv][1][gw]), wa = xyz(s_state[wv][2][gw]);
+                const d3 gF = mk3(s_force[wv][0][gw], s_force[wv][1][gw], s_force[wv][2][gw]);
+                const d3 gT = mk3(s_force[wv][3][gw], s_force[wv][4][gw], s_force[wv][5][gw]);
+                // The force sum's cotangent; the wall's position moves dw
+                // against `side`.
+                const double gS = listed ? g.wall[(p.wall_base + w) * ADJ_WALL + 3] : 0.0;
+                adj_contact_wall(p, va, wa, xa4.w, wn, dw, wvel, gF, gT, gS, gvw, gww, gdel, gwv,
+                                 gp);
+                gxw += gdel * e;
+            }
+            if (listed) {
+                const double vp = wave_sum(-side * gdel), vu = wave_sum(gwv);
+                if (lane == 0) {
+                    red[ADJ_NPARAM + 2 * w][wv] = vp;
+                    red[ADJ_NPARAM + 2 * w + 1][wv] = vu;
+                }
+            }
+        }
+    }
+    if (any_wall) {
+        // Lane 0's parts to the lanes that hold the sums.
+        const int src = (int)(lane - q);
+        const d3 v1 = mk3(__shfl(gvw.x, src, 64), __shfl(gvw.y, src, 64), __shfl(gvw.z, src, 64));
+        const d3 w1 = mk3(__shfl(gww.x, src, 64), __shfl(gww.y, src, 64), __shfl(gww.z, src, 64));
+        acc += q == 0 ? gxw : q == 1 ? v1 : w1;
+    }
+    // 4. the particle's input cotangents
+    double4* const lin = q == 0 ? +g.Lin[0] : q == 1 ? +g.Lin[1] : +g.Lin[2];
+    if (in && q < 3) lin[a] = make_double4(acc.x, acc.y, acc.z, 0.0);
+    // Partial sums of the workgroup: wavefront butterflies, then the four
+    // wavefronts in order (a fixed order: reproducible bit for bit).  The
+    // walls' quantities are zero in a wavefront that touches none.
+#pragma unroll
+    for (int k = 0; k < ADJ_GWN; ++k) {
+        const double v = wave_sum(gp.s[k]);
+        if (lane == 0) red[k][wv] = v;
+    }
+    if (any_wall) {
+#pragma unroll
+        for (int k = ADJ_GWN; k < ADJ_NPARAM; ++k) {
+            const double v = wave_sum(gp.s[k]);
+            if (lane == 0) red[k][wv] = v;
+        }
+    } else if (lane >= ADJ_GWN && lane < ADJ_NPARAM) {
+        red[lane][wv] = 0.0;
     }
     __syncthreads();
     if (threadIdx.x < ADJ_NPART) {
@@ -763,6 +817,8 @@ __global__ __launch_bounds__(RED_WG) void k_adj_reduce(AdjStep st, AdjState g) {
     __shared__ double share[RED_Q][256];
     __shared__ double tot[RED_Q];
     __shared__ double wsum[MAXWALLS];
+    touch_lines<sizeof(AdjStep) + sizeof(AdjState)>((cvoid*)__builtin_amdgcn_kernarg_segment_ptr());
+    touch_lines<sizeof(DevParams)>((cvoid*)(st.ptab + blockIdx.x));
     CParams& p = *(CParams*)(st.ptab + blockIdx.x);
     const uint32_t wb0 = p.base / ADJ_PPB, nwb = p.npad / ADJ_PPB;
     const uint32_t nwg = st.ntot / ADJ_PPB;

@@ -36,9 +36,8 @@ constexpr int ADJ_NBPARAM = 4;
 // velocity and acceleration the step leaves, and of the force sum it reads.
 constexpr int ADJ_WALL = 4;
 
-// What the forward pass recorded for one step.  The state is in the step's
-// sorted order; rows and displacements are original-index rows; indices
-// are batch indices.
+// What the forward pass recorded for one step, in the step's sorted order;
+// indices are batch indices.
 struct AdjStep {
     const DevParams* ptab;     // per-simulation parameters (device)
     const uint32_t* chunk_sim; // simulation of each 256-particle chunk
@@ -49,9 +48,10 @@ struct AdjStep {
     const double4* w;          // angular velocities
     const uint32_t* perm;      // sorted index -> original index
     const double4* dt0;        // ntot x NC tangential displacements before the step
-    const uint32_t* srt;       // ntot x NC the partner's sorted index, per contact
     const uint32_t* rows;      // ntot x NC contact rows after the interaction pass
-    const uint32_t* prev_rows; // the previous step's rows, or null on the first step
+                               //   (partners by sorted index)
+    const uint2* prev;         // slots that held a partner before the step | those
+                               //   that still hold it
     const double4* wall_nx;    // walls at the step start (all simulations' walls)
     const double4* wall_mvfd;
     int first;                 // the run's first step (acc0 = 0)
@@ -79,9 +79,10 @@ struct AdjState {
     const double4* Laa_out;
     double4* La_in;          // of the accelerations it read (acc0)
     double4* Laa_in;
-    const double4* Ldt_in;   // ntot x NC: of the displacements the step writes
+    const double4* Ldt_in;   // ntot x NC (original-index rows): of the displacements
+                             //   the step writes
     double4* Ldt_out;        // ntot x NC: of the displacements the step read, at the
-                             //   slots occupied in prev_rows
+                             //   slots that held a partner before it
     double* part;            // ADJ_NPART partial sums of every adjoint workgroup,
                              //   quantity by quantity
     double* gparam;          // nsim x ADJ_NPARAM, accumulated over the steps

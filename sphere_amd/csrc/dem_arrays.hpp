@@ -87,16 +87,17 @@ struct DevArrays {
     uint32_t* crow;      // packed partner index (in perm_rows' order) + image code
     uint32_t* perm_rows; // the order the row words index: sorted index -> original
     double4* delta_t;    // tangential displacement per slot (w unused)
-    // Recording for the adjoint (null otherwise): the contact pass writes
-    // its rows and, per contact, the displacement before the step and the
-    // partner's sorted index (original-index rows); the state the step
-    // starts from and the order, in sorted order; the walls.  The bond pass
+    // Recording for the adjoint (null otherwise), in the step's sorted order:
+    // the contact pass writes its rows (partners by sorted index), per
+    // particle the slots that held a partner when the step began and those
+    // that still hold it, per contact the displacement before the step; the
+    // state the step starts from and the order; the walls.  The bond pass
     // writes each bond's inputs (x, v, w of both particles, displacement
     // and rotation; 8 per bond), its particles and whether it applied
     // forces, and the bond gather whether particle nb0 scanned every bond.
     uint32_t* tape_rows;
+    uint2* tape_prev;
     double4* tape_dt0;
-    uint32_t* tape_srt;
     uint32_t* tape_perm;
     double4* tape_x;
     double4* tape_v;

@@ -11,6 +11,7 @@
 #include "dem_arrays.hpp"
 #include "dem_kernels.hpp"
 #include "dem_math.hpp"
+#include "dem_scalar.hpp"
 #include "dem_types.hpp"
 
 namespace sphx {
@@ -24,37 +25,6 @@ constexpr double PI = 3.14159265358979;  // src/constants.h:14
 // uniform fields become scalar loads that stores to global memory do not
 // invalidate, instead of vector loads reissued after every store.
 typedef const __attribute__((address_space(4))) DevParams CParams;
-
-// Scalar loads of one word of each 64-byte line of [ptr, ptr + BYTES), all in
-// flight together.  The compiler reads kernel arguments, parameters and loop
-// state where they are used, each read waiting for a line the scalar cache
-// has not seen in this launch; after one such pass they all hit.  Measured
-// with the contact pass's first loads ungated (no chunk map for one
-// simulation, list entries and position requested with the original index):
-// contact 13.3 -> 11.4 us on 601 particles, 26.2 -> 23.9 on 1e5; integration
-// 6.2 -> 5.8 and walls 3.3 -> 3.0 on 601.
-typedef const __attribute__((address_space(4))) void cvoid;
-template <uint32_t BYTES, uint32_t BYTES2 = 0>
-__device__ __forceinline__ void touch_lines(cvoid* ptr, cvoid* ptr2 = nullptr) {
-    // A structure need not start on a line: its last word is read as well.
-    constexpr uint32_t n = (BYTES + 63) / 64 + 1, n2 = BYTES2 ? (BYTES2 + 63) / 64 + 1 : 0;
-    static_assert(n + n2 <= 12, "at most 12 lines");
-    const auto* w = (const __attribute__((address_space(4))) uint32_t*)ptr;
-    const auto* w2 = (const __attribute__((address_space(4))) uint32_t*)ptr2;
-    uint32_t v[12];
-#pragma unroll
-    for (uint32_t k = 0; k < 12; ++k) {
-        const uint32_t at = 16 * k < (BYTES - 4) / 4 ? 16 * k : (BYTES - 4) / 4;
-        v[k] = w[at];
-        if constexpr (BYTES2 > 0) {
-            const uint32_t k2 = k < n ? 0 : k - n;
-            const uint32_t at2 = 16 * k2 < (BYTES2 - 4) / 4 ? 16 * k2 : (BYTES2 - 4) / 4;
-            if (k >= n) v[k] = w2[at2];
-        }
-    }
-    asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]), "s"(v[6]),
-                 "s"(v[7]), "s"(v[8]), "s"(v[9]), "s"(v[10]), "s"(v[11]));
-}
 
 // The walls' state: only the wall pass writes it, so the kernels before it
 // in a step read it through the constant address space as well.
@@ -790,12 +760,14 @@ __device__ __forceinline__ uint32_t word_to_current(const DevArrays& a, uint32_t
     return (w & ~CW_IDX_MASK) | a.rank[a.perm_rows[idx]];
 }
 
-// A row word of the current sorted order mapped to the partner's original
-// index (the adjoint's tape keeps original indices).
-__device__ __forceinline__ uint32_t word_to_orig(const DevArrays& a, uint32_t w) {
-    const uint32_t idx = w & CW_IDX_MASK;
-    if (idx == EMPTY) return w;
-    return (w & ~CW_IDX_MASK) | a.perm[idx];
+// The adjoint's record of slot i, whose word was w0 when the step began and
+// is w1 now (both in the current order): whether it held a partner, and
+// whether it holds the same one.
+__device__ __forceinline__ void tape_slot(uint32_t w0, uint32_t w1, int i, uint32_t& held,
+                                          uint32_t& same) {
+    const uint32_t p0 = w0 & CW_IDX_MASK;
+    if (p0 != EMPTY) held |= 1u << i;
+    if (p0 != EMPTY && p0 == (w1 & CW_IDX_MASK)) same |= 1u << i;
 }
 
 // The state the contact passes read by sorted index: the step's sorted
@@ -1106,10 +1078,7 @@ __global__ __launch_bounds__(BLOCK, CONTACT_MIN_BLOCKS) void k_contact(const Dev
                     const double4 vel_b = S.v[rb_j];
                     const d3 angvel_b = xyz(S.w[rb_j]);
                     const double4 dt0 = a.delta_t[mp];
-                    if (a.tape_dt0) {
-                        a.tape_dt0[mp] = dt0;
-                        a.tape_srt[mp] = rb_s;
-                    }
+                    if (a.tape_dt0) a.tape_dt0[(size_t)ia * NC + i] = dt0;
                     d3 nd;
                     Contrib C;
                     contrib_init(C);
@@ -1132,13 +1101,20 @@ __global__ __launch_bounds__(BLOCK, CONTACT_MIN_BLOCKS) void k_contact(const Dev
                 a.delta_t[mp] = make_double4(0.0, 0.0, 0.0, 0.0);
             }
         }
+        if (a.tape_rows) {
+            uint32_t held = 0, same = 0;
+            for (int i = 0; i < NC; ++i) {
+                uint32_t w0 = a.crow[(size_t)ia_orig * NC + i];
+                if (lp->order_changed != 0u) w0 = word_to_current(a, w0);
+                tape_slot(w0, row[i], i, held, same);
+                a.tape_rows[(size_t)ia * NC + i] = row[i];
+            }
+            a.tape_prev[ia] = make_uint2(held, same);
+        }
         uint4* wrow = reinterpret_cast<uint4*>(a.crow + (size_t)ia_orig * NC);
 #pragma unroll
         for (int q = 0; q < NC / 4; ++q)
             wrow[q] = make_uint4(row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]);
-        if (a.tape_rows)
-            for (int i = 0; i < NC; ++i)
-                a.tape_rows[(size_t)ia_orig * NC + i] = word_to_orig(a, row[i]);
     }
     walls_and_outputs(p, a, A, xa, vel_a, av_a, Lz, ia_orig, 4);
 }
@@ -2030,10 +2006,8 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
             const double len = length(xab);
             const double dn = len - (rc + rb);
             if (dn < 0.0) {
-                if (a.tape_dt0) {
-                    a.tape_dt0[mp] = dt0;
-                    a.tape_srt[mp] = rb_s;
-                }
+                // (The wavefront's particles are consecutive in sorted order.)
+                if (a.tape_dt0) a.tape_dt0[(size_t)(ia - gw + h) * NC + sidx] = dt0;
                 d3 nd;
                 if constexpr (CM == 2)
                     nd = contact_linear(p, C, vel_c, xyz(av_c), vel_b, xyz(av_b), rc, rb, xab,
@@ -2106,13 +2080,21 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const bool any_ended = ended;
     if (quiet && any_ended && g.q == 0) a.vcount[ia] = make_uint2(vcnt, 0u);
     wave_sync();
+    if (a.tape_rows) {
+        uint32_t held = 0, same = 0;
+#pragma unroll
+        for (int k = 0; k < SPL; ++k) {
+            uint32_t w0 = a.crow[(size_t)ia_orig * NC + g.q * SPL + k];
+            if (remap) w0 = word_to_current(a, w0);
+            tape_slot(w0, gs[g.q * SPL + k], (int)g.q * SPL + k, held, same);
+        }
+        copy_words<SPL>(a.tape_rows + (size_t)ia * NC + g.q * SPL, gs + g.q * SPL);
+        held = group_or<LPP>(held);
+        same = group_or<LPP>(same);
+        if (g.q == 0) a.tape_prev[ia] = make_uint2(held, same);
+    }
     if (!quiet || any_ended || remap)
         copy_words<SPL>(a.crow + (size_t)ia_orig * NC + g.q * SPL, gs + g.q * SPL);
-    if (a.tape_rows) {
-#pragma unroll
-        for (int k = 0; k < SPL; ++k)
-            a.tape_rows[(size_t)ia_orig * NC + g.q * SPL + k] = word_to_orig(a, gs[g.q * SPL + k]);
-    }
     walls_and_outputs(p, a, A, xa_o, vel_o, av_o, Lz, ia_orig, g.q < 4 ? (int)g.q : -1);
     if constexpr (FUSED) {
         // The particle's force and torque are final (its own row and the
@@ -3029,17 +3011,6 @@ __global__ __launch_bounds__(BLOCK) void k_check_sqrt32(unsigned long long* bad,
 
 }  // namespace
 
-// Contact rows whose words index the order of perm_rows, rewritten with the
-// partners' original indices.
-__global__ __launch_bounds__(BLOCK) void k_rows_to_orig(const uint32_t* __restrict__ rows,
-                                                       const uint32_t* __restrict__ perm_rows,
-                                                       uint32_t* __restrict__ out, uint32_t n) {
-    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t w = rows[i], idx = w & CW_IDX_MASK;
-    out[i] = idx == EMPTY ? w : (w & ~CW_IDX_MASK) | perm_rows[idx];
-}
-
 // ---------------------------------------------------------------------------
 // Launch wrappers
 
@@ -3163,14 +3134,6 @@ hipError_t launch_walls(const DevArrays& a, int resort, int passes, int bits, in
                         hipStream_t s) {
     hipLaunchKernelGGL(k_walls, dim3(a.nsim), dim3(WALLS_WG), 0, s, a, resort, passes, bits,
                        sorted_bits);
-    return hipGetLastError();
-}
-
-hipError_t launch_rows_to_orig(const uint32_t* rows, const uint32_t* perm_rows, uint32_t* out,
-                               uint32_t n, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rows_to_orig, dim3(n_blocks(n)), dim3(BLOCK), 0, s, rows, perm_rows,
-                       out, n);
     return hipGetLastError();
 }
 

@@ -2225,12 +2225,12 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     const size_t ntot = A.ntot, nc = ntot * NC, nb = A.nbond;
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     // Tape per step: x, v, w at the step start and the order (sorted), the
-    // displacements of the step's contacts before it and their partners'
-    // sorted indices (written by the contact pass, at their slots), the
-    // walls, the rows the contact pass left, and the bonds' inputs.
+    // displacements of the step's contacts before it (written by the contact
+    // pass, at their slots), the walls, the rows the contact pass left and
+    // which of their slots were held before, and the bonds' inputs.
     const size_t per_step = up(ntot * 3 * sizeof(double4)) + up(ntot * 4) +
-                            up(nc * sizeof(double4)) + up(nc * 4) +
-                            up(2 * nwt * sizeof(double4)) + up(nc * 4) +
+                            up(nc * sizeof(double4)) + up(2 * nwt * sizeof(double4)) +
+                            up(nc * 4) + up(ntot * sizeof(uint2)) +
                             (nb ? up(nb * 8 * sizeof(double4)) + up(nb * sizeof(uint4)) +
                                       up(nsim * 4)
                                 : 0);
@@ -2243,7 +2243,7 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
                            up(4 * nb * sizeof(double4)) + up(6 * nb * sizeof(double4)) +
                            up(nb * ADJ_NBPARAM * 8) + up(nwg * ADJ_NPART * 8) +
                            up(nsim * ADJ_NPARAM * 8) + up(nwt * ADJ_WALL * 8 + 8) +
-                           up(rows * 3 * sizeof(double)) + up(nc * 4) + 256;
+                           up(rows * 3 * sizeof(double)) + 256;
     // A checkpoint: every device allocation of the context.
     size_t snap_b = 0;
     for (size_t b : c->alloc_bytes) snap_b += up(b);
@@ -2295,7 +2295,8 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     char* tape = static_cast<char*>(c->adj_buf);
     struct Rec {
         double4 *x, *v, *w, *dt0, *wnx, *wmv, *bond_in;
-        uint32_t *perm, *srt, *rows, *bond_full;
+        uint32_t *perm, *rows, *bond_full;
+        uint2* prev;
         uint4* bond_idx;
     };
     std::vector<Rec> rec(K);
@@ -2310,13 +2311,13 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
         q += up(ntot * 4);
         r.dt0 = reinterpret_cast<double4*>(q);
         q += up(nc * sizeof(double4));
-        r.srt = reinterpret_cast<uint32_t*>(q);
-        q += up(nc * 4);
         r.wnx = reinterpret_cast<double4*>(q);
         r.wmv = r.wnx + nwt;
         q += up(2 * nwt * sizeof(double4));
         r.rows = reinterpret_cast<uint32_t*>(q);
         q += up(nc * 4);
+        r.prev = reinterpret_cast<uint2*>(q);
+        q += up(ntot * sizeof(uint2));
         r.bond_in = nullptr;
         r.bond_idx = nullptr;
         r.bond_full = nullptr;
@@ -2364,8 +2365,6 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     g.wall = reinterpret_cast<double*>(take(nwt * ADJ_WALL * 8 + 8));
     g.asym = reinterpret_cast<uint32_t*>(g.wall + nwt * ADJ_WALL);
     double* stage = reinterpret_cast<double*>(take(rows * 3 * sizeof(double)));
-    // A checkpoint's rows with the partners' original indices (the tape's).
-    uint32_t* prev_orig = reinterpret_cast<uint32_t*>(take(nc * 4));
     char* snaps = tape + K * per_step + state_b;  // (nseg + 1) checkpoints when nseg > 1
     AdjStep base_st;
     memset(&base_st, 0, sizeof base_st);
@@ -2407,11 +2406,6 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     if (plan) marks = plan->marks;
     else marks.resize(nseg > 1 ? nseg + 1 : 0);
     using HostMark = AdjHostMark;
-    size_t crow_off = 0, prow_off = 0;
-    for (size_t k = 0, off = 0; k < c->allocs.size(); off += up(c->alloc_bytes[k]), ++k) {
-        if (c->allocs[k] == (void*)A.crow) crow_off = off;
-        if (c->allocs[k] == (void*)A.perm_rows) prow_off = off;
-    }
     auto checkpoint = [&](uint64_t m, bool save) -> int {
         char* cbase = snaps + m * snap_b;
         size_t off = 0;
@@ -2469,7 +2463,7 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             const Rec& r = rec[k];
             A.tape_rows = r.rows;
             A.tape_dt0 = r.dt0;
-            A.tape_srt = r.srt;
+            A.tape_prev = r.prev;
             A.tape_perm = r.perm;
             A.tape_x = r.x;
             A.tape_v = r.v;
@@ -2480,7 +2474,8 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             A.tape_bond_idx = r.bond_idx;
             A.tape_bond_full = r.bond_full;
             rc_ = enqueue_step(c);
-            A.tape_rows = A.tape_srt = A.tape_perm = A.tape_bond_full = nullptr;
+            A.tape_rows = A.tape_perm = A.tape_bond_full = nullptr;
+            A.tape_prev = nullptr;
             A.tape_dt0 = A.tape_x = A.tape_v = A.tape_w = A.tape_wnx = A.tape_wmv = nullptr;
             A.tape_bond_in = nullptr;
             A.tape_bond_idx = nullptr;
@@ -2488,10 +2483,9 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
         }
         return rc_;
     };
-    // Reverse of the recorded steps [k0, k0 + n), last first.  prev0: the
-    // rows before step k0 (null for the run's first step).
+    // Reverse of the recorded steps [k0, k0 + n), last first.
     int cur = 0;
-    auto reverse = [&](uint64_t k0, uint64_t n, const uint32_t* prev0) -> int {
+    auto reverse = [&](uint64_t k0, uint64_t n) -> int {
         for (uint64_t kk = n; kk-- > 0;) {
             const Rec& r = rec[kk];
             const uint64_t gk = k0 + kk;
@@ -2501,9 +2495,8 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             st.w = r.w;
             st.perm = r.perm;
             st.dt0 = r.dt0;
-            st.srt = r.srt;
             st.rows = r.rows;
-            st.prev_rows = kk > 0 ? rec[kk - 1].rows : prev0;
+            st.prev = r.prev;
             st.wall_nx = r.wnx;
             st.wall_mvfd = r.wmv;
             st.bond_in = r.bond_in;
@@ -2579,24 +2572,13 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     }
     // The reverse pass.
     if (nseg == 1) {
-        if (!rc) rc = reverse(0, nsteps, nullptr);
+        if (!rc) rc = reverse(0, nsteps);
     } else {
         for (uint64_t m = nseg; m-- > 0 && !rc;) {
             const uint64_t n = std::min<uint64_t>(K, nsteps - m * K);
             rc = checkpoint(m, false);
             if (!rc) rc = record(n, m * K);
-            // The rows before step m K: those the checkpoint's contact rows
-            // hold, with original indices.
-            const uint32_t* prev0 = nullptr;
-            if (m > 0 && !rc) {
-                const char* ck = snaps + m * snap_b;
-                e = launch_rows_to_orig(reinterpret_cast<const uint32_t*>(ck + crow_off),
-                                        reinterpret_cast<const uint32_t*>(ck + prow_off),
-                                        prev_orig, (uint32_t)nc, s);
-                if (e != hipSuccess) return hip_fail(c, e, "checkpoint rows");
-                prev0 = prev_orig;
-            }
-            if (!rc) rc = reverse(m * K, n, prev0);
+            if (!rc) rc = reverse(m * K, n);
         }
         if (!rc) rc = checkpoint(nseg, false);
     }

@@ -128,3 +128,28 @@ def test_resort_of_many_movers(n, movers):
             for f in ("perm", "cellid", "contacts", "x", "vel", "force", "delta_t"):
                 assert numpy.array_equal(ctx.get(f), ref.get(f)), (k, f)
         assert ctx.scalar("sorts") >= 1
+
+
+# The reverse pass's wavefronts of 16 particles: several rounds of evaluations
+# (about 190 contacts a wavefront), a last wavefront with few particles,
+# walls on every side, recorded whole and in segments.
+@pytest.mark.parametrize("kind,checkpoint", [("fcc", 0), ("fcc", 2), (17, 0), (65, 0)])
+def test_adjoint_wavefront_edges(kind, checkpoint):
+    s = cases.fcc_case() if kind == "fcc" else cases.lattice_bed(kind, 3, 0.01, 0.1)
+    n, image, steps = int(s.np[0]), s.tobytes(), 5
+    rng = numpy.random.default_rng(n)
+    cx, cv, dv = (rng.standard_normal((n, 3)) for _ in range(3))
+    with engine.Context(image) as ctx:
+        ctx.set_scalar("adj_checkpoint", checkpoint)
+        g = ctx.adjoint(steps, cx, cv, None)
+    got = {"k_n": g["k_n"], "gamma_t": g["gamma_t"], "v0": float(numpy.sum(g["v"] * dv))}
+    for name, ad in got.items():
+        t = oracle.TangentOracle(image)
+        if name == "v0":
+            t.seed_field("vel", dv)
+        else:
+            t.seed_param(name, 1.0)
+        t.step(steps)
+        want = float(numpy.sum(cx * t.tangent("x")) + numpy.sum(cv * t.tangent("vel")))
+        # Forward against reverse mode: 1e-6, as the other tangent checks.
+        assert abs(ad - want) <= 1e-6 * abs(want), (name, ad, want)
