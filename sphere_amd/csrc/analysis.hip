@@ -67,15 +67,33 @@ __global__ __launch_bounds__(TILE) void k_overlaps(const double4* __restrict__ x
     if (in && !pairs) counts[i] = n;
 }
 
-// Extremes of the positions and radii for the overlap grid, in one
-// workgroup: out = {min x, min y, min z, max x, max y, max z, max r, all
-// finite ? 1 : 0}.
-__global__ __launch_bounds__(1024) void k_overlap_bounds(const double4* __restrict__ x,
-                                                         uint32_t np, double* __restrict__ out) {
-    __shared__ double red[8][1024];
+// ---------------------------------------------------------------------------
+// The overlap list through a uniform grid, without a host round trip before
+// the list's length is known: extremes (many workgroups), the grid from them
+// (one work-item), cell counts, their exclusive scan, the particles copied in
+// cell order, the search (16 work-items per particle, up to OV_SLAB overlaps
+// kept, ordered by j), the exclusive scan of the counts, and the list.  Bound
+// by the launches on small simulations (ten of 3-5 us), by the search on
+// large ones: 100,003 particles 0.10 ms in all, 47 us of it the search; one
+// work-item per particle walking 27 cells through an index took 89 us for
+// each of two passes and 55 on 5,000 (11 here), with the scans on the host
+// between them.
+
+constexpr uint32_t OV_WG = 256;
+constexpr uint32_t OV_CELLS = 8;        // cells per work-item of the scans
+constexpr uint32_t OV_LANES = 16;       // work-items per particle of the search
+constexpr uint32_t OV_SEARCH_WG = 1024;
+constexpr uint32_t OV_FIXED = 0x80000000u;
+static_assert(OV_SEARCH_WG / OV_LANES == OV_PPB, "particles per search workgroup");
+
+__global__ __launch_bounds__(OV_WG) void k_ov_bounds(const double4* __restrict__ x, uint32_t np,
+                                                     OverlapWork w) {
+    __shared__ double red[8][OV_WG / 64];
+    const uint32_t stride = gridDim.x * OV_WG;
+    for (uint32_t c = blockIdx.x * OV_WG + threadIdx.x; c <= w.ncap; c += stride) w.cell_start[c] = 0u;
     double v[8] = {__builtin_inf(), __builtin_inf(), __builtin_inf(), -__builtin_inf(),
                    -__builtin_inf(), -__builtin_inf(), 0.0, 1.0};
-    for (uint32_t i = threadIdx.x; i < np; i += 1024) {
+    for (uint32_t i = blockIdx.x * OV_WG + threadIdx.x; i < np; i += stride) {
         const double4 p = x[i];
         v[0] = fmin(v[0], p.x);
         v[1] = fmin(v[1], p.y);
@@ -88,18 +106,66 @@ __global__ __launch_bounds__(1024) void k_overlap_bounds(const double4* __restri
               __builtin_isfinite(p.w) && p.w >= 0.0))
             v[7] = 0.0;
     }
-    for (int k = 0; k < 8; ++k) red[k][threadIdx.x] = v[k];
-    __syncthreads();
-    for (uint32_t h = 512; h > 0; h >>= 1) {
-        if (threadIdx.x < h) {
-            const uint32_t o = threadIdx.x + h;
-            for (int k = 0; k < 3; ++k) red[k][threadIdx.x] = fmin(red[k][threadIdx.x], red[k][o]);
-            for (int k = 3; k < 7; ++k) red[k][threadIdx.x] = fmax(red[k][threadIdx.x], red[k][o]);
-            red[7][threadIdx.x] = fmin(red[7][threadIdx.x], red[7][o]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        for (int h = 32; h > 0; h >>= 1) {
+            const double o = __shfl_xor(v[k], h, 64);
+            v[k] = (k < 3 || k == 7) ? fmin(v[k], o) : fmax(v[k], o);
         }
-        __syncthreads();
+        if ((threadIdx.x & 63u) == 0) red[k][threadIdx.x / 64u] = v[k];
     }
-    if (threadIdx.x < 8) out[threadIdx.x] = red[threadIdx.x][0];
+    __syncthreads();
+    if (threadIdx.x < 8) {
+        const int k = (int)threadIdx.x;
+        double r = red[k][0];
+        for (uint32_t q = 1; q < OV_WG / 64; ++q)
+            r = (k < 3 || k == 7) ? fmin(r, red[k][q]) : fmax(r, red[k][q]);
+        w.bounds[blockIdx.x * 8 + k] = r;
+    }
+}
+
+// A uniform grid whose cells are at least the largest contact distance
+// (2 r_max, with a margin for the rounding of the cell coordinates) holds
+// every overlapping pair within adjacent cells.  The grid is coarsened until
+// it has at most ncap cells.  Positions that are not finite have no grid.
+__global__ __launch_bounds__(64) void k_ov_grid(uint32_t nblocks, OverlapWork w) {
+    const uint32_t lane = threadIdx.x;
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const bool lower = k < 3 || k == 7;
+        v[k] = w.bounds[k];
+        for (uint32_t b = lane; b < nblocks; b += 64)
+            v[k] = lower ? fmin(v[k], w.bounds[b * 8 + k]) : fmax(v[k], w.bounds[b * 8 + k]);
+        for (int h = 32; h > 0; h >>= 1) {
+            const double o = __shfl_xor(v[k], h, 64);
+            v[k] = lower ? fmin(v[k], o) : fmax(v[k], o);
+        }
+    }
+    if (lane != 0) return;
+    OverlapGrid g;
+    g.use = v[7] == 1.0 ? 1 : 0;
+    double maxabs = 0.0, emax = 0.0, ext[3];
+    for (int d = 0; d < 3; ++d) {
+        maxabs = fmax(maxabs, fmax(fabs(v[d]), fabs(v[3 + d])));
+        ext[d] = v[3 + d] - v[d];
+        emax = fmax(emax, ext[d]);
+        g.lo[d] = v[d];
+        g.n[d] = 1;
+    }
+    double h = 2.0 * v[6] * (1.0 + 1e-6) + 1e-12 * maxabs;
+    if (!(h > 0.0)) h = emax > 0.0 ? emax : 1.0;
+    while (g.use) {
+        uint64_t total = 1;
+        for (int d = 0; d < 3; ++d) {
+            g.n[d] = (int)fmin(ext[d] / h, (double)(1 << 20)) + 1;
+            total *= (uint64_t)g.n[d];
+        }
+        if (total <= (uint64_t)w.ncap) break;
+        h *= 1.5;
+    }
+    g.inv_h = 1.0 / h;
+    *w.grid = g;
 }
 
 __device__ __forceinline__ int grid_coord(double v, double lo, double inv_h, int n) {
@@ -115,90 +181,244 @@ __device__ __forceinline__ uint32_t grid_key(const double4& p, const OverlapGrid
     return ((uint32_t)iz * (uint32_t)g.n[1] + (uint32_t)iy) * (uint32_t)g.n[0] + (uint32_t)ix;
 }
 
-__global__ __launch_bounds__(256) void k_overlap_bin(const double4* __restrict__ x, uint32_t np,
-                                                     OverlapGrid g, uint32_t* __restrict__ key,
-                                                     uint32_t* __restrict__ cell_count) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= np) return;
-    const uint32_t k = grid_key(x[i], g);
-    key[i] = k;
-    atomicAdd(&cell_count[k], 1u);
+// cell_start[c] holds cell c's count until the scan.
+__global__ __launch_bounds__(OV_WG) void k_ov_bin(const double4* __restrict__ x, uint32_t np,
+                                                  OverlapWork w) {
+    const uint32_t i = blockIdx.x * OV_WG + threadIdx.x;
+    if (!w.grid->use || i >= np) return;
+    const uint32_t k = grid_key(x[i], *w.grid);
+    w.key[i] = k;
+    atomicAdd(&w.cell_start[k], 1u);
 }
 
-__global__ __launch_bounds__(256) void k_overlap_scatter(const uint32_t* __restrict__ key,
-                                                         uint32_t np,
-                                                         uint32_t* __restrict__ cursor,
-                                                         uint32_t* __restrict__ order) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= np) return;
-    order[atomicAdd(&cursor[key[i]], 1u)] = i;
+// Exclusive prefix of a value per work-item over the workgroup of T, and the
+// workgroup's total.
+template <typename V, uint32_t T>
+__device__ __forceinline__ V block_exclusive(V v, V& total) {
+    __shared__ V wave_sum[T / 64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x / 64u;
+    V inc = v;
+    for (uint32_t h = 1; h < 64; h <<= 1) {
+        const V o = __shfl_up(inc, h, 64);
+        if (lane >= h) inc += o;
+    }
+    if (lane == 63) wave_sum[wave] = inc;
+    __syncthreads();
+    V before = 0;
+    total = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < T / 64; ++k) {
+        const V s = wave_sum[k];
+        before += k < wave ? s : (V)0;
+        total += s;
+    }
+    __syncthreads();
+    return before + inc - v;
+}
+
+__global__ __launch_bounds__(OV_WG) void k_ov_cell_sums(OverlapWork w) {
+    const uint32_t c0 = (blockIdx.x * OV_WG + threadIdx.x) * OV_CELLS;
+    uint32_t s = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < OV_CELLS; ++k)
+        if (c0 + k <= w.ncap) s += w.cell_start[c0 + k];
+    uint32_t total;
+    (void)block_exclusive<uint32_t, OV_WG>(s, total);
+    if (threadIdx.x == 0) w.cell_sum[blockIdx.x] = total;
+}
+
+// Exclusive scan in place of n block sums by one workgroup; returns the total.
+template <typename V>
+__device__ __forceinline__ V scan_sums(V* v, uint32_t n) {
+    V run = 0;
+    for (uint32_t b = 0; b < n; b += 1024) {
+        const uint32_t k = b + threadIdx.x;
+        const V s = k < n ? v[k] : (V)0;
+        V total;
+        const V pre = block_exclusive<V, 1024>(s, total);
+        if (k < n) v[k] = run + pre;
+        run += total;
+    }
+    return run;
+}
+
+__global__ __launch_bounds__(1024) void k_ov_scan_cells(OverlapWork w, uint32_t n) {
+    (void)scan_sums(w.cell_sum, n);
+}
+
+__global__ __launch_bounds__(1024) void k_ov_scan_counts(OverlapWork w, uint32_t n) {
+    const unsigned long long total = scan_sums(w.block_off, n);
+    if (threadIdx.x == 0) w.grid->total = total;
+}
+
+__global__ __launch_bounds__(OV_WG) void k_ov_cells(OverlapWork w) {
+    const uint32_t c0 = (blockIdx.x * OV_WG + threadIdx.x) * OV_CELLS;
+    uint32_t n[OV_CELLS], s = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < OV_CELLS; ++k) {
+        n[k] = c0 + k <= w.ncap ? w.cell_start[c0 + k] : 0u;
+        s += n[k];
+    }
+    uint32_t total;
+    uint32_t run = block_exclusive<uint32_t, OV_WG>(s, total) + w.cell_sum[blockIdx.x];
+#pragma unroll
+    for (uint32_t k = 0; k < OV_CELLS; ++k) {
+        if (c0 + k > w.ncap) continue;
+        w.cell_start[c0 + k] = run;
+        if (c0 + k < w.ncap) w.cursor[c0 + k] = run;
+        run += n[k];
+    }
+}
+
+// The particles in cell order (any order within a cell), with their index and
+// whether they are fixed (fixvel other than 0 takes part in no overlap).
+__global__ __launch_bounds__(OV_WG) void k_ov_scatter(const double4* __restrict__ x,
+                                                      const double4* __restrict__ vel, uint32_t np,
+                                                      OverlapWork w) {
+    const uint32_t i = blockIdx.x * OV_WG + threadIdx.x;
+    if (!w.grid->use || i >= np) return;
+    const double4 xi = x[i];
+    const bool fixed = !(vel[i].w == 0);
+    const uint32_t pos = atomicAdd(&w.cursor[w.key[i]], 1u);
+    w.cx[pos] = xi;
+    w.cj[pos] = i | (fixed ? OV_FIXED : 0u);
+}
+
+// The cells of row r (0..8: z major, then y) around a particle: their range of
+// particles in cell order.
+__device__ __forceinline__ void cell_row(const OverlapWork& w, const OverlapGrid& g, int cx, int cy,
+                                         int cz, int r, uint32_t& lo, uint32_t& hi) {
+    const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
+    lo = hi = 0;
+    if (y < 0 || y >= g.n[1] || z < 0 || z >= g.n[2]) return;
+    const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < g.n[0] ? cx + 1 : g.n[0] - 1;
+    const uint32_t base = ((uint32_t)z * (uint32_t)g.n[1] + (uint32_t)y) * (uint32_t)g.n[0];
+    lo = w.cell_start[base + (uint32_t)x0];
+    hi = w.cell_start[base + (uint32_t)x1 + 1u];
 }
 
 // The overlap test of DEM::findOverlaps (src/sphere.cpp:694-716) for the
-// j > i in the 27 cells around i's.  Pass 1 (pairs == nullptr) counts;
-// pass 2 writes from offs[i] on and then orders the run by j (insertion
-// sort: a particle has a handful of overlaps), which gives the reference's
-// i-major, j-ascending list whatever order the cells hold.
-__global__ __launch_bounds__(256) void k_overlaps_grid(
-    const double4* __restrict__ x, const double4* __restrict__ vel, uint32_t np, OverlapGrid g,
-    const uint32_t* __restrict__ cell_start, const uint32_t* __restrict__ order,
-    uint32_t* __restrict__ counts, const uint64_t* __restrict__ offs, uint32_t* __restrict__ pairs,
-    double* __restrict__ delta) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= np) return;
-    const double4 xi = x[i];
-    if (vel[i].w != 0) {
-        if (!pairs) counts[i] = 0;
-        return;
-    }
-    const int cx = grid_coord(xi.x, g.lo[0], g.inv_h, g.n[0]);
-    const int cy = grid_coord(xi.y, g.lo[1], g.inv_h, g.n[1]);
-    const int cz = grid_coord(xi.z, g.lo[2], g.inv_h, g.n[2]);
-    uint32_t n = 0;
-    const uint64_t w0 = pairs ? offs[i] : 0;
-    for (int z = cz - 1; z <= cz + 1; ++z) {
-        if (z < 0 || z >= g.n[2]) continue;
-        for (int y = cy - 1; y <= cy + 1; ++y) {
-            if (y < 0 || y >= g.n[1]) continue;
-            for (int xx = cx - 1; xx <= cx + 1; ++xx) {
-                if (xx < 0 || xx >= g.n[0]) continue;
-                const uint32_t c = ((uint32_t)z * (uint32_t)g.n[1] + (uint32_t)y) *
-                                       (uint32_t)g.n[0] + (uint32_t)xx;
-                for (uint32_t k = cell_start[c]; k < cell_start[c + 1]; ++k) {
-                    const uint32_t j = order[k];
-                    if (j <= i) continue;
-                    const double4 xj = x[j];
-                    const double dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-                    const double len = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
-                    const double dn = len - (xi.w + xj.w);
-                    if (dn < 0.0 && vel[j].w == 0) {
-                        if (pairs) {
-                            pairs[2 * (w0 + n)] = i;
-                            pairs[2 * (w0 + n) + 1] = j;
-                            delta[w0 + n] = dn;
-                        }
-                        ++n;
+// j > i in the 27 cells around i's, a row of three cells (one range in cell
+// order) per work-item.  The first OV_SLAB overlaps of a particle are kept in
+// ascending j; a particle with more is searched again when the list is
+// written.
+__global__ __launch_bounds__(OV_SEARCH_WG) void k_ov_search(const double4* __restrict__ x,
+                                                            const double4* __restrict__ vel,
+                                                            uint32_t np, OverlapWork w) {
+    __shared__ uint32_t s_n[OV_PPB];
+    __shared__ uint32_t s_j[OV_PPB][OV_SLAB];
+    __shared__ double s_d[OV_PPB][OV_SLAB];
+    const OverlapGrid g = *w.grid;
+    if (!g.use) return;
+    const uint32_t t = threadIdx.x / OV_LANES, lane = threadIdx.x % OV_LANES;
+    const uint32_t i = blockIdx.x * OV_PPB + t;
+    if (lane == 0) s_n[t] = 0;
+    __syncthreads();
+    const bool in = i < np;
+    if (in && lane < 9 && vel[i].w == 0) {
+        const double4 xi = x[i];
+        const int cx = grid_coord(xi.x, g.lo[0], g.inv_h, g.n[0]);
+        const int cy = grid_coord(xi.y, g.lo[1], g.inv_h, g.n[1]);
+        const int cz = grid_coord(xi.z, g.lo[2], g.inv_h, g.n[2]);
+        uint32_t lo, hi;
+        cell_row(w, g, cx, cy, cz, (int)lane, lo, hi);
+        for (uint32_t k = lo; k < hi; k += 4) {
+            uint32_t jj[4];
+            double4 xj[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t at = k + u < hi ? k + u : k;
+                jj[u] = w.cj[at];
+                xj[u] = w.cx[at];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                if (k + u >= hi || (jj[u] & OV_FIXED) || jj[u] <= i) continue;
+                const double dx = xj[u].x - xi.x, dy = xj[u].y - xi.y, dz = xj[u].z - xi.z;
+                const double len = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
+                const double dn = len - (xi.w + xj[u].w);
+                if (dn < 0.0) {
+                    const uint32_t at = atomicAdd(&s_n[t], 1u);
+                    if (at < OV_SLAB) {
+                        s_j[t][at] = jj[u];
+                        s_d[t][at] = dn;
                     }
                 }
             }
         }
     }
-    if (!pairs) {
-        counts[i] = n;
+    __syncthreads();
+    const uint32_t n = s_n[t];
+    if (in && n <= OV_SLAB && lane < n) {
+        const uint32_t j = s_j[t][lane];
+        uint32_t rank = 0;
+        for (uint32_t k = 0; k < n; ++k) rank += s_j[t][k] < j ? 1u : 0u;
+        w.slab_j[(size_t)i * OV_SLAB + rank] = j;
+        w.slab_d[(size_t)i * OV_SLAB + rank] = s_d[t][lane];
+    }
+    if (in && lane == 0) w.counts[i] = n;
+    if (threadIdx.x < 64) {
+        unsigned long long s = s_n[threadIdx.x];
+        for (int h = 32; h > 0; h >>= 1) s += __shfl_xor(s, h, 64);
+        if (threadIdx.x == 0) w.block_off[blockIdx.x] = s;
+    }
+}
+
+// The list, one wavefront per search workgroup's particles.  Nothing is
+// written when it is longer than `cap`.
+__global__ __launch_bounds__(64) void k_ov_emit(const double4* __restrict__ x, uint32_t np,
+                                                OverlapWork w, uint32_t* __restrict__ pairs,
+                                                double* __restrict__ delta,
+                                                unsigned long long cap) {
+    static_assert(OV_PPB == 64, "a wavefront per block");
+    const OverlapGrid g = *w.grid;
+    if (!g.use || g.total > cap) return;
+    const uint32_t i = blockIdx.x * OV_PPB + threadIdx.x;
+    const uint32_t n = i < np ? w.counts[i] : 0u;
+    uint32_t inc = n;
+    for (uint32_t h = 1; h < 64; h <<= 1) {
+        const uint32_t o = __shfl_up(inc, h, 64);
+        if (threadIdx.x >= h) inc += o;
+    }
+    const unsigned long long w0 = w.block_off[blockIdx.x] + (inc - n);
+    if (n <= OV_SLAB) {
+        for (uint32_t k = 0; k < n; ++k) {
+            pairs[2 * (w0 + k)] = i;
+            pairs[2 * (w0 + k) + 1] = w.slab_j[(size_t)i * OV_SLAB + k];
+            delta[w0 + k] = w.slab_d[(size_t)i * OV_SLAB + k];
+        }
         return;
     }
-    for (uint32_t a = 1; a < n; ++a) {
-        const uint32_t jj = pairs[2 * (w0 + a) + 1];
-        const double dd = delta[w0 + a];
-        uint32_t b = a;
-        while (b > 0 && pairs[2 * (w0 + b - 1) + 1] > jj) {
-            pairs[2 * (w0 + b) + 1] = pairs[2 * (w0 + b - 1) + 1];
-            delta[w0 + b] = delta[w0 + b - 1];
-            --b;
+    const double4 xi = x[i];
+    const int cx = grid_coord(xi.x, g.lo[0], g.inv_h, g.n[0]);
+    const int cy = grid_coord(xi.y, g.lo[1], g.inv_h, g.n[1]);
+    const int cz = grid_coord(xi.z, g.lo[2], g.inv_h, g.n[2]);
+    uint32_t m = 0;
+    for (int r = 0; r < 9; ++r) {
+        uint32_t lo, hi;
+        cell_row(w, g, cx, cy, cz, r, lo, hi);
+        for (uint32_t k = lo; k < hi; ++k) {
+            const uint32_t j = w.cj[k];
+            if ((j & OV_FIXED) || j <= i) continue;
+            const double4 xj = w.cx[k];
+            const double dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+            const double len = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
+            const double dn = len - (xi.w + xj.w);
+            if (dn < 0.0) {
+                // In ascending j among those found so far.
+                uint32_t b = m++;
+                while (b > 0 && pairs[2 * (w0 + b - 1) + 1] > j) {
+                    pairs[2 * (w0 + b) + 1] = pairs[2 * (w0 + b - 1) + 1];
+                    delta[w0 + b] = delta[w0 + b - 1];
+                    --b;
+                }
+                pairs[2 * (w0 + b)] = i;
+                pairs[2 * (w0 + b) + 1] = j;
+                delta[w0 + b] = dn;
+            }
         }
-        pairs[2 * (w0 + b) + 1] = jj;
-        delta[w0 + b] = dd;
     }
+    for (uint32_t k = 0; k < m; ++k) pairs[2 * (w0 + k)] = i;
 }
 
 __device__ __forceinline__ double spherical_cap(double h, double r) {
@@ -264,47 +484,63 @@ __global__ __launch_bounds__(64) void k_porosity(const double4* __restrict__ x, 
 // order (each slice's result is rounded term by term), so the terms are
 // formed apart from it: the wavefronts after the first evaluate a tile of
 // particles each round and leave the terms in LDS, compacted in particle
-// order, while the first work-item subtracts the tile before, sixteen terms
-// read ahead of the adds.  Bound by the rounds (about 1.8 us for 960
+// order, while the first work-item subtracts the tiles before, sixteen terms
+// read ahead of the adds.  Bound by the rounds (about 3.6 us for 1,920
 // particles) and, where a slice holds many particles, by the chain of adds.
-// One work-item per slice took 0.23 us a particle for any number of slices:
-// 100,003 particles in 10 slices 23.6 ms there, 0.20 ms here; 5,000 in 10
-// slices 1.19 ms and 0.02 ms.
+// One work-item per slice took 0.23-0.29 us a particle for any number of
+// slices: 100,003 particles in 12 slices 29.4 ms there, 0.19 ms here; 5,000 in
+// 10 slices 1.26 ms and 0.014 ms.
 constexpr uint32_t PW = 16;                // wavefronts
-constexpr uint32_t PTILE = 64 * (PW - 1);  // particles per round
+constexpr uint32_t PTILE = 64 * (PW - 1);  // particles per tile
+constexpr uint32_t PU = 2;                 // tiles per round
 __global__ __launch_bounds__(64 * PW) void k_porosity_slice(const double4* __restrict__ x,
                                                             uint32_t np, double h_slice,
                                                             double V_slice,
                                                             double* __restrict__ z_pos,
                                                             double* __restrict__ porosity) {
-    __shared__ __align__(16) double term[2 * PTILE + 32];
-    __shared__ uint32_t cnt[2][PW];
+    __shared__ __align__(16) double term[2 * PU * PTILE + 32];
+    __shared__ uint32_t cnt[2][PU * PW];
     const int iz = (int)blockIdx.x;
     const double lo = iz * h_slice;
     const double hi = lo + h_slice;
     const uint32_t wave = threadIdx.x / 64u, lane = threadIdx.x % 64u;
     const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t rounds = (np + PTILE - 1) / PTILE;
+    const uint32_t rounds = (np + PU * PTILE - 1) / (PU * PTILE);
     double V_void = V_slice;
-    uint32_t i = threadIdx.x - 64u;  // the particle of this round (wave > 0)
-    double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
-    if (wave > 0 && i < np) xi = x[i];
-    // Round r evaluates tile r and subtracts tile r - 1.
+    // This round's particles, i and i + PTILE (wave > 0).
+    uint32_t i = threadIdx.x - 64u;
+    double4 xi[PU];
+#pragma unroll
+    for (uint32_t u = 0; u < PU; ++u) {
+        xi[u] = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (wave > 0 && i + u * PTILE < np) xi[u] = x[i + u * PTILE];
+    }
+    if (threadIdx.x < 2 * PU * PW) cnt[threadIdx.x / (PU * PW)][threadIdx.x % (PU * PW)] = 0;
+    __syncthreads();
+    // Round r evaluates its tiles and subtracts those of round r - 1.
     for (uint32_t r = 0; r <= rounds; ++r) {
         const uint32_t h = r & 1u;
-        double t0 = 0.0, t1 = 0.0;
-        int n = 0;
-        uint64_t b0 = 0, b1 = 0;
+        double t0[PU], t1[PU];
+        int n[PU];
+        uint32_t at[PU];
+#pragma unroll
+        for (uint32_t u = 0; u < PU; ++u) n[u] = 0;
         if (wave > 0) {
-            if (i < np) n = slice_terms(xi, lo, hi, t0, t1);
-            b0 = __ballot(n > 0);
-            b1 = __ballot(n > 1);
-            if (lane == 0) cnt[h][wave] = (uint32_t)(__popcll(b0) + __popcll(b1));
-            i += PTILE;
-            if (i < np) xi = x[i];
+#pragma unroll
+            for (uint32_t u = 0; u < PU; ++u) {
+                if (i + u * PTILE < np) n[u] = slice_terms(xi[u], lo, hi, t0[u], t1[u]);
+                const uint64_t b0 = __ballot(n[u] > 0), b1 = __ballot(n[u] > 1);
+                at[u] = (uint32_t)(__popcll(b0 & below) + __popcll(b1 & below));
+                if (lane == 0)
+                    cnt[h][u * PW + wave] = (uint32_t)(__popcll(b0) + __popcll(b1));
+            }
+            i += PU * PTILE;
+#pragma unroll
+            for (uint32_t u = 0; u < PU; ++u)
+                if (i + u * PTILE < np) xi[u] = x[i + u * PTILE];
         } else if (threadIdx.x == 0 && r > 0) {
             uint32_t m = 0;
-            for (uint32_t w = 1; w < PW; ++w) m += cnt[h ^ 1u][w];
+            for (uint32_t w = 0; w < PU * PW; ++w) m += cnt[h ^ 1u][w];
             double a[16], b[16];
 #pragma unroll
             for (int k = 0; k < 16; ++k) a[k] = term[k];
@@ -329,12 +565,14 @@ __global__ __launch_bounds__(64 * PW) void k_porosity_slice(const double4* __res
                 if (j + 16 + k < m) V_void -= b[k];
         }
         __syncthreads();
-        if (n > 0) {
-            uint32_t off = 0;
-            for (uint32_t w = 1; w < wave; ++w) off += cnt[h][w];
-            off += (uint32_t)(__popcll(b0 & below) + __popcll(b1 & below));
-            term[off] = t0;
-            if (n > 1) term[off + 1] = t1;
+#pragma unroll
+        for (uint32_t u = 0; u < PU; ++u) {
+            if (n[u] > 0) {
+                uint32_t off = at[u];
+                for (uint32_t w = 0; w < u * PW + wave; ++w) off += cnt[h][w];
+                term[off] = t0[u];
+                if (n[u] > 1) term[off + 1] = t1[u];
+            }
         }
         __syncthreads();
     }
@@ -354,34 +592,53 @@ hipError_t launch_overlaps(const double4* x, const double4* vel, uint32_t np, ui
     return hipGetLastError();
 }
 
-hipError_t launch_overlap_bounds(const double4* x, uint32_t np, double* out, hipStream_t s) {
-    hipLaunchKernelGGL(k_overlap_bounds, dim3(1), dim3(1024), 0, s, x, np, out);
+size_t overlap_work_layout(uint32_t np, char* base, OverlapWork* w) {
+    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        char* p = base + off;
+        off += up(bytes);
+        return p;
+    };
+    w->ncap = np < 2048u ? 4096u : 2u * np;
+    const size_t cells = w->ncap + 1u;
+    w->grid = (OverlapGrid*)take(sizeof(OverlapGrid));
+    w->bounds = (double*)take(OV_BOUNDS * 64);
+    w->key = (uint32_t*)take((size_t)np * 4);
+    w->cj = (uint32_t*)take((size_t)np * 4);
+    w->cx = (double4*)take((size_t)np * 32);
+    w->counts = (uint32_t*)take((size_t)np * 4);
+    w->slab_j = (uint32_t*)take((size_t)np * OV_SLAB * 4);
+    w->slab_d = (double*)take((size_t)np * OV_SLAB * 8);
+    w->cell_start = (uint32_t*)take(cells * 4);
+    w->cursor = (uint32_t*)take(cells * 4);
+    w->cell_sum = (uint32_t*)take((cells / (OV_WG * OV_CELLS) + 1) * 4);
+    w->block_off = (unsigned long long*)take((np / OV_PPB + 1) * 8);
+    return off;
+}
+
+hipError_t launch_overlap_search(const double4* x, const double4* vel, uint32_t np,
+                                 const OverlapWork& w, hipStream_t s) {
+    const uint32_t nb = (np + OV_WG - 1) / OV_WG;
+    const uint32_t bounds = nb < OV_BOUNDS ? nb : OV_BOUNDS;
+    const uint32_t cb = (w.ncap + 1u + OV_WG * OV_CELLS - 1) / (OV_WG * OV_CELLS);
+    const uint32_t sb = (np + OV_PPB - 1) / OV_PPB;
+    hipLaunchKernelGGL(k_ov_bounds, dim3(bounds), dim3(OV_WG), 0, s, x, np, w);
+    hipLaunchKernelGGL(k_ov_grid, dim3(1), dim3(64), 0, s, bounds, w);
+    hipLaunchKernelGGL(k_ov_bin, dim3(nb), dim3(OV_WG), 0, s, x, np, w);
+    hipLaunchKernelGGL(k_ov_cell_sums, dim3(cb), dim3(OV_WG), 0, s, w);
+    hipLaunchKernelGGL(k_ov_scan_cells, dim3(1), dim3(1024), 0, s, w, cb);
+    hipLaunchKernelGGL(k_ov_cells, dim3(cb), dim3(OV_WG), 0, s, w);
+    hipLaunchKernelGGL(k_ov_scatter, dim3(nb), dim3(OV_WG), 0, s, x, vel, np, w);
+    hipLaunchKernelGGL(k_ov_search, dim3(sb), dim3(OV_SEARCH_WG), 0, s, x, vel, np, w);
+    hipLaunchKernelGGL(k_ov_scan_counts, dim3(1), dim3(1024), 0, s, w, sb);
     return hipGetLastError();
 }
 
-hipError_t launch_overlap_bin(const double4* x, uint32_t np, const OverlapGrid& g, uint32_t* key,
-                              uint32_t* cell_count, hipStream_t s) {
-    if (np == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_overlap_bin, dim3((np + 255) / 256), dim3(256), 0, s, x, np, g, key,
-                       cell_count);
-    return hipGetLastError();
-}
-
-hipError_t launch_overlap_scatter(const uint32_t* key, uint32_t np, uint32_t* cursor,
-                                  uint32_t* order, hipStream_t s) {
-    if (np == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_overlap_scatter, dim3((np + 255) / 256), dim3(256), 0, s, key, np, cursor,
-                       order);
-    return hipGetLastError();
-}
-
-hipError_t launch_overlaps_grid(const double4* x, const double4* vel, uint32_t np,
-                                const OverlapGrid& g, const uint32_t* cell_start,
-                                const uint32_t* order, uint32_t* counts, const uint64_t* offs,
-                                uint32_t* pairs, double* delta, hipStream_t s) {
-    if (np == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_overlaps_grid, dim3((np + 255) / 256), dim3(256), 0, s, x, vel, np, g,
-                       cell_start, order, counts, offs, pairs, delta);
+hipError_t launch_overlap_emit(const double4* x, uint32_t np, const OverlapWork& w,
+                               uint32_t* pairs, double* delta, uint64_t cap, hipStream_t s) {
+    hipLaunchKernelGGL(k_ov_emit, dim3((np + OV_PPB - 1) / OV_PPB), dim3(64), 0, s, x, np, w, pairs,
+                       delta, (unsigned long long)cap);
     return hipGetLastError();
 }
 

@@ -13,28 +13,45 @@ namespace sphx {
 hipError_t launch_overlaps(const double4* x, const double4* vel, uint32_t np, uint32_t* counts,
                            const uint64_t* offs, uint32_t* pairs, double* delta, hipStream_t s);
 
-// Uniform grid for the overlap search: cells of side 1/inv_h >= the largest
+// Uniform grid of the overlap search: cells of side 1/inv_h >= the largest
 // contact distance, n[d] cells per axis from lo[d]; key = (z n1 + y) n0 + x.
 struct OverlapGrid {
     double lo[3];
     double inv_h;
     int n[3];
-    int pad;
+    int use;                   // 0: positions not finite, no grid
+    unsigned long long total;  // overlaps found
 };
 
-// Position/radius extremes (8 doubles: min xyz, max xyz, max r, finite flag).
-hipError_t launch_overlap_bounds(const double4* x, uint32_t np, double* out, hipStream_t s);
-// key[i] = cell of particle i; cell_count[key] += 1 (cell_count zeroed).
-hipError_t launch_overlap_bin(const double4* x, uint32_t np, const OverlapGrid& g, uint32_t* key,
-                              uint32_t* cell_count, hipStream_t s);
-// order[cursor[key[i]]++] = i (cursor = exclusive prefix of the counts).
-hipError_t launch_overlap_scatter(const uint32_t* key, uint32_t np, uint32_t* cursor,
-                                  uint32_t* order, hipStream_t s);
-// launch_overlaps through the grid: same counts, same list.
-hipError_t launch_overlaps_grid(const double4* x, const double4* vel, uint32_t np,
-                                const OverlapGrid& g, const uint32_t* cell_start,
-                                const uint32_t* order, uint32_t* counts, const uint64_t* offs,
-                                uint32_t* pairs, double* delta, hipStream_t s);
+constexpr uint32_t OV_SLAB = 8;      // overlaps kept per particle
+constexpr uint32_t OV_PPB = 64;      // particles per search workgroup
+constexpr uint32_t OV_BOUNDS = 256;  // workgroups of the extremes
+
+// Device arrays of the grid search for up to np particles.
+struct OverlapWork {
+    OverlapGrid* grid;
+    double* bounds;       // OV_BOUNDS x 8 extremes
+    uint32_t* key;        // cell per particle
+    uint32_t* cj;         // index | fixed flag, in cell order
+    double4* cx;          // position and radius, in cell order
+    uint32_t* counts;     // overlaps with j > i
+    uint32_t* slab_j;     // OV_SLAB partners per particle, ascending
+    double* slab_d;
+    uint32_t* cell_start; // ncap + 1
+    uint32_t* cursor;
+    uint32_t* cell_sum;
+    unsigned long long* block_off;
+    uint32_t ncap;        // most cells of the grid
+};
+
+// The arrays placed from `base` on; returns the bytes they take.
+size_t overlap_work_layout(uint32_t np, char* base, OverlapWork* w);
+// The search: afterwards w.grid holds whether the grid served and the total.
+hipError_t launch_overlap_search(const double4* x, const double4* vel, uint32_t np,
+                                 const OverlapWork& w, hipStream_t s);
+// The list of a search, launch_overlaps' list; nothing if it exceeds cap.
+hipError_t launch_overlap_emit(const double4* x, uint32_t np, const OverlapWork& w,
+                               uint32_t* pairs, double* delta, uint64_t cap, hipStream_t s);
 
 // DEM::porosity of z_slices slices of height h_slice (volume V_slice).
 hipError_t launch_porosity(const double4* x, uint32_t np, int z_slices, double h_slice,

@@ -183,6 +183,12 @@ struct sph_ctx {
     void* adj_buf = nullptr;
     size_t adj_bytes = 0;
     AdjPlan* adj_plan = nullptr;  // a recorded forward pass awaiting its reverse
+    // The readers' device arrays and page-locked staging (kept between calls).
+    void* rd_work = nullptr;
+    size_t rd_work_bytes = 0;
+    void* rd_list = nullptr;
+    size_t rd_list_bytes = 0;
+    void* rd_stage = nullptr;
     uint64_t adj_checkpoint = 0;
     // Contact and integration in one pass where the step allows it (off by
     // default: measured slower than the two kernels, 72.1 + 6.2 us for the
@@ -2816,6 +2822,9 @@ void sph_close(sph_ctx* c) {
     }
     for (void* p : c->allocs) (void)hipFree(p);
     if (c->adj_buf) (void)hipFree(c->adj_buf);
+    if (c->rd_work) (void)hipFree(c->rd_work);
+    if (c->rd_list) (void)hipFree(c->rd_list);
+    if (c->rd_stage) (void)hipHostFree(c->rd_stage);
     delete c->adj_plan;
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -2825,29 +2834,54 @@ const char* sph_last_error(const sph_ctx* c) { return c ? c->err.c_str() : g_ope
 const char* sph_open_error(void) { return g_open_error.c_str(); }
 const char* sph_version_string(void) { return "sphere_hip 0.1 (.bin 2.15, gfx950)"; }
 
-int sph_find_overlaps(sph_ctx* c, int sim, uint32_t* pairs, double* overlaps, uint64_t cap,
-                      uint64_t* count) {
-    CHECK_SIM(c, sim);
-    if (!count || (cap && (!pairs || !overlaps))) return SPH_E_ARG;
-    const Sim& S = c->sims[sim];
-    const uint32_t np = S.h.np, b0 = S.P.base;
-    const double4* x = c->A.x + b0;
-    const double4* vel = c->A.vel + b0;
+// The readers' device arrays, kept by the context between calls (up to
+// RD_KEEP bytes) and grown as needed.
+static constexpr size_t RD_KEEP = (size_t)512 << 20;
+
+static int reader_buffer(sph_ctx* c, void** buf, size_t* have, size_t bytes) {
+    if (bytes <= *have) return SPH_OK;
+    if (*buf) {
+        HIPCHK(c, hipStreamSynchronize(c->stream), "sync");
+        (void)hipFree(*buf);
+    }
+    *buf = nullptr;
+    *have = 0;
+    HIPCHK(c, hipMalloc(buf, bytes), "hipMalloc");
+    *have = bytes;
+    return SPH_OK;
+}
+
+static void trim_readers(sph_ctx* c) {
+    if (c->rd_work_bytes + c->rd_list_bytes <= RD_KEEP) return;
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(c->rd_work);
+    (void)hipFree(c->rd_list);
+    c->rd_work = c->rd_list = nullptr;
+    c->rd_work_bytes = c->rd_list_bytes = 0;
+}
+
+// Page-locked staging for the readers' small results (kept by the context).
+static constexpr size_t RD_STAGE = 64 << 10;
+static char* reader_stage(sph_ctx* c) {
+    if (!c->rd_stage && hipHostMalloc(&c->rd_stage, RD_STAGE, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->rd_stage = nullptr;
+    }
+    return static_cast<char*>(c->rd_stage);
+}
+
+// The all-pairs search, for positions that are not finite.
+static int overlaps_all_pairs(sph_ctx* c, const double4* x, const double4* vel, uint32_t np,
+                              uint32_t* pairs, double* overlaps, uint64_t cap,
+                              uint64_t* count) {
     hipStream_t s = c->stream;
     uint32_t* counts = nullptr;
     uint64_t* offs = nullptr;
     uint32_t* dpairs = nullptr;
     double* ddelta = nullptr;
-    double* dbounds = nullptr;
-    uint32_t* key = nullptr;
-    uint32_t* cells = nullptr;
-    uint32_t* cursor = nullptr;
-    uint32_t* order = nullptr;
     auto release = [&]() {
         (void)hipStreamSynchronize(s);
-        for (void* p : {(void*)counts, (void*)offs, (void*)dpairs, (void*)ddelta, (void*)dbounds,
-                        (void*)key, (void*)cells, (void*)cursor, (void*)order})
-            (void)hipFree(p);
+        for (void* p : {(void*)counts, (void*)offs, (void*)dpairs, (void*)ddelta}) (void)hipFree(p);
     };
 #define AFAIL(e_, what)                        \
     do {                                       \
@@ -2857,72 +2891,9 @@ int sph_find_overlaps(sph_ctx* c, int sim, uint32_t* pairs, double* overlaps, ui
             return hip_fail(c, ee_, what);     \
         }                                      \
     } while (0)
-    AFAIL(hipMalloc(&counts, (size_t)np * 4 + 4), "hipMalloc");
-    AFAIL(hipMalloc(&offs, (size_t)np * 8 + 8), "hipMalloc");
-
-    // A uniform grid whose cells are at least the largest contact distance
-    // (2 r_max, with a margin for the rounding of the cell coordinates)
-    // holds every overlapping pair within adjacent cells.  The grid is
-    // coarsened until it has at most max(2 np, 4096) cells.  Positions that
-    // are not finite fall back to the all-pairs search.
-    double bounds[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (np >= 2) {
-        AFAIL(hipMalloc(&dbounds, 64), "hipMalloc");
-        AFAIL(launch_overlap_bounds(x, np, dbounds, s), "overlap bounds");
-        AFAIL(hipMemcpyAsync(bounds, dbounds, 64, hipMemcpyDeviceToHost, s), "D2H");
-        AFAIL(hipStreamSynchronize(s), "sync");
-    }
-    const bool use_grid = np >= 2 && bounds[7] == 1.0;
-    OverlapGrid g{};
-    if (use_grid) {
-        double maxabs = 0.0, emax = 0.0, ext[3];
-        for (int d = 0; d < 3; ++d) {
-            maxabs = std::max(maxabs, std::max(std::fabs(bounds[d]), std::fabs(bounds[3 + d])));
-            ext[d] = bounds[3 + d] - bounds[d];
-            emax = std::max(emax, ext[d]);
-            g.lo[d] = bounds[d];
-        }
-        double h = 2.0 * bounds[6] * (1.0 + 1e-6) + 1e-12 * maxabs;
-        if (!(h > 0.0)) h = emax > 0.0 ? emax : 1.0;
-        const uint64_t limit = std::max<uint64_t>(2ull * np, 4096);
-        for (;;) {
-            uint64_t total = 1;
-            for (int d = 0; d < 3; ++d) {
-                g.n[d] = (int)std::min(ext[d] / h, (double)(1 << 20)) + 1;
-                total *= (uint64_t)g.n[d];
-            }
-            if (total <= limit) break;
-            h *= 1.5;
-        }
-        g.inv_h = 1.0 / h;
-        const size_t ncells = (size_t)g.n[0] * g.n[1] * g.n[2];
-        AFAIL(hipMalloc(&key, (size_t)np * 4), "hipMalloc");
-        AFAIL(hipMalloc(&order, (size_t)np * 4), "hipMalloc");
-        AFAIL(hipMalloc(&cells, (ncells + 1) * 4), "hipMalloc");
-        AFAIL(hipMalloc(&cursor, ncells * 4), "hipMalloc");
-        AFAIL(hipMemsetAsync(cursor, 0, ncells * 4, s), "memset");
-        AFAIL(launch_overlap_bin(x, np, g, key, cursor, s), "overlap bin");
-        std::vector<uint32_t> start(ncells + 1);
-        AFAIL(hipMemcpyAsync(start.data(), cursor, ncells * 4, hipMemcpyDeviceToHost, s), "D2H");
-        AFAIL(hipStreamSynchronize(s), "sync");
-        uint32_t run = 0;
-        for (size_t k = 0; k < ncells; ++k) {
-            const uint32_t n = start[k];
-            start[k] = run;
-            run += n;
-        }
-        start[ncells] = run;
-        AFAIL(hipMemcpyAsync(cells, start.data(), (ncells + 1) * 4, hipMemcpyHostToDevice, s),
-              "H2D");
-        AFAIL(hipMemcpyAsync(cursor, cells, ncells * 4, hipMemcpyDeviceToDevice, s), "D2D");
-        AFAIL(launch_overlap_scatter(key, np, cursor, order, s), "overlap scatter");
-        AFAIL(hipStreamSynchronize(s), "sync");
-    }
-    auto search = [&](const uint64_t* o, uint32_t* p, double* dl) {
-        return use_grid ? launch_overlaps_grid(x, vel, np, g, cells, order, counts, o, p, dl, s)
-                        : launch_overlaps(x, vel, np, counts, o, p, dl, s);
-    };
-    AFAIL(search(nullptr, nullptr, nullptr), "overlaps");
+    AFAIL(hipMalloc(&counts, (size_t)np * 4), "hipMalloc");
+    AFAIL(hipMalloc(&offs, (size_t)np * 8), "hipMalloc");
+    AFAIL(launch_overlaps(x, vel, np, counts, nullptr, nullptr, nullptr, s), "overlaps");
     std::vector<uint32_t> hc(np);
     std::vector<uint64_t> ho(np);
     AFAIL(hipMemcpyAsync(hc.data(), counts, (size_t)np * 4, hipMemcpyDeviceToHost, s), "D2H");
@@ -2938,7 +2909,7 @@ int sph_find_overlaps(sph_ctx* c, int sim, uint32_t* pairs, double* overlaps, ui
         AFAIL(hipMemcpyAsync(offs, ho.data(), (size_t)np * 8, hipMemcpyHostToDevice, s), "H2D");
         AFAIL(hipMalloc(&dpairs, total * 8), "hipMalloc");
         AFAIL(hipMalloc(&ddelta, total * 8), "hipMalloc");
-        AFAIL(search(offs, dpairs, ddelta), "overlaps");
+        AFAIL(launch_overlaps(x, vel, np, counts, offs, dpairs, ddelta, s), "overlaps");
         AFAIL(hipMemcpyAsync(pairs, dpairs, take * 8, hipMemcpyDeviceToHost, s), "D2H");
         AFAIL(hipMemcpyAsync(overlaps, ddelta, take * 8, hipMemcpyDeviceToHost, s), "D2H");
     }
@@ -2947,41 +2918,117 @@ int sph_find_overlaps(sph_ctx* c, int sim, uint32_t* pairs, double* overlaps, ui
     return SPH_OK;
 }
 
+int sph_find_overlaps(sph_ctx* c, int sim, uint32_t* pairs, double* overlaps, uint64_t cap,
+                      uint64_t* count) {
+    CHECK_SIM(c, sim);
+    if (!count || (cap && (!pairs || !overlaps))) return SPH_E_ARG;
+    const Sim& S = c->sims[sim];
+    const uint32_t np = S.h.np, b0 = S.P.base;
+    const double4* x = c->A.x + b0;
+    const double4* vel = c->A.vel + b0;
+    hipStream_t s = c->stream;
+    *count = 0;
+    if (np < 2) return SPH_OK;
+    OverlapWork w;
+    int rc = reader_buffer(c, &c->rd_work, &c->rd_work_bytes, overlap_work_layout(np, nullptr, &w));
+    if (rc) return rc;
+    overlap_work_layout(np, static_cast<char*>(c->rd_work), &w);
+    HIPCHK(c, launch_overlap_search(x, vel, np, w, s), "overlaps");
+    // The list goes out with the search, into as much room as a settled bed
+    // takes; a longer one is written again once its length is known.
+    uint64_t room = 0;
+    auto make_room = [&](uint64_t n) {
+        const int r = reader_buffer(c, &c->rd_list, &c->rd_list_bytes, n * 16);
+        room = c->rd_list_bytes / 16;
+        return r;
+    };
+    auto emit = [&]() {
+        uint32_t* dp = static_cast<uint32_t*>(c->rd_list);
+        return launch_overlap_emit(x, np, w, dp, reinterpret_cast<double*>(dp + 2 * room), room, s);
+    };
+    if (cap > 0) {
+        rc = make_room(2 * (uint64_t)np);
+        if (rc) return rc;
+        HIPCHK(c, emit(), "overlaps");
+    }
+    OverlapGrid g;
+    char* stage = reader_stage(c);
+    HIPCHK(c, hipMemcpyAsync(stage ? (void*)stage : (void*)&g, w.grid, sizeof g,
+                             hipMemcpyDeviceToHost, s), "D2H");
+    HIPCHK(c, hipStreamSynchronize(s), "sync");
+    if (stage) memcpy(&g, stage, sizeof g);
+    if (!g.use) return overlaps_all_pairs(c, x, vel, np, pairs, overlaps, cap, count);
+    *count = g.total;
+    const uint64_t take = std::min<uint64_t>(g.total, cap);
+    if (take > 0) {
+        if (g.total > room) {
+            rc = make_room(g.total);
+            if (rc) return rc;
+            HIPCHK(c, emit(), "overlaps");
+        }
+        const uint32_t* dp = static_cast<const uint32_t*>(c->rd_list);
+        HIPCHK(c, hipMemcpyAsync(pairs, dp, take * 8, hipMemcpyDeviceToHost, s), "D2H");
+        HIPCHK(c, hipMemcpyAsync(overlaps, dp + 2 * room, take * 8, hipMemcpyDeviceToHost, s), "D2H");
+        HIPCHK(c, hipStreamSynchronize(s), "sync");
+    }
+    trim_readers(c);
+    return SPH_OK;
+}
+
+// DEM::porosity into z_pos and porosity, the results staged in `d` on the
+// device (2 z_slices doubles; null: the readers' arrays) and, if given, in
+// `stage` (page-locked).
+static int porosity_run(sph_ctx* c, int sim, int z_slices, double* z_pos, double* porosity,
+                        double* d, char* stage) {
+    const Sim& S = c->sims[sim];
+    const uint32_t np = S.h.np, b0 = S.P.base;
+    hipStream_t s = c->stream;
+    double4 local[2];
+    double4* head = stage ? reinterpret_cast<double4*>(stage) : local;
+    head[0] = make_double4(0.0, 0.0, 0.0, S.h.L[2]);
+    head[1] = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (S.h.nw > 0)
+        HIPCHK(c, hipMemcpyAsync(head, c->A.w_nx + S.P.wall_base, 32, hipMemcpyDeviceToHost, s),
+               "D2H");
+    if (np > 0)
+        HIPCHK(c, hipMemcpyAsync(head + 1, c->A.x + b0 + np - 1, 32, hipMemcpyDeviceToHost, s),
+               "D2H");
+    if (S.h.nw > 0 || np > 0) HIPCHK(c, hipStreamSynchronize(s), "sync");
+    const double h_slice = (head[0].w - S.h.origo[2]) / (double)z_slices;
+    // The reference checks the slice height against "r_max()", which
+    // returns the last particle's radius (src/sphere.cpp:474-484).
+    if (h_slice <= head[1].w * 2.0)
+        return fail(c, SPH_E_INPUT, "Error! The number of z-slices is too high.");
+    const double V_slice = h_slice * S.h.L[0] * S.h.L[1];
+    if (!d) {
+        const int rc = reader_buffer(c, &c->rd_list, &c->rd_list_bytes, (size_t)z_slices * 16);
+        if (rc) return rc;
+        d = static_cast<double*>(c->rd_list);
+    }
+    // Every slice's two results are written by the kernel: nothing in the
+    // array needs clearing first.
+    HIPCHK(c, launch_porosity(c->A.x + b0, np, z_slices, h_slice, V_slice, d, d + z_slices, s),
+           "porosity");
+    const size_t bytes = (size_t)z_slices * 8;
+    if (stage && 2 * bytes <= RD_STAGE) {
+        HIPCHK(c, hipMemcpyAsync(stage, d, 2 * bytes, hipMemcpyDeviceToHost, s), "D2H");
+        HIPCHK(c, hipStreamSynchronize(s), "sync");
+        memcpy(z_pos, stage, bytes);
+        memcpy(porosity, stage + bytes, bytes);
+        return SPH_OK;
+    }
+    HIPCHK(c, hipMemcpyAsync(z_pos, d, bytes, hipMemcpyDeviceToHost, s), "D2H");
+    HIPCHK(c, hipMemcpyAsync(porosity, d + z_slices, bytes, hipMemcpyDeviceToHost, s), "D2H");
+    HIPCHK(c, hipStreamSynchronize(s), "sync");
+    return SPH_OK;
+}
+
 int sph_porosity(sph_ctx* c, int sim, int z_slices, double* z_pos, double* porosity) {
     CHECK_SIM(c, sim);
     if (z_slices <= 0 || !z_pos || !porosity) return SPH_E_ARG;
-    const Sim& S = c->sims[sim];
-    const uint32_t np = S.h.np, b0 = S.P.base;
-    double top = S.h.L[2];
-    if (S.h.nw > 0) {
-        double4 w;
-        int rc = d2h(c, &w, c->A.w_nx + S.P.wall_base, 32);
-        if (rc) return rc;
-        top = w.w;
-    }
-    const double h_slice = (top - S.h.origo[2]) / (double)z_slices;
-    double4 last = make_double4(0.0, 0.0, 0.0, 0.0);
-    if (np > 0) {
-        int rc = d2h(c, &last, c->A.x + b0 + np - 1, 32);
-        if (rc) return rc;
-    }
-    // The reference checks the slice height against "r_max()", which
-    // returns the last particle's radius (src/sphere.cpp:474-484).
-    if (h_slice <= last.w * 2.0)
-        return fail(c, SPH_E_INPUT, "Error! The number of z-slices is too high.");
-    const double V_slice = h_slice * S.h.L[0] * S.h.L[1];
-    double* d = nullptr;
-    HIPCHK(c, hipMalloc(&d, (size_t)z_slices * 16), "hipMalloc");
-    hipError_t e = launch_porosity(c->A.x + b0, np, z_slices, h_slice, V_slice, d, d + z_slices,
-                                   c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(z_pos, d, (size_t)z_slices * 8,
-                                            hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(porosity, d + z_slices, (size_t)z_slices * 8,
-                                            hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(d);
-    if (e != hipSuccess) return hip_fail(c, e, "porosity");
-    return SPH_OK;
+    const int rc = porosity_run(c, sim, z_slices, z_pos, porosity, nullptr, reader_stage(c));
+    trim_readers(c);
+    return rc;
 }
 
 int sph_porosity_noalloc(sph_ctx* c, int sim, int z_slices, double* z_pos, double* porosity) {
@@ -2992,36 +3039,7 @@ int sph_porosity_noalloc(sph_ctx* c, int sim, int z_slices, double* z_pos, doubl
                     "sph_porosity_noalloc", z_slices, SPH_POROSITY_NOALLOC_MAX_SLICES);
     double* d = scratch_of(c->device);
     if (!d) return fail(c, SPH_E_DEVICE, "no staging array on device %d", c->device);
-    const Sim& S = c->sims[sim];
-    const uint32_t np = S.h.np, b0 = S.P.base;
-    double top = S.h.L[2];
-    if (S.h.nw > 0) {
-        double4 w;
-        int rc = d2h(c, &w, c->A.w_nx + S.P.wall_base, 32);
-        if (rc) return rc;
-        top = w.w;
-    }
-    const double h_slice = (top - S.h.origo[2]) / (double)z_slices;
-    double4 last = make_double4(0.0, 0.0, 0.0, 0.0);
-    if (np > 0) {
-        int rc = d2h(c, &last, c->A.x + b0 + np - 1, 32);
-        if (rc) return rc;
-    }
-    // src/sphere.cpp:474-484, as in sph_porosity.
-    if (h_slice <= last.w * 2.0)
-        return fail(c, SPH_E_INPUT, "Error! The number of z-slices is too high.");
-    const double V_slice = h_slice * S.h.L[0] * S.h.L[1];
-    // Every slice's two results are written by the kernel: nothing in the
-    // array needs clearing first.
-    hipError_t e = launch_porosity(c->A.x + b0, np, z_slices, h_slice, V_slice, d, d + z_slices,
-                                   c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(z_pos, d, (size_t)z_slices * 8,
-                                            hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(porosity, d + z_slices, (size_t)z_slices * 8,
-                                            hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) return hip_fail(c, e, "porosity");
-    return SPH_OK;
+    return porosity_run(c, sim, z_slices, z_pos, porosity, d, nullptr);
 }
 
 int sph_selftest_sqrt32(int device, uint64_t lo, uint64_t hi, uint64_t* mismatches) {

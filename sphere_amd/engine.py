@@ -261,13 +261,18 @@ class Context:
     def find_overlaps(self, sim=0):
         """DEM::findOverlaps on the GPU (sph_find_overlaps): (pairs (k, 2),
         i < j, ascending; overlaps (k,), negative)."""
+        # One call into as much room as a settled bed takes (about 1.5
+        # overlaps per particle), a second one only for a longer list.
         n = ctypes.c_uint64()
-        self._chk(self._L.sph_find_overlaps(self._h, sim, None, None, 0, ctypes.byref(n)))
-        pairs = numpy.zeros((n.value, 2), dtype=numpy.uint32)
-        delta = numpy.zeros(n.value)
-        self._chk(self._L.sph_find_overlaps(self._h, sim, pairs.ctypes.data, delta.ctypes.data,
-                                            n.value, ctypes.byref(n)))
-        return pairs, delta
+        cap = 2 * int(self.scalar("np", sim=sim))
+        while True:
+            pairs = numpy.empty((cap, 2), dtype=numpy.uint32)
+            delta = numpy.empty(cap)
+            self._chk(self._L.sph_find_overlaps(self._h, sim, pairs.ctypes.data,
+                                                delta.ctypes.data, cap, ctypes.byref(n)))
+            if n.value <= cap:
+                return pairs[:n.value].copy(), delta[:n.value].copy()
+            cap = n.value
 
     def porosity(self, z_slices=10, sim=0):
         """DEM::porosity on the GPU (sph_porosity): (z positions, porosities)."""

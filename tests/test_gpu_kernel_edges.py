@@ -153,3 +153,28 @@ def test_adjoint_wavefront_edges(kind, checkpoint):
         want = float(numpy.sum(cx * t.tangent("x")) + numpy.sum(cv * t.tangent("vel")))
         # Forward against reverse mode: 1e-6, as the other tangent checks.
         assert abs(ad - want) <= 1e-6 * abs(want), (name, ad, want)
+
+
+# Overlap lists: no pair possible, search workgroups of 64 exactly and not,
+# particles with more overlaps than are kept (8), lists longer than two a
+# particle (written a second time), fixed particles, a buffer too short.
+@pytest.mark.parametrize("n,radius", [
+    (1, 0.01), (2, 0.07), (63, 0.03), (64, 0.05), (65, 0.07), (700, 0.03), (2049, 0.02),
+    (5000, 0.004)])
+def test_overlap_list_edges(n, radius):
+    import ctypes
+    s = _cloud(n, 5, r=(0.5 * radius, radius))
+    s.fixvel[::7] = 1.0
+    image = s.tobytes()
+    pb, db = oracle.Oracle(image).find_overlaps()
+    with engine.Context(image) as ctx:
+        for _ in range(2):
+            pa, da = ctx.find_overlaps()
+            assert numpy.array_equal(pa, pb) and numpy.array_equal(da, db)
+        L, m = engine.load(), ctypes.c_uint64()
+        k = len(pb) // 2
+        pairs, delta = numpy.zeros((k, 2), dtype=numpy.uint32), numpy.zeros(k)
+        assert L.sph_find_overlaps(ctx._h, 0, pairs.ctypes.data, delta.ctypes.data, k,
+                                   ctypes.byref(m)) == 0
+        assert m.value == len(pb)
+        assert numpy.array_equal(pairs, pb[:k]) and numpy.array_equal(delta, db[:k])
