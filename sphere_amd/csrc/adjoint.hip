@@ -356,6 +356,9 @@ __global__ __launch_bounds__(256) void k_adj_step(AdjStep st, AdjState g) {
     const uint32_t ia = blockIdx.x * ADJ_PPB + threadIdx.x / ALPP;
     const bool in = ia - p.base < p.np;
     const double dt = p.dt;
+    // The workgroup's sums so far, when the steps accumulate.
+    double* const part = g.part + (size_t)threadIdx.x * gridDim.x + blockIdx.x;
+    const double before = st.accumulate && threadIdx.x < ADJ_NPART ? *part : 0.0;
     PGrad gp;
 #pragma unroll
     for (int k = 0; k < ADJ_NPARAM; ++k) gp.s[k] = 0.0;
@@ -622,7 +625,7 @@ __global__ __launch_bounds__(256) void k_adj_step(AdjStep st, AdjState g) {
     __syncthreads();
     if (threadIdx.x < ADJ_NPART) {
         const int k = threadIdx.x;
-        g.part[(size_t)k * gridDim.x + blockIdx.x] = red[k][0] + red[k][1] + red[k][2] + red[k][3];
+        *part = before + (red[k][0] + red[k][1] + red[k][2] + red[k][3]);
     }
 }
 
@@ -959,13 +962,18 @@ hipError_t launch_adj_pack(double* dst, const double4* src, const AdjStep& st, h
     return hipGetLastError();
 }
 
+hipError_t launch_adj_reduce(const AdjStep& st, const AdjState& g, hipStream_t s) {
+    hipLaunchKernelGGL(k_adj_reduce, dim3(st.nsim), dim3(RED_WG), 0, s, st, g);
+    return hipGetLastError();
+}
+
 hipError_t launch_adj_step(const AdjStep& st, const AdjState& g, hipStream_t s) {
     hipLaunchKernelGGL(k_adj_step, dim3(st.ntot / ADJ_PPB), dim3(256), 0, s, st, g);
     if (st.nbond) {
         hipLaunchKernelGGL(k_adj_bonds, dim3((st.nbond + 255) / 256), dim3(256), 0, s, st, g);
         hipLaunchKernelGGL(k_adj_bond_gather, dim3(st.ntot / 256), dim3(256), 0, s, st, g);
     }
-    hipLaunchKernelGGL(k_adj_reduce, dim3(st.nsim), dim3(RED_WG), 0, s, st, g);
+    if (!st.accumulate) return launch_adj_reduce(st, g, s);
     return hipGetLastError();
 }
 

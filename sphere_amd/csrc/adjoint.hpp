@@ -56,6 +56,8 @@ struct AdjStep {
     const double4* wall_mvfd;
     int first;                 // the run's first step (acc0 = 0)
     int last;                  // the recorded pass's last step (no displacement cotangent)
+    int accumulate;            // the workgroups' partial sums run on over the steps and are
+                               //   reduced once (no wall feels its force sum, no bonds)
     // Bonds (nbond = 0 without): each bond's inputs in this step (x_i, x_j,
     // v_i, v_j, w_i, w_j, delta0, omega0), its particles and whether it
     // applied forces; per simulation whether the bond gather of particle
@@ -84,7 +86,7 @@ struct AdjState {
     double4* Ldt_out;        // ntot x NC: of the displacements the step read, at the
                              //   slots that held a partner before it
     double* part;            // ADJ_NPART partial sums of every adjoint workgroup,
-                             //   quantity by quantity
+                             //   quantity by quantity (zero at first if they run on)
     double* gparam;          // nsim x ADJ_NPARAM, accumulated over the steps
     double* wall;            // total walls x ADJ_WALL reverse state
     uint32_t* asym;          // contacts missing from their partner's row
@@ -103,9 +105,12 @@ hipError_t launch_adj_pack(double* dst, const double4* src, const AdjStep& st, h
 hipError_t launch_adj_accumulate(double4* dst, const double* src, const AdjStep& st,
                                  hipStream_t s);
 // Reverse of one step: particles (contacts, walls, integration), then the
-// bonds and their per-particle gather, then per simulation the fixed-order
-// sums of the partials and the reverse of the walls' equation of motion.
+// bonds and their per-particle gather, then (unless st.accumulate) per
+// simulation the fixed-order sums of the partials and the reverse of the
+// walls' equation of motion.
 hipError_t launch_adj_step(const AdjStep& st, const AdjState& g, hipStream_t s);
+// That last part alone, after the steps of an accumulating pass.
+hipError_t launch_adj_reduce(const AdjStep& st, const AdjState& g, hipStream_t s);
 
 }  // namespace sphx
 

@@ -2379,6 +2379,12 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     base_st.nsim = (uint32_t)nsim;
     base_st.ntot = (uint32_t)ntot;
     base_st.nbond = (uint32_t)nb;
+    // The particles' cotangents need a step's sums only where a wall's motion
+    // depends on its force sum (wmode 1); otherwise they are formed once.
+    bool feedback = nb > 0;
+    for (const Sim& S : c->sims)
+        for (uint32_t w = 0; w < S.h.nw; ++w) feedback = feedback || S.h.wmode[w] == 1;
+    base_st.accumulate = feedback ? 0 : 1;
     base_st.bond_sim = A.bond_sim;
     base_st.badj_off = A.badj_off;
     base_st.badj = A.badj;
@@ -2402,6 +2408,8 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
         e = hipMemsetAsync(LA[0], 0, 2 * ntot * 32, s);  // LA[0], LAA[0]
         if (e == hipSuccess) e = hipMemsetAsync(g.gparam, 0, nsim * ADJ_NPARAM * 8, s);
         if (e == hipSuccess) e = hipMemsetAsync(g.wall, 0, nwt * ADJ_WALL * 8 + 8, s);
+        if (e == hipSuccess && base_st.accumulate)
+            e = hipMemsetAsync(g.part, 0, nwg * ADJ_NPART * 8, s);
         if (e == hipSuccess && nb) e = hipMemsetAsync(lb0, 0, 4 * nb * sizeof(double4), s);
         if (e != hipSuccess) return hip_fail(c, e, "memset");
     }
@@ -2589,6 +2597,12 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
         if (!rc) rc = checkpoint(nseg, false);
     }
     if (rc) return rc;
+    if (base_st.accumulate) {
+        AdjStep st = base_st;
+        st.wall_mvfd = A.w_mvfd;  // (not used by walls without feedback)
+        e = launch_adj_reduce(st, g, s);
+        if (e != hipSuccess) return hip_fail(c, e, "adjoint sums");
+    }
     double* outs[3] = {g_x0, g_v0, g_w0};
     for (int f = 0; f < 3 && !rc; ++f) {
         if (!outs[f] || !rows) continue;
