@@ -334,12 +334,13 @@ int sph_read_state_sim(sph_ctx* ctx, int sim, const char* path);
  * contact workgroup size (128, 256, 512; 4 lanes), the candidate-list
  * capacity (16, 24, 32) and the workgroup order (SPH_S_XCD_ORDER), each
  * judged by the contact kernel's mean time over steps_per_trial steps
- * (HIP events) after steps_per_trial / 2 untimed steps; then the radix
+ * (HIP events; up to 8,192 particles by the step's kernels together) after
+ * steps_per_trial / 2 untimed steps; then the radix
  * digit width (4, 6, 8 bits), judged by four full sorts of the current keys.
  * Every setting gives the same results bit for bit, so the trials are
  * ordinary steps: the simulation advances by 1.5 x steps_per_trial steps
  * per contact trial (up to 11).  *us_per_step (may be NULL) receives the
- * contact kernel's best mean time in microseconds; SPH_S_CONTACT_LANES,
+ * best mean time in microseconds; SPH_S_CONTACT_LANES,
  * SPH_S_CONTACT_WG, SPH_S_VL_CAP, SPH_S_RADIX_BITS and SPH_S_XCD_ORDER then
  * read the chosen settings. */
 int sph_autotune(sph_ctx* ctx, uint64_t steps_per_trial, double* us_per_step);

@@ -85,6 +85,7 @@ struct DevArrays {
     double4* x_build;    // position at the last list build, original index
     // contact history (NC words per particle, original-index rows)
     uint32_t* crow;      // packed partner index (in perm_rows' order) + image code
+    double* wall0;       // small totals: each particle's force on wall 0 (or null)
     uint32_t* perm_rows; // the order the row words index: sorted index -> original
     double4* delta_t;    // tangential displacement per slot (w unused)
     // Recording for the adjoint (null otherwise), in the step's sorted order:

@@ -833,10 +833,10 @@ __device__ __forceinline__ bool register_contact(uint32_t* row, uint32_t ib, uin
 // (all four when periodic == 0, the y walls when periodic == 2), each
 // spelled out so that nothing is indexed dynamically; then the particle's
 // outputs at its original index o when `write` is set.
-__device__ __forceinline__ void walls_and_outputs(CParams& p, const DevArrays& a, Acc& A,
-                                                  const double4 xa, const double4 vel_a,
-                                                  const double4 av_a, double Lz, uint32_t o,
-                                                  int part) {
+__device__ __forceinline__ double walls_and_outputs(CParams& p, const DevArrays& a, Acc& A,
+                                                    const double4 xa, const double4 vel_a,
+                                                    const double4 av_a, double Lz, uint32_t o,
+                                                    int part) {
     const double ra = xa.w;
     double wf0 = 0.0, wf1 = 0.0, wf2 = 0.0, wf3 = 0.0, wf4 = 0.0;
     {
@@ -891,6 +891,7 @@ __device__ __forceinline__ void walls_and_outputs(CParams& p, const DevArrays& a
     if (part == 1 || part == 4) rec[OUT_T] = make_double4(A.T.x, A.T.y, A.T.z, 0.0);
     if (part == 2 || part == 4) rec[OUT_E] = make_double4(A.es_dot, A.ev_dot, A.p, wf0);
     if (part == 3 || part == 4) rec[OUT_W] = make_double4(wf1, wf2, wf3, wf4);
+    return wf0;
 }
 
 // es += es_dot dt and ev += ev_dot dt of the contact pass's outputs
@@ -2095,13 +2096,14 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
     }
     if (!quiet || any_ended || remap)
         copy_words<SPL>(a.crow + (size_t)ia_orig * NC + g.q * SPL, gs + g.q * SPL);
-    walls_and_outputs(p, a, A, xa_o, vel_o, av_o, Lz, ia_orig, g.q < 4 ? (int)g.q : -1);
+    const double wf0 =
+        walls_and_outputs(p, a, A, xa_o, vel_o, av_o, Lz, ia_orig, g.q < 4 ? (int)g.q : -1);
     if constexpr (FUSED) {
+        if (a.wall0 && g.q == 3) a.wall0[ia_orig] = wf0;
         // The particle's force and torque are final (its own row and the
         // walls): integrate it now (src/integration.cuh:14-305), from the
         // step's sorted copies, into the next step's set, and hash it for
         // the next step.  (Fixed grid height, no bonds, no wmode-3 wall.)
-        static_assert(!FUSED || LPP == 4, "one vector component per lane");
         // Lane 0 holds the force, lane 1 the torque, lane 2 the energy
         // rates: lane q takes component q of each.
         if (g.q == 2) {
@@ -2114,7 +2116,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
                      tz = g.template bc<1>(A.T.z);
         const double fq = g.q == 0 ? fx : g.q == 1 ? fy : fz;
         const double tq = g.q == 0 ? tx : g.q == 1 ? ty : tz;
-        const double xn = integrate_component(p, a, lp, ia_orig, g.q, fq, tq, xa_o, vel_o, av_o, ia);
+        // (One vector component per lane: lanes beyond the fourth only take
+        // part in the exchange.)
+        double xn = 0.0;
+        if (g.q < 4)
+            xn = integrate_component(p, a, lp, ia_orig, g.q, fq, tq, xa_o, vel_o, av_o, ia);
         const double4 x_new = make_double4(g.template bc<0>(xn), g.template bc<1>(xn),
                                            g.template bc<2>(xn), g.template bc<3>(xn));
         HashFlags f;
@@ -2557,8 +2563,14 @@ constexpr uint32_t MV_WAVE = 64;     // movers up to which each search takes a w
 // Copying and rebuilding all places and cells in 256 work-items took 55-78 us
 // on a column of 4,096 in a wide grid and 300 us on 20,000 particles; this
 // takes 6 and 9.
+//
+// With `fresh` the sorted copies the next step reads (set `nxt`) follow;
+// otherwise they stay in the previous order and `stale` is set: the next step
+// then reads the original-index arrays through perm, and its integration pass
+// writes the copies in the new order.
 __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp, int passes,
-                                     int bits, int sorted_bits) {
+                                     int bits, int sorted_bits, bool fresh, uint32_t nxt,
+                                     bool& stale) {
     __shared__ unsigned long long comp[MV_CAP];  // movers' (new key, index), ascending
     __shared__ uint32_t rk[MV_CAP];              // movers' old positions, ascending
     __shared__ uint32_t npos[MV_CAP];            // movers' new positions
@@ -2597,11 +2609,9 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
         for (uint32_t c = tid; c < p.ncells; c += WALLS_WG)
             a.cell_start[p.cell_base + c] = 0xffffffffu;
         __syncthreads();
-        // (The sorted copies are left in the previous order: the next step
-        // reads the original-index arrays through perm, copies_stale, and
-        // its integration pass writes them in the new order.)
+        stale = !fresh;
         for (uint32_t j = tid; j < N; j += WALLS_WG)
-            cells_one(p, a, B + j, sorted_bits, 0u, false);
+            cells_one(p, a, B + j, sorted_bits, nxt, !stale);
         __syncthreads();
         return RESORTED_FULL;
     }
@@ -2733,12 +2743,18 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
         a.val_tmp[B + j] = o;
     }
     __syncthreads();
+    stale = !fresh;
     for (uint32_t t = tid; t < total; t += WALLS_WG) {
         const uint32_t j = place_of(t, last);
         const uint32_t o = a.val_tmp[B + j];
         a.skey[B + j] = a.key_tmp[B + j];
         a.perm[B + j] = o;
         a.rank[o] = B + j;
+        if (!stale) {
+            a.xs[nxt][B + j] = a.x[o];
+            a.vs[nxt][B + j] = a.vel[o];
+            a.ws[nxt][B + j] = a.angvel[o];
+        }
     }
     __syncthreads();
     // Cell boundaries at the rewritten places and right behind each run
@@ -2770,13 +2786,58 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
     return RESORTED_MERGE;
 }
 
+// The wall-force block partials of one simulation by one workgroup (the
+// reference's summation kernel, 256 original indices per partial), summed
+// left to right in thread 0; at most 1,024 blocks.  Wall 0's forces come from
+// a compact array: from the particles' output records one workgroup's reads
+// took the step from 18.8 to 21.2 us on 5,000 particles.
+__device__ __forceinline__ double wall_sum_small(CParams& p, const DevArrays& a, uint32_t w,
+                                                 double* stage) {
+    constexpr uint32_t WAVES = WALLS_WG / 64;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    // A wavefront per block: each lane holds the four values block_tree_sum
+    // adds first, two blocks' loads in flight.
+    for (uint32_t c0 = wave; c0 < p.nblocks; c0 += 2u * WAVES) {
+        double v[2][4];
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h)
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const uint32_t local = (c0 + h * WAVES) * BLOCK + i * 64u + lane;
+                v[h][i] = 0.0;
+                if (local < p.np)
+                    v[h][i] += w == 0 ? a.wall0[p.base + local]
+                                      : wall_force_pp(a, p.base + local, w);
+            }
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            double s = (v[h][0] + v[h][2]) + (v[h][1] + v[h][3]);
+#pragma unroll
+            for (int i = 32; i > 0; i >>= 1) {
+                const double o = __shfl_down(s, (unsigned)i, 64);
+                if ((int)lane < i) s += o;
+            }
+            if (lane == 0 && c0 + h * WAVES < p.nblocks) stage[c0 + h * WAVES] = s;
+        }
+    }
+    __syncthreads();
+    double sum = 0.0;
+    if (threadIdx.x == 0)
+        for (uint32_t j = 0; j < p.nblocks; ++j) sum += stage[j];
+    __syncthreads();
+    return sum;
+}
+
 // integrateWalls + the loop advance (src/integration.cuh:344-450,
 // src/device.cu:2454-2462,2500-2538), one workgroup.  Every dynamic wall
 // integrates wall 0's force sum (src/device.cu:2504-2505).  With `resort`
 // set it first re-sorts for the next step when the integration pass found
-// particles that changed cell (the next step then launches no sort).
-__global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resort, int passes,
-                                                    int bits, int sorted_bits) {
+// particles that changed cell (the next step then launches no sort); with 2
+// it always refreshes the sorted copies (a contact pass that integrates
+// writes the arrays a stale reader would read).  With `partials` set no pass
+// before it has formed the wall-force partials nor kept the order of the rows.
+__global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resort, int partials,
+                                                    int passes, int bits, int sorted_bits) {
     __shared__ double stage[2048];
     __shared__ uint32_t do_sort;
     touch_args();
@@ -2814,15 +2875,29 @@ __global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resor
     // The serial sums of the block partials: wall 0's (every wall integrates
     // it, P8), or with per-wall sums each wall's.
     const uint32_t nsum = !walls ? 0u : (p.wall_sums ? p.nw : 1u);
+    if (partials && lp->order_changed)
+        for (uint32_t j = threadIdx.x; j < p.npad; j += 4u * WALLS_WG) {
+            uint32_t o[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+                if (j + i * WALLS_WG < p.npad) o[i] = a.perm[p.base + j + i * WALLS_WG];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+                if (j + i * WALLS_WG < p.npad) a.perm_rows[p.base + j + i * WALLS_WG] = o[i];
+        }
     for (uint32_t k = 0; k < nsum; ++k) {
-        const double fs = serial_sum(a.partial + (size_t)k * a.nchunk + p.chunk_base, p.nblocks,
-                                     stage);
+        const double fs =
+            partials ? wall_sum_small(p, a, k, stage)
+                     : serial_sum(a.partial + (size_t)k * a.nchunk + p.chunk_base, p.nblocks, stage);
         if (threadIdx.x == 0) s_fsum[k] = fs;
     }
     __syncthreads();
     const uint32_t movers = lp->nmovers;
     uint32_t resorted = 0;
-    if (do_sort) resorted = resort_one_block(p, a, lp, passes, bits, sorted_bits);
+    bool stale = false;
+    if (do_sort)
+        resorted = resort_one_block(p, a, lp, passes, bits, sorted_bits, resort == 2, slot ^ 1u,
+                                    stale);
     if (mine) {
         const uint32_t wi = p.wall_base + w;
         w_mvfd.z = s_fsum[p.wall_sums ? w : 0u];  // 0.0 + partial[0] + partial[1] + ...
@@ -2843,7 +2918,7 @@ __global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resor
     // The next step's contact pass maps its rows to the new order and reads
     // the state through perm.
     lp->order_changed = do_sort;
-    lp->copies_stale = do_sort;
+    lp->copies_stale = stale ? 1u : 0u;
     if (p.adaptive == 1 && walls) lp->grid_Lz = grid_top;
     if (t_now >= 10.0 && t_now < 15.0 && vstate == 1) lp->velocity_state = 2;
     else if (t_now >= 15.0 && vstate == 2) lp->velocity_state = 1;
@@ -3093,9 +3168,14 @@ hipError_t launch_contact(const DevArrays& a, int contactmodel, int lanes, int w
     return hipGetLastError();
 }
 
-hipError_t launch_contact_integrate(const DevArrays& a, int contactmodel, hipStream_t s) {
-    const dim3 b(BLOCK), g(a.nchunk * 4u);
-    if (contactmodel == 2)
+hipError_t launch_contact_integrate(const DevArrays& a, int contactmodel, int lanes,
+                                    hipStream_t s) {
+    const dim3 b(BLOCK), g(a.nchunk * (unsigned)lanes);
+    if (lanes == 8 && contactmodel == 2)
+        hipLaunchKernelGGL((k_contact_g<2, 8, true, BLOCK>), g, b, 0, s, a);
+    else if (lanes == 8)
+        hipLaunchKernelGGL((k_contact_g<3, 8, true, BLOCK>), g, b, 0, s, a);
+    else if (contactmodel == 2)
         hipLaunchKernelGGL((k_contact_g<2, 4, true, BLOCK>), g, b, 0, s, a);
     else
         hipLaunchKernelGGL((k_contact_g<3, 4, true, BLOCK>), g, b, 0, s, a);
@@ -3130,9 +3210,9 @@ hipError_t launch_integrate_q(const DevArrays& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_walls(const DevArrays& a, int resort, int passes, int bits, int sorted_bits,
-                        hipStream_t s) {
-    hipLaunchKernelGGL(k_walls, dim3(a.nsim), dim3(WALLS_WG), 0, s, a, resort, passes, bits,
+hipError_t launch_walls(const DevArrays& a, int resort, int partials, int passes, int bits,
+                        int sorted_bits, hipStream_t s) {
+    hipLaunchKernelGGL(k_walls, dim3(a.nsim), dim3(WALLS_WG), 0, s, a, resort, partials, passes, bits,
                        sorted_bits);
     return hipGetLastError();
 }

@@ -36,10 +36,11 @@ hipError_t launch_contact(const DevArrays& a, int contactmodel, int lanes, int w
                           hipStream_t s);
 // bondsLinear per bond, then a per-particle gather in bond order
 // (src/cohesion.cuh:8-233).
-// Contact pass (models 2 and 3, four lanes per particle) that also
+// Contact pass (models 2 and 3, four or eight lanes per particle) that also
 // integrates each particle and hashes it for the next step; then the wall
 // force partials.  For a fixed grid height, without bonds or a wmode-3 wall.
-hipError_t launch_contact_integrate(const DevArrays& a, int contactmodel, hipStream_t s);
+hipError_t launch_contact_integrate(const DevArrays& a, int contactmodel, int lanes,
+                                    hipStream_t s);
 hipError_t launch_wall_partials(const DevArrays& a, hipStream_t s);
 hipError_t launch_bonds(const DevArrays& a, hipStream_t s);
 // findShearStressOnFixedMovingParticles + summation + serial sum
@@ -55,10 +56,11 @@ hipError_t launch_integrate_q(const DevArrays& a, hipStream_t s);
 // Per simulation: serial sum of the partials + integrateWalls + loop advance
 // (src/integration.cuh:344-450, src/device.cu:2500-2538).  With resort != 0
 // it also re-sorts the simulation for the next step, in one workgroup, when
-// the integration pass (launched with hash_next) found a cell change.
+// the integration pass (launched with hash_next) found a cell change; with 2
+// the sorted copies follow.  With partials != 0 it forms the partials itself.
 hipError_t launch_check_sqrt32(unsigned long long* bad, uint64_t lo, uint64_t hi, hipStream_t s);
-hipError_t launch_walls(const DevArrays& a, int resort, int passes, int bits, int sorted_bits,
-                        hipStream_t s);
+hipError_t launch_walls(const DevArrays& a, int resort, int partials, int passes, int bits,
+                        int sorted_bits, hipStream_t s);
 // Fill n words with v.
 hipError_t launch_fill_u32(uint32_t* dst, unsigned n, uint32_t v, hipStream_t s);
 

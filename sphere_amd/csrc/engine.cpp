@@ -110,12 +110,24 @@ struct Sim {
     int64_t iter = 0;
 };
 
+// Particles (padding included) up to which a step with the default settings
+// runs as two kernels: eight work-items per particle in a contact pass that
+// also integrates, and a walls kernel that sums the wall forces itself.  The
+// step is a chain of latencies there, so one pass less and shorter chains per
+// work-item win; beyond it the registers the integration adds cost the
+// throughput and the one workgroup's sum grows.  Step, two kernels / three, in
+// us: 300 particles 17.0 / 19.6, 601 17.3 / 20.2, 3,000 17.7 / 21.6, 5,000
+// 18.8 / 21.8, 8,000 19.7 / 22.0, 10,000 22.9 / 22.5, 12,000 24.3 / 22.9; a
+// column of 4,096 16.2 / 22.1.  (Eight work-items and three kernels: 601 18.0,
+// 5,000 20.6.)
+constexpr uint32_t SMALL_NTOT = 8192;
+
 // The adjoint's host bookkeeping at a checkpoint: the loop mirrors and the
 // hash/re-sort state enqueue_step reads.
 struct AdjHostMark {
     std::vector<double> t;
     std::vector<int64_t> iter;
-    bool hash_pending, prev_walls_resorted;
+    bool hash_pending, prev_walls_resorted, copies_fresh;
 };
 
 // A recorded forward pass awaiting its reverse (sph_adjoint_record).
@@ -159,6 +171,10 @@ struct sph_ctx {
     int sort_mode = 2;
     bool resort_at_end = true;     // the choice for the steps being enqueued
     bool prev_walls_resorted = false;
+    // The sorted copies the next step reads are in its order (a contact pass
+    // that integrates must not read the arrays it writes).
+    bool copies_fresh = true;
+    int list_lanes = 0;  // work-items per particle the lists' hit masks are laid out for
     // Asynchronous sample of the loop counters for the automatic choice.
     DevLoop* loop_sample = nullptr;   // pinned host memory (all simulations)
     hipEvent_t sample_ev = nullptr;
@@ -190,9 +206,10 @@ struct sph_ctx {
     size_t rd_list_bytes = 0;
     void* rd_stage = nullptr;
     uint64_t adj_checkpoint = 0;
-    // Contact and integration in one pass where the step allows it (off by
-    // default: measured slower than the two kernels, 72.1 + 6.2 us for the
-    // fused pass and its wall partials against 53.3 + 19.6 us).
+    // SPH_S_FUSED: contact and integration in one pass where the step allows
+    // it.  Off by default: above SMALL_NTOT, where the default settings do so by
+    // themselves, measured slower than the two kernels (1e5 particles: 55.7
+    // against 46.8 us a step).
     bool fused = false;
     int integrate_lanes = 1;  // SPH_S_INTEGRATE_LANES
     // per-kernel profile (stage name, total ms, launches)
@@ -546,6 +563,7 @@ int allocate(sph_ctx* c) {
     ALLOC(A.mv_last, ns * MV_CAP);
     ALLOC(A.crow, np * NC);
     ALLOC(A.perm_rows, np);
+    if (np <= SMALL_NTOT) ALLOC(A.wall0, np);
     ALLOC(A.delta_t, np * NC);
     ALLOC(A.w_nx, nw); ALLOC(A.w_mvfd, nw); ALLOC(A.w_acc, nw);
     ALLOC(A.tau_pp, np);
@@ -999,6 +1017,32 @@ void sample_loop(sph_ctx* c) {
     c->sample_pending = true;
 }
 
+int set_loop_flag(sph_ctx* c, int sim, uint32_t DevLoop::*flag);
+
+// How a step's kernels run.
+struct StepForm {
+    int lanes;      // work-items per particle in the contact pass
+    bool fused;     // contact and integration in one pass
+    bool partials;  // the walls kernel forms the wall-force partials
+};
+
+StepForm step_form(const sph_ctx* c) {
+    StepForm f{c->contact_lanes, c->fused, false};
+    const bool history = c->contactmodel == 2 || c->contactmodel == 3;
+    // Each particle's force is final after its own contact row: a fixed grid
+    // height, no bonds, no wmode-3 wall.
+    const bool can_fuse = history && !c->any_adaptive && c->A.nbond == 0 && !c->shear_stress;
+    const bool defaults = c->contact_lanes == 4 && c->contact_wg == 256 &&
+                          c->integrate_lanes == 1 && !c->fused;
+    if (history && defaults && c->A.ntot <= SMALL_NTOT) {
+        f.lanes = 8;
+        f.fused = f.partials = can_fuse;
+    } else {
+        f.fused = c->fused && can_fuse && c->contact_lanes == 4;
+    }
+    return f;
+}
+
 int enqueue_step(sph_ctx* c) {
     const DevArrays& A = c->A;
     hipStream_t s = c->stream;
@@ -1023,22 +1067,32 @@ int enqueue_step(sph_ctx* c) {
         HIPCHK(c, launch_cells(A, c->sorted_bits, s), "cells");
         pr.end();
     }
-    // Contact and integration in one pass where each particle's force is
-    // final after its own contact row: a fixed grid height, no bonds, no
-    // wmode-3 wall, four lanes per particle.
-    const bool fused = c->fused && hash_in_integrate && A.nbond == 0 && !c->shear_stress &&
-                       c->contact_lanes == 4 && (c->contactmodel == 2 || c->contactmodel == 3);
+    const StepForm form = step_form(c);
+    // The lists' hit masks follow the number of lanes.
+    if (c->list_lanes != form.lanes) {
+        if (c->list_lanes != 0)
+            for (int k = 0; k < (int)c->sims.size(); ++k) {
+                const int rc = set_loop_flag(c, k, &DevLoop::force_rebuild);
+                if (rc) return rc;
+            }
+        c->list_lanes = form.lanes;
+    }
+    // A pass that integrates must not read the arrays it writes: it waits for
+    // a step that begins with the sorted copies in its own order.
+    const bool fused = form.fused && c->copies_fresh;
     if (fused) {
         pr.begin("contact_integrate");
-        HIPCHK(c, launch_contact_integrate(A, (int)c->contactmodel, s), "contact");
+        HIPCHK(c, launch_contact_integrate(A, (int)c->contactmodel, form.lanes, s), "contact");
         pr.end();
-        // Also after a re-sort: the order the fused pass left its rows in.
-        pr.begin("wall_partials");
-        HIPCHK(c, launch_wall_partials(A, s), "partials");
-        pr.end();
+        if (!form.partials) {
+            // Also after a re-sort: the order the fused pass left its rows in.
+            pr.begin("wall_partials");
+            HIPCHK(c, launch_wall_partials(A, s), "partials");
+            pr.end();
+        }
     } else {
         pr.begin("contact");
-        HIPCHK(c, launch_contact(A, (int)c->contactmodel, c->contact_lanes, c->contact_wg, s),
+        HIPCHK(c, launch_contact(A, (int)c->contactmodel, form.lanes, c->contact_wg, s),
                "contact");
         pr.end();
     }
@@ -1070,9 +1124,10 @@ int enqueue_step(sph_ctx* c) {
     }
     const bool resort = hash_in_integrate && c->resort_at_end;
     pr.begin("walls");
-    HIPCHK(c, launch_walls(A, resort ? 1 : 0, c->passes, c->radix_bits, c->sorted_bits, s),
-           "walls");
+    HIPCHK(c, launch_walls(A, !resort ? 0 : form.fused ? 2 : 1, fused && form.partials ? 1 : 0,
+                           c->passes, c->radix_bits, c->sorted_bits, s), "walls");
     pr.end();
+    c->copies_fresh = !resort || form.fused;
     c->prev_walls_resorted = resort;
     // Host mirror of the loop counters (src/device.cu:2536-2538).
     for (Sim& sim : c->sims) {
@@ -1099,6 +1154,8 @@ int enqueue_graph_steps(sph_ctx* c, uint64_t n, uint64_t* done) {
     if (G <= 0 || n < (uint64_t)G || c->profile || c->hash_pending ||
         c->prev_walls_resorted != resort)
         return SPH_OK;
+    const StepForm form = step_form(c);
+    if (c->list_lanes != form.lanes || (form.fused && !c->copies_fresh)) return SPH_OK;
     hipGraphExec_t exec = nullptr;
     for (auto& g : c->graphs)
         if (g.steps == G && g.resort == resort && g.lanes == c->contact_lanes) exec = g.exec;
@@ -2442,6 +2499,7 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             }
             hm.hash_pending = c->hash_pending;
             hm.prev_walls_resorted = c->prev_walls_resorted;
+            hm.copies_fresh = c->copies_fresh;
         } else {
             for (size_t k = 0; k < nsim; ++k) {
                 c->sims[k].h.t = hm.t[k];
@@ -2449,6 +2507,7 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             }
             c->hash_pending = hm.hash_pending;
             c->prev_walls_resorted = hm.prev_walls_resorted;
+            c->copies_fresh = hm.copies_fresh;
         }
         return SPH_OK;
     };
@@ -2705,6 +2764,9 @@ int sph_autotune(sph_ctx* c, uint64_t steps_per_trial, double* us_per_step) {
     // only when at least 3% faster.
     const uint64_t warm = std::max<uint64_t>(1, steps_per_trial / 2);
     const bool history = c->sims[0].h.contactmodel == 2 || c->sims[0].h.contactmodel == 3;
+    // A small total's default form shares the work out differently between
+    // its kernels: there the settings are judged by the step's kernels together.
+    const bool whole = c->A.wall0 != nullptr;
     auto contact_trial = [&](double* us) -> int {
         int rc = sph_step(c, warm);
         if (!rc) rc = sph_sync(c);
@@ -2721,10 +2783,13 @@ int sph_autotune(sph_ctx* c, uint64_t steps_per_trial, double* us_per_step) {
         c->profile = was;
         if (rc) return rc;
         *us = 0.0;
-        for (size_t k = 0; k < c->prof_names.size(); ++k)
-            if ((c->prof_names[k] == "contact" || c->prof_names[k] == "contact_integrate") &&
-                c->prof_n[k] > 0)
-                *us = 1000.0 * c->prof_ms[k] / (double)c->prof_n[k];
+        for (size_t k = 0; k < c->prof_names.size(); ++k) {
+            const std::string& n = c->prof_names[k];
+            if (c->prof_n[k] > 0 &&
+                (n == "contact" || n == "contact_integrate" ||
+                 (whole && (n == "integrate" || n == "wall_partials" || n == "walls"))))
+                *us += 1000.0 * c->prof_ms[k] / (double)c->prof_n[k];
+        }
         return *us > 0.0 ? SPH_OK : fail(c, SPH_E_DEVICE, "autotune: no contact launches timed");
     };
     auto sort_trial = [&](double* us) -> int {

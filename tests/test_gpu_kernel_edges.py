@@ -178,3 +178,37 @@ def test_overlap_list_edges(n, radius):
                                    ctypes.byref(m)) == 0
         assert m.value == len(pb)
         assert numpy.array_equal(pairs, pb[:k]) and numpy.array_equal(delta, db[:k])
+
+
+# The two-kernel step of small totals (up to 8,192 particles with their
+# padding) and the three-kernel step just above, re-sorting at nearly every
+# step: a round of the wall-force sum takes 8,192 particles, and settings are
+# changed in between, so that steps of either form, with other list layouts
+# and with stale sorted copies, follow each other.
+@pytest.mark.parametrize("n", [300, 4097, 8192, 8193])
+def test_small_total_step_form(n):
+    rng = numpy.random.default_rng(n)
+    s = _cloud(n, 13, r=(0.002, 0.003))
+    s.x = rng.uniform(0.05, 0.45, (n, 3))
+    cell = float(s.L[0]) / int(s.num[0])
+    pick = rng.choice(n, size=max(3, n // 100), replace=False)
+    s.vel[pick, :3] = rng.uniform(-0.3, 0.3, (len(pick), 3)) * cell / float(s.time_dt[0])
+    s.x[rng.choice(n, size=n // 3, replace=False), 2] = 0.45
+    s.consolidate(1.0e3)
+    s.w_x[0] = 0.4515  # pressed into the third of them at the top
+    image = s.tobytes()
+    ref, pressed = oracle.Oracle(image), 0
+    with engine.Context(image) as ctx:
+        ctx.set_scalar("sort_mode", 1)
+        for name, value in ((None, 0), ("contact_lanes", 16), ("contact_lanes", 4), ("fused", 1),
+                            ("fused", 0), ("sort_mode", 0), ("sort_mode", 1),
+                            ("graph_steps", 2)):
+            if name:
+                ctx.set_scalar(name, value)
+            ctx.step(4)
+            ref.step(4)
+            for f in ("perm", "contacts", "x", "vel", "angvel", "force", "delta_t", "walls_mvfd"):
+                assert numpy.array_equal(ctx.get(f), ref.get(f)), (name, value, f)
+            pressed += ref.get("walls_mvfd")[0, 2] != 0.0
+        if n > 300:  # (three movers seldom leave their cells)
+            assert ctx.scalar("sorts") >= 8 and pressed
