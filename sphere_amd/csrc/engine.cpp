@@ -2839,8 +2839,9 @@ int sph_autotune(sph_ctx* c, uint64_t steps_per_trial, double* us_per_step) {
         double cur = 0.0;
         if (rc || (rc = sph_get_scalar(c, which, &cur))) return;
         rc = sort ? sort_trial(&best) : contact_trial(&best);  // the incumbent
+        const double first = cur;
         for (double v : values) {
-            if (v == cur || rc) continue;
+            if (v == first || rc) continue;
             rc = set_all(which, v);
             double t = 0.0;
             if (!rc) rc = sort ? sort_trial(&t) : contact_trial(&t);
