@@ -349,6 +349,10 @@ int sph_profile(sph_ctx* ctx, int enable);
 int sph_profile_report(sph_ctx* ctx, char* buf, size_t cap);
 
 void sph_close(sph_ctx* ctx);
+/* The device memory kept for later contexts (a closed context's adjoint tape,
+ * one per device, at most 8 GiB) is given back now.  It is also given back
+ * whenever an allocation of the engine fails. */
+void sph_trim(void);
 const char* sph_last_error(const sph_ctx* ctx);
 /* Error message of the last failed sph_open / sph_open_mem on this thread. */
 const char* sph_open_error(void);

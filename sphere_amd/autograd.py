@@ -22,6 +22,8 @@ length).  Lengths are differentiated as exact roots and the contact list and
 branches of each step are frozen, as in sph_adjoint.
 """
 
+import copy
+
 import numpy
 import torch
 
@@ -67,15 +69,22 @@ class Trajectory:
 
     def image(self, theta, x0=None, v0=None):
         """The .bin image of the template with theta (and x0, v0) applied."""
-        from .sim import sim
-        s = sim().frombytes(self.template.tobytes())
+        # The template's own arrays but for the changed ones (a decoded copy of
+        # all of them where a changed one is not as a decoded one would be).
+        s = copy.copy(self.template)
+        fields = [f for name in self.params for f in self.ties[name]]
+        if any(getattr(getattr(s, f), "dtype", None) != numpy.float64 for f in fields):
+            from .sim import sim
+            s = sim().frombytes(s.tobytes())
         for name, value in zip(self.params, numpy.asarray(theta, dtype=numpy.float64)):
             for field in self.ties[name]:
-                getattr(s, field)[0] = float(value)
+                a = numpy.array(getattr(s, field))
+                a[0] = float(value)
+                setattr(s, field, a)
         if x0 is not None:
-            s.x[:, :3] = numpy.asarray(x0, dtype=numpy.float64).reshape(self.np, 3)
+            s.x = numpy.array(x0, dtype=numpy.float64).reshape(self.np, 3)
         if v0 is not None:
-            s.vel[:, :3] = numpy.asarray(v0, dtype=numpy.float64).reshape(self.np, 3)
+            s.vel = numpy.array(v0, dtype=numpy.float64).reshape(self.np, 3)
         return s.tobytes()
 
     def __call__(self, theta, x0=None, v0=None):

@@ -122,6 +122,9 @@ struct Sim {
 // 5,000 20.6.)
 constexpr uint32_t SMALL_NTOT = 8192;
 
+constexpr int SCRATCH_MAX_DEVICES = 64;
+constexpr size_t STAGE_BYTES = (size_t)256 << 10;
+
 // The adjoint's host bookkeeping at a checkpoint: the loop mirrors and the
 // hash/re-sort state enqueue_step reads.
 struct AdjHostMark {
@@ -144,6 +147,8 @@ struct sph_ctx {
     DevArrays A;
     DevParams* d_ptab = nullptr;  // device copy of the parameter blocks
     std::vector<void*> allocs;
+    void* arena = nullptr;            // the one allocation they are parts of
+    size_t zero_bytes = 0, ones_bytes = 0;  // its first parts, by initial value
     std::vector<size_t> alloc_bytes;  // size of each allocation, in order
     hipStream_t stream = nullptr;
     int device = 0;
@@ -177,6 +182,7 @@ struct sph_ctx {
     int list_lanes = 0;  // work-items per particle the lists' hit masks are laid out for
     // Asynchronous sample of the loop counters for the automatic choice.
     DevLoop* loop_sample = nullptr;   // pinned host memory (all simulations)
+    char* stage = nullptr;            // behind it: small reads pass through here
     hipEvent_t sample_ev = nullptr;
     bool sample_pending = false;
     int64_t sample_iter0 = 0;
@@ -517,70 +523,169 @@ void layout(sph_ctx* c) {
     c->contactmodel = c->sims[0].h.contactmodel;
 }
 
-template <class T> int dev_alloc(sph_ctx* c, T** p, size_t count) {
-    *p = nullptr;
-    if (count == 0) count = 1;
-    hipError_t e = hipMalloc((void**)p, count * sizeof(T));
-    if (e != hipSuccess) return hip_fail(c, e, "hipMalloc");
-    c->allocs.push_back((void*)*p);
-    c->alloc_bytes.push_back(count * sizeof(T));
-    return SPH_OK;
+// The adjoint's tape outlives its context: one buffer per device, at most
+// TAPE_KEEP bytes, for the next context that needs one of about its size.  A
+// calibration opens a context per evaluation, each with a tape of gigabytes,
+// and the driver clears freed memory in the background: allocations then wait
+// for it again and again (16 beds of 1,003 particles, 200 steps: half of the
+// passes took 117 ms or more, up to 930, instead of 14).  A buffer is put here
+// only after its context's stream has finished; it is given back when any
+// allocation of the engine fails and by sph_trim.
+constexpr size_t TAPE_KEEP = (size_t)8 << 30;
+struct TapePool {
+    std::mutex mu;
+    struct Slot { void* p = nullptr; size_t bytes = 0; } slot[SCRATCH_MAX_DEVICES];
+    static bool known(int device) { return device >= 0 && device < SCRATCH_MAX_DEVICES; }
+    size_t held(int device) {
+        if (!known(device)) return 0;
+        std::lock_guard<std::mutex> lock(mu);
+        return slot[device].bytes;
+    }
+    // A kept buffer of at least `need` bytes (and not of many times as many),
+    // or null; one that is too small is freed.
+    void* take(int device, size_t need, size_t* bytes) {
+        if (!known(device)) return nullptr;
+        std::lock_guard<std::mutex> lock(mu);
+        Slot& s = slot[device];
+        if (!s.p || s.bytes / 8 > need) return nullptr;
+        void* p = s.p;
+        *bytes = s.bytes;
+        s = Slot();
+        if (*bytes >= need) return p;
+        (void)hipFree(p);
+        return nullptr;
+    }
+    void give(int device, void* p, size_t bytes) {
+        if (!p) return;
+        if (known(device) && bytes <= TAPE_KEEP) {
+            std::lock_guard<std::mutex> lock(mu);
+            Slot& s = slot[device];
+            if (bytes > s.bytes) {
+                std::swap(p, s.p);
+                s.bytes = bytes;
+            }
+        }
+        if (p) (void)hipFree(p);
+    }
+    // Frees what is kept for a device (all with -1); false when nothing was.
+    bool trim(int device) {
+        std::lock_guard<std::mutex> lock(mu);
+        bool any = false;
+        for (int d = 0; d < SCRATCH_MAX_DEVICES; ++d)
+            if (slot[d].p && (device < 0 || d == device)) {
+                (void)hipFree(slot[d].p);
+                slot[d] = Slot();
+                any = true;
+            }
+        return any;
+    }
+};
+TapePool& tape_pool() {
+    static TapePool* pool = new TapePool;  // never destroyed: contexts may outlive statics
+    return *pool;
 }
 
-#define ALLOC(ptr, n)                               \
-    do {                                            \
-        int rc_ = dev_alloc(c, &(ptr), (size_t)(n)); \
-        if (rc_) return rc_;                         \
-    } while (0)
+// hipMalloc for the context's device; what the pool keeps there is given back
+// when it fails.
+hipError_t dev_malloc(sph_ctx* c, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && tape_pool().trim(c->device)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+// The context's device arrays are parts of one allocation: 60 allocations and
+// as many frees took a quarter of the time to open and close a small context.
+struct Arena {
+    sph_ctx* c;
+    std::vector<void**> slots;
+    size_t bytes = 0;
+    template <class T> void take(T** p, size_t count) {
+        static_assert(sizeof(T*) == sizeof(void*), "one pointer type");
+        *p = nullptr;
+        const size_t b = std::max<size_t>(count, 1) * sizeof(T);
+        slots.push_back(reinterpret_cast<void**>(p));
+        c->alloc_bytes.push_back(b);
+        bytes += up(b);
+    }
+    static size_t up(size_t b) { return (b + 511) & ~(size_t)511; }
+    int commit() {
+        hipError_t e = dev_malloc(c, &c->arena, bytes);
+        if (e != hipSuccess) return hip_fail(c, e, "hipMalloc");
+        char* at = static_cast<char*>(c->arena);
+        for (size_t k = 0; k < slots.size(); ++k) {
+            void* const here = at;
+            memcpy(slots[k], &here, sizeof here);
+            c->allocs.push_back(here);
+            at += up(c->alloc_bytes[k]);
+        }
+        return SPH_OK;
+    }
+};
+
+#define ALLOC(ptr, n) arena.take(&(ptr), (size_t)(n))
 
 int allocate(sph_ctx* c) {
     DevArrays& A = c->A;
+    Arena arena{c};
     const size_t np = A.ntot, nb = A.nbond, nkeys = A.nkeys, ns = A.nsim;
     size_t nw = 0, rh = 0;
     for (const Sim& sim : c->sims) {
         nw += sim.h.nw;
         rh += 256u * n_tiles(sim.P.npad);
     }
+    // Arrays that start as zero, together (cleared by one fill).
     ALLOC(A.x, np); ALLOC(A.vel, np); ALLOC(A.angvel, np); ALLOC(A.angpos, np);
     ALLOC(A.xyzsum, np); ALLOC(A.acc, np); ALLOC(A.angacc, np);
     ALLOC(A.out, np * 4); ALLOC(A.es, np); ALLOC(A.ev, np);
-    ALLOC(A.key, np); ALLOC(A.key_prev, np); ALLOC(A.skey, np); ALLOC(A.perm, np);
-    ALLOC(A.key_tmp, np); ALLOC(A.val_tmp, np);
-    // The batch-wide sort and the per-simulation one-workgroup sorts.
-    ALLOC(A.rhist, std::max<size_t>(256 * (size_t)n_tiles((unsigned)np), rh));
-    ALLOC(A.cell_start, nkeys); ALLOC(A.cell_end, nkeys);
+    ALLOC(A.delta_t, np * NC);
     for (int k = 0; k < 2; ++k) {
         ALLOC(A.xs[k], np);
         ALLOC(A.vs[k], np);
         ALLOC(A.ws[k], np);
     }
-    ALLOC(A.rank, np);
-    ALLOC(A.vlist, np * NV);
     ALLOC(A.vcount, np);
     ALLOC(A.x_build, np);
+    ALLOC(A.tau_pp, np);
+    ALLOC(A.tau_eff, ns);
+    ALLOC(A.cell_end, nkeys);
+    ALLOC(A.w_acc, nw);
+    ALLOC(A.glob, 1);
+    c->zero_bytes = arena.bytes;
+    // Arrays that start with every bit set.
+    ALLOC(A.key_prev, np);
+    ALLOC(A.cell_start, nkeys);
+    c->ones_bytes = arena.bytes - c->zero_bytes;
+    ALLOC(A.key, np); ALLOC(A.skey, np); ALLOC(A.perm, np);
+    ALLOC(A.key_tmp, np); ALLOC(A.val_tmp, np);
+    // The batch-wide sort and the per-simulation one-workgroup sorts.
+    ALLOC(A.rhist, std::max<size_t>(256 * (size_t)n_tiles((unsigned)np), rh));
+    ALLOC(A.rank, np);
+    ALLOC(A.vlist, np * NV);
     ALLOC(A.movers, ns * MV_CAP);
     ALLOC(A.skey_bk, np); ALLOC(A.perm_bk, np);
     ALLOC(A.mv_last, ns * MV_CAP);
     ALLOC(A.crow, np * NC);
     ALLOC(A.perm_rows, np);
     if (np <= SMALL_NTOT) ALLOC(A.wall0, np);
-    ALLOC(A.delta_t, np * NC);
-    ALLOC(A.w_nx, nw); ALLOC(A.w_mvfd, nw); ALLOC(A.w_acc, nw);
-    ALLOC(A.tau_pp, np);
+    ALLOC(A.w_nx, nw); ALLOC(A.w_mvfd, nw);
     ALLOC(A.partial, (size_t)MAXWALLS * A.nchunk);
-    ALLOC(A.tau_partial, A.nchunk); ALLOC(A.tau_eff, ns);
+    ALLOC(A.tau_partial, A.nchunk);
     ALLOC(A.bonds, 2 * nb); ALLOC(A.bonds_delta, nb); ALLOC(A.bonds_omega, nb);
     ALLOC(A.bond_f, nb); ALLOC(A.bond_t, nb); ALLOC(A.bond_ok, nb);
     ALLOC(A.badj_off, np + 1);
     ALLOC(A.badj, 2 * nb);
     ALLOC(A.loop, ns);
-    ALLOC(A.glob, 1);
     ALLOC(c->d_ptab, ns);
-    A.ptab = c->d_ptab;
     uint32_t* chunk_sim = nullptr;
     uint32_t* bond_sim = nullptr;
     ALLOC(chunk_sim, A.nchunk);
     ALLOC(bond_sim, nb);
+    const int rc = arena.commit();
+    if (rc) return rc;
+    A.ptab = c->d_ptab;
     A.chunk_sim = chunk_sim;
     A.bond_sim = bond_sim;
     return SPH_OK;
@@ -640,68 +745,59 @@ int upload_state(sph_ctx* c) {
     HIPCHK(c, hipMemcpyAsync((dst), (src), (bytes), hipMemcpyHostToDevice, s), "H2D")
     // Whole-batch initial values.  Padding particles keep zero state, their
     // padding key (never re-hashed) and empty rows.
-    HIPCHK(c, hipMemsetAsync(A.x, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.vel, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.angvel, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.angpos, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.xyzsum, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.acc, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.angacc, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.out, 0, N * 128, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.es, 0, N * 8, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.ev, 0, N * 8, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.delta_t, 0, N * NC * sizeof(double4), s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.vcount, 0, N * 8, s), "memset");
-    for (int k = 0; k < 2; ++k) {
-        HIPCHK(c, hipMemsetAsync(A.xs[k], 0, N * 32, s), "memset");
-        HIPCHK(c, hipMemsetAsync(A.vs[k], 0, N * 32, s), "memset");
-        HIPCHK(c, hipMemsetAsync(A.ws[k], 0, N * 32, s), "memset");
-    }
-    HIPCHK(c, hipMemsetAsync(A.x_build, 0, N * 32, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.tau_pp, 0, N * 8, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.tau_eff, 0, A.nsim * 8, s), "memset");
-    HIPCHK(c, hipMemsetAsync(A.glob, 0, sizeof(DevGlobal), s), "memset");
+    HIPCHK(c, hipMemsetAsync(c->arena, 0, c->zero_bytes, s), "memset");
+    HIPCHK(c, hipMemsetAsync(static_cast<char*>(c->arena) + c->zero_bytes, 0xff, c->ones_bytes, s),
+           "memset");
     // Contact rows start empty (the reference fills np, src/device.cu:458-462)
     // with zero displacement.
-    std::vector<uint32_t> rows(N * NC, EMPTY);
-    H2D(A.crow, rows.data(), N * NC * 4);
-    std::vector<uint32_t> ident(N), keys(N), ff(N, 0xffffffffu), chunk_sim(A.nchunk);
+    HIPCHK(c, launch_fill_u32(A.crow, (unsigned)(N * NC), EMPTY, s), "fill");
+    std::vector<uint32_t> ident(N), keys(N), chunk_sim(A.nchunk);
     for (size_t i = 0; i < N; ++i) ident[i] = (uint32_t)i;
     H2D(A.perm, ident.data(), N * 4);
-    H2D(A.rank, ident.data(), N * 4);
-    H2D(A.perm_rows, ident.data(), N * 4);
-    H2D(A.key_prev, ff.data(), N * 4);
-    std::vector<uint32_t> cs(A.nkeys, 0xffffffffu);
-    H2D(A.cell_start, cs.data(), (size_t)A.nkeys * 4);
-    HIPCHK(c, hipMemsetAsync(A.cell_end, 0, (size_t)A.nkeys * 4, s), "memset");
+    HIPCHK(c, hipMemcpyAsync(A.rank, A.perm, N * 4, hipMemcpyDeviceToDevice, s), "copy");
+    HIPCHK(c, hipMemcpyAsync(A.perm_rows, A.perm, N * 4, hipMemcpyDeviceToDevice, s), "copy");
     std::vector<double> wn, wm;
     std::vector<uint32_t> bonds, bond_sim;
     std::vector<double> bd, bo;
     std::vector<uint32_t> off(N + 1, 0u);
     std::vector<DevLoop> loops(A.nsim);
-    std::vector<std::vector<double>> out_staging(c->sims.size());
+    // A batch's particle arrays are put together first: one copy per array,
+    // not per simulation (16 simulations of 1,003: 9 copies instead of 144).
+    const bool one = c->sims.size() == 1;
+    std::vector<double> out_all(N * 16, 0.0);
+    for (const Sim& sim : c->sims) pack_out(sim.h, out_all.data() + 16 * sim.P.base, sim.h.np);
+    H2D(A.out, out_all.data(), N * 128);
+    std::vector<std::vector<double>> staging;
+    auto put = [&](void* dst, const std::vector<double> Host::*field, size_t width) -> int {
+        if (one) {
+            const std::vector<double>& v = c->sims[0].h.*field;
+            if (c->sims[0].h.np) H2D(dst, v.data(), c->sims[0].h.np * width * 8);
+            return SPH_OK;
+        }
+        staging.emplace_back(N * width, 0.0);
+        std::vector<double>& all = staging.back();
+        for (const Sim& sim : c->sims)
+            if (sim.h.np)
+                memcpy(all.data() + sim.P.base * width, (sim.h.*field).data(),
+                       sim.h.np * width * 8);
+        H2D(dst, all.data(), N * width * 8);
+        return SPH_OK;
+    };
+    struct { void* dst; std::vector<double> Host::*field; size_t width; } fields[] = {
+        {A.x, &Host::x, 4}, {A.vel, &Host::vel, 4}, {A.angvel, &Host::angvel, 4},
+        {A.angpos, &Host::angpos, 4}, {A.xyzsum, &Host::xyzsum, 4}, {A.es, &Host::es, 1},
+        {A.ev, &Host::ev, 1}};
+    for (auto& f : fields) {
+        const int rc = put(f.dst, f.field, f.width);
+        if (rc) return rc;
+    }
+    HIPCHK(c, hipMemcpyAsync(A.x_build, A.x, N * 32, hipMemcpyDeviceToDevice, s), "copy");
     for (const Sim& sim : c->sims) {
         const Host& h = sim.h;
         const DevParams& P = sim.P;
         const size_t np = h.np, b0 = P.base;
         for (uint32_t i = 0; i < P.npad / BLOCK; ++i) chunk_sim[P.chunk_base + i] = P.sim;
         for (size_t i = 0; i < P.npad; ++i) keys[b0 + i] = P.pad_key;
-        if (np) {
-            H2D(A.x + b0, h.x.data(), np * 32);
-            H2D(A.vel + b0, h.vel.data(), np * 32);
-            H2D(A.angvel + b0, h.angvel.data(), np * 32);
-            H2D(A.angpos + b0, h.angpos.data(), np * 32);
-            H2D(A.xyzsum + b0, h.xyzsum.data(), np * 32);
-            {
-                std::vector<double>& rec = out_staging[P.sim];
-                rec.assign(np * 16, 0.0);
-                pack_out(h, rec.data(), np);
-                H2D(A.out + 4 * b0, rec.data(), np * 128);
-            }
-            H2D(A.es + b0, h.es.data(), np * 8);
-            H2D(A.ev + b0, h.ev.data(), np * 8);
-            H2D(A.x_build + b0, h.x.data(), np * 32);
-        }
         wn.insert(wn.end(), h.w_nx.begin(), h.w_nx.end());
         wm.insert(wm.end(), h.w_mvfd.begin(), h.w_mvfd.end());
         // Bonds in batch indices, with the adjacency (CSR, ascending bond id
@@ -729,12 +825,11 @@ int upload_state(sph_ctx* c) {
     // Padding keys, and real keys before the first hash (the first step
     // always hashes).
     H2D(A.key, keys.data(), N * 4);
-    H2D(A.skey, keys.data(), N * 4);
+    HIPCHK(c, hipMemcpyAsync(A.skey, A.key, N * 4, hipMemcpyDeviceToDevice, s), "copy");
     H2D(const_cast<uint32_t*>(A.chunk_sim), chunk_sim.data(), chunk_sim.size() * 4);
     if (!wn.empty()) {
         H2D(A.w_nx, wn.data(), wn.size() * 8);
         H2D(A.w_mvfd, wm.data(), wm.size() * 8);
-        HIPCHK(c, hipMemsetAsync(A.w_acc, 0, wn.size() / 4 * 8, s), "memset");
     }
     std::vector<uint32_t> adj;
     if (!bonds.empty()) {
@@ -768,7 +863,6 @@ int upload_state(sph_ctx* c) {
 // all of them.
 // Device address of `scratch` on each device, looked up once per device
 // with that device current (at the first context opened on it).
-constexpr int SCRATCH_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 double* g_scratch_dev[SCRATCH_MAX_DEVICES] = {};
 
@@ -861,7 +955,8 @@ int open_images(const std::vector<std::pair<const void*, size_t>>& images, int d
     memset(&c->A, 0, sizeof c->A);
     for (Sim& sim : c->sims) fill_params(sim);
     layout(c);
-    if (hipHostMalloc((void**)&c->loop_sample, c->sims.size() * sizeof(DevLoop),
+    const size_t sample_bytes = (c->sims.size() * sizeof(DevLoop) + 255) & ~(size_t)255;
+    if (hipHostMalloc((void**)&c->loop_sample, sample_bytes + STAGE_BYTES,
                       hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->sample_ev, hipEventDisableTiming) != hipSuccess) {
         // Without the sample the automatic placement keeps its first choice.
@@ -870,6 +965,7 @@ int open_images(const std::vector<std::pair<const void*, size_t>>& images, int d
         c->loop_sample = nullptr;
         c->sample_ev = nullptr;
     }
+    if (c->loop_sample) c->stage = reinterpret_cast<char*>(c->loop_sample) + sample_bytes;
     int rc = allocate(c);
     if (rc == SPH_OK) rc = upload_state(c);
     if (rc != SPH_OK) {
@@ -1284,6 +1380,12 @@ int64_t field_bytes(const sph_ctx* c, int k, int f) {
 
 int d2h(sph_ctx* c, void* dst, const void* src, size_t bytes) {
     if (bytes == 0) return SPH_OK;
+    if (c->stage && bytes <= STAGE_BYTES) {
+        HIPCHK(c, hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream), "D2H");
+        HIPCHK(c, hipStreamSynchronize(c->stream), "sync");
+        memcpy(dst, c->stage, bytes);
+        return SPH_OK;
+    }
     HIPCHK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream), "D2H");
     HIPCHK(c, hipStreamSynchronize(c->stream), "sync");
     return SPH_OK;
@@ -2314,7 +2416,8 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     // tape does not fit; then the longest segments that fit.
     size_t free_b = 0, total_b = 0;
     HIPCHK(c, hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-    const double avail = 0.9 * (double)(free_b + c->adj_bytes);
+    const double avail =
+        0.9 * (double)(free_b + c->adj_bytes + tape_pool().held(c->device));
     auto need_for = [&](uint64_t K) {
         const uint64_t nseg = (nsteps + K - 1) / K;
         return (double)per_step * (double)K + (double)state_b +
@@ -2344,15 +2447,16 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
     if (need > (double)c->adj_bytes) {
         HIPCHK(c, hipStreamSynchronize(c->stream), "sync");
         if (c->adj_buf) (void)hipFree(c->adj_buf);
-        c->adj_buf = nullptr;
         c->adj_bytes = 0;
-        if (hipMalloc(&c->adj_buf, (size_t)need) != hipSuccess) {
+        c->adj_buf = tape_pool().take(c->device, (size_t)need, &c->adj_bytes);
+        if (!c->adj_buf) c->adj_bytes = (size_t)need;
+        if (!c->adj_buf && dev_malloc(c, &c->adj_buf, (size_t)need) != hipSuccess) {
             (void)hipGetLastError();
             c->adj_buf = nullptr;
+            c->adj_bytes = 0;
             return fail(c, SPH_E_DEVICE, "hipMalloc failed for the adjoint tape (%.1f GB)",
                         need / 1e9);
         }
-        c->adj_bytes = (size_t)need;
     }
     hipStream_t s = c->stream;
     char* tape = static_cast<char*>(c->adj_buf);
@@ -2900,8 +3004,8 @@ void sph_close(sph_ctx* c) {
         for (hipEvent_t e : c->prof->pool) (void)hipEventDestroy(e);
         delete c->prof;
     }
-    for (void* p : c->allocs) (void)hipFree(p);
-    if (c->adj_buf) (void)hipFree(c->adj_buf);
+    if (c->arena) (void)hipFree(c->arena);
+    tape_pool().give(c->device, c->adj_buf, c->adj_bytes);
     if (c->rd_work) (void)hipFree(c->rd_work);
     if (c->rd_list) (void)hipFree(c->rd_list);
     if (c->rd_stage) (void)hipHostFree(c->rd_stage);
@@ -2909,6 +3013,8 @@ void sph_close(sph_ctx* c) {
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
+
+void sph_trim(void) { (void)tape_pool().trim(-1); }
 
 const char* sph_last_error(const sph_ctx* c) { return c ? c->err.c_str() : g_open_error.c_str(); }
 const char* sph_open_error(void) { return g_open_error.c_str(); }
@@ -2926,7 +3032,7 @@ static int reader_buffer(sph_ctx* c, void** buf, size_t* have, size_t bytes) {
     }
     *buf = nullptr;
     *have = 0;
-    HIPCHK(c, hipMalloc(buf, bytes), "hipMalloc");
+    HIPCHK(c, dev_malloc(c, buf, bytes), "hipMalloc");
     *have = bytes;
     return SPH_OK;
 }
@@ -2971,8 +3077,8 @@ static int overlaps_all_pairs(sph_ctx* c, const double4* x, const double4* vel, 
             return hip_fail(c, ee_, what);     \
         }                                      \
     } while (0)
-    AFAIL(hipMalloc(&counts, (size_t)np * 4), "hipMalloc");
-    AFAIL(hipMalloc(&offs, (size_t)np * 8), "hipMalloc");
+    AFAIL(dev_malloc(c, (void**)&counts, (size_t)np * 4), "hipMalloc");
+    AFAIL(dev_malloc(c, (void**)&offs, (size_t)np * 8), "hipMalloc");
     AFAIL(launch_overlaps(x, vel, np, counts, nullptr, nullptr, nullptr, s), "overlaps");
     std::vector<uint32_t> hc(np);
     std::vector<uint64_t> ho(np);
@@ -2987,8 +3093,8 @@ static int overlaps_all_pairs(sph_ctx* c, const double4* x, const double4* vel, 
     const uint64_t take = std::min<uint64_t>(total, cap);
     if (take > 0) {
         AFAIL(hipMemcpyAsync(offs, ho.data(), (size_t)np * 8, hipMemcpyHostToDevice, s), "H2D");
-        AFAIL(hipMalloc(&dpairs, total * 8), "hipMalloc");
-        AFAIL(hipMalloc(&ddelta, total * 8), "hipMalloc");
+        AFAIL(dev_malloc(c, (void**)&dpairs, total * 8), "hipMalloc");
+        AFAIL(dev_malloc(c, (void**)&ddelta, total * 8), "hipMalloc");
         AFAIL(launch_overlaps(x, vel, np, counts, offs, dpairs, ddelta, s), "overlaps");
         AFAIL(hipMemcpyAsync(pairs, dpairs, take * 8, hipMemcpyDeviceToHost, s), "D2H");
         AFAIL(hipMemcpyAsync(overlaps, ddelta, take * 8, hipMemcpyDeviceToHost, s), "D2H");

@@ -71,7 +71,7 @@ SCALARS = {"time": 0, "time_total": 1, "dt": 2, "file_dt": 3, "iter": 4, "step_c
 SYMBOLS = ("sph_open", "sph_open_mem", "sph_step", "sph_sync", "sph_run", "sph_write_bin",
            "sph_write_mem", "sph_get_field", "sph_set_field", "sph_field_bytes",
            "sph_get_scalar", "sph_set_scalar", "sph_get_contacts", "sph_get_cells",
-           "sph_profile", "sph_profile_report", "sph_close", "sph_last_error",
+           "sph_profile", "sph_profile_report", "sph_close", "sph_trim", "sph_last_error",
            "sph_open_error", "sph_version_string", "sph_open_batch", "sph_open_batch_mem",
            "sph_num_sims", "sph_write_bin_sim", "sph_write_mem_sim", "sph_get_field_sim",
            "sph_set_field_sim", "sph_field_bytes_sim", "sph_get_scalar_sim",
@@ -124,6 +124,8 @@ def load():
     L.sph_profile_report.argtypes = [vp, ctypes.c_char_p, ctypes.c_size_t]
     L.sph_close.argtypes = [vp]
     L.sph_close.restype = None
+    L.sph_trim.argtypes = []
+    L.sph_trim.restype = None
     L.sph_last_error.argtypes = [vp]
     L.sph_last_error.restype = ctypes.c_char_p
     L.sph_open_error.restype = ctypes.c_char_p
@@ -403,6 +405,11 @@ class Context:
             name, us, n = line.split()
             rep[name] = (float(us), int(n))
         return rep
+
+
+def trim():
+    """Give back the device memory kept for later contexts (sph_trim)."""
+    load().sph_trim()
 
 
 def run_file(path, out_dir, sid, verbose=True, dry=False, device=-1, sidecar=False,

@@ -212,3 +212,29 @@ def test_small_total_step_form(n):
             pressed += ref.get("walls_mvfd")[0, 2] != 0.0
         if n > 300:  # (three movers seldom leave their cells)
             assert ctx.scalar("sorts") >= 8 and pressed
+
+
+# A closed context's tape serves the next context that fits into it: smaller
+# (but not by much), larger, much smaller, after everything was given back,
+# recorded whole and in segments, with two contexts open at once.
+@pytest.mark.parametrize("checkpoint", [0, 3])
+def test_adjoint_tapes_of_successive_contexts(checkpoint):
+    beds = {n: cases.lattice_bed(n, 4, 0.01, 0.1).tobytes() for n in (60, 700, 900)}
+    seeds = {n: numpy.random.default_rng(n).standard_normal((n, 3)) for n in beds}
+
+    def gradient(ctx, n):
+        ctx.set_scalar("adj_checkpoint", checkpoint)
+        g = ctx.adjoint(7, seeds[n], None, None)
+        return numpy.concatenate([g["x"].ravel(), g["v"].ravel(), [g["k_n"], g["mu_s"]]])
+
+    want = {}
+    for n, image in beds.items():
+        engine.trim()
+        with engine.Context(image) as ctx:
+            want[n] = gradient(ctx, n)
+    for n in (700, 900, 700, 60, 900):
+        with engine.Context(beds[n]) as ctx, engine.Context(beds[700]) as other:
+            # The same operations in the same order, whatever the memory held.
+            assert numpy.array_equal(gradient(ctx, n), want[n]), n
+            assert numpy.array_equal(gradient(other, 700), want[700]), n
+    engine.trim()
