@@ -334,7 +334,7 @@ int sph_read_state_sim(sph_ctx* ctx, int sim, const char* path);
  * contact workgroup size (128, 256, 512; 4 lanes), the candidate-list
  * capacity (16, 24, 32) and the workgroup order (SPH_S_XCD_ORDER), each
  * judged by the contact kernel's mean time over steps_per_trial steps
- * (HIP events; up to 8,192 particles by the step's kernels together) after
+ * (HIP events; up to 18,432 particles by the step's kernels together) after
  * steps_per_trial / 2 untimed steps; then the radix
  * digit width (4, 6, 8 bits), judged by four full sorts of the current keys.
  * Every setting gives the same results bit for bit, so the trials are

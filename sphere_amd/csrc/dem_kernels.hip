@@ -2788,13 +2788,22 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
 
 // The wall-force block partials of one simulation by one workgroup (the
 // reference's summation kernel, 256 original indices per partial), summed
-// left to right in thread 0; at most 1,024 blocks.  Wall 0's forces come from
-// a compact array: from the particles' output records one workgroup's reads
-// took the step from 18.8 to 21.2 us on 5,000 particles.
+// left to right in thread 0; at most 2,048 blocks.  Bound by the round trips of
+// one workgroup's reads: all of a lane's are out before the first is used
+// (waiting for each took the step from 17.5 to 19.4 us on 8,000 particles), and
+// wall 0's forces come from a compact array (from the particles' output
+// records 25.5 us).
 __device__ __forceinline__ double wall_sum_small(CParams& p, const DevArrays& a, uint32_t w,
                                                  double* stage) {
     constexpr uint32_t WAVES = WALLS_WG / 64;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    // (Walls beyond the side walls take no force: wall_force_pp.)
+    const bool none = w >= OUT_NWALL;
+    const size_t stride = w == 0 ? 1 : 16;
+    const double* const src =
+        w == 0 ? a.wall0 + p.base
+               : reinterpret_cast<const double*>(a.out + (size_t)p.base * 4 + OUT_W) +
+                     (none ? 0u : w - 1u);
     // A wavefront per block: each lane holds the four values block_tree_sum
     // adds first, two blocks' loads in flight.
     for (uint32_t c0 = wave; c0 < p.nblocks; c0 += 2u * WAVES) {
@@ -2804,10 +2813,14 @@ __device__ __forceinline__ double wall_sum_small(CParams& p, const DevArrays& a,
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
                 const uint32_t local = (c0 + h * WAVES) * BLOCK + i * 64u + lane;
-                v[h][i] = 0.0;
-                if (local < p.np)
-                    v[h][i] += w == 0 ? a.wall0[p.base + local]
-                                      : wall_force_pp(a, p.base + local, w);
+                v[h][i] = src[(size_t)(local < p.np ? local : 0u) * stride];
+            }
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h)
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const uint32_t local = (c0 + h * WAVES) * BLOCK + i * 64u + lane;
+                v[h][i] = local < p.np && !none ? 0.0 + v[h][i] : 0.0;
             }
 #pragma unroll
         for (uint32_t h = 0; h < 2; ++h) {

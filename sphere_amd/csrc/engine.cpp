@@ -116,11 +116,12 @@ struct Sim {
 // step is a chain of latencies there, so one pass less and shorter chains per
 // work-item win; beyond it the registers the integration adds cost the
 // throughput and the one workgroup's sum grows.  Step, two kernels / three, in
-// us: 300 particles 17.0 / 19.6, 601 17.3 / 20.2, 3,000 17.7 / 21.6, 5,000
-// 18.8 / 21.8, 8,000 19.7 / 22.0, 10,000 22.9 / 22.5, 12,000 24.3 / 22.9; a
-// column of 4,096 16.2 / 22.1.  (Eight work-items and three kernels: 601 18.0,
-// 5,000 20.6.)
-constexpr uint32_t SMALL_NTOT = 8192;
+// us: 300 particles 15.5 / 19.6, 601 16.2 / 20.2, 3,000 16.4 / 21.6, 8,000
+// 17.4 / 22.0, 12,000 21.4 / 23.5, 15,400 22.0 / 23.5, 20,000 25.3 / 25.2,
+// 30,000 29.4 / 26.9; a column of 4,096 15.5 / 22.1.  (Eight work-items and
+// three kernels: 601 18.0, 5,000 20.6; four work-items and two kernels: 10,000
+// 20.3 against 19.8.)
+constexpr uint32_t SMALL_NTOT = 18432;
 
 constexpr int SCRATCH_MAX_DEVICES = 64;
 constexpr size_t STAGE_BYTES = (size_t)256 << 10;

@@ -180,12 +180,12 @@ def test_overlap_list_edges(n, radius):
         assert numpy.array_equal(pairs, pb[:k]) and numpy.array_equal(delta, db[:k])
 
 
-# The two-kernel step of small totals (up to 8,192 particles with their
+# The two-kernel step of small totals (up to 18,432 particles with their
 # padding) and the three-kernel step just above, re-sorting at nearly every
 # step: a round of the wall-force sum takes 8,192 particles, and settings are
 # changed in between, so that steps of either form, with other list layouts
 # and with stale sorted copies, follow each other.
-@pytest.mark.parametrize("n", [300, 4097, 8192, 8193])
+@pytest.mark.parametrize("n", [300, 4097, 8192, 8193, 18432, 18433])
 def test_small_total_step_form(n):
     rng = numpy.random.default_rng(n)
     s = _cloud(n, 13, r=(0.002, 0.003))
