@@ -106,11 +106,16 @@ enum sph_scalar {
     SPH_S_NSIMS = 13,      /* simulations in the context (read-only) */
     SPH_S_CONTACT_LANES = 14, /* work-items per particle in the contact kernel for
                                  contact models 2 and 3: 1, 4 (default), 8 or 16.
-                                 Results are identical for every value. */
+                                 With the default kernel settings (lanes 4,
+                                 workgroups of 256, integration lanes 1, not fused)
+                                 contexts of up to 18,432 particles use 8 and
+                                 integrate in the same pass.  Results are identical
+                                 for every value. */
     SPH_S_SORT_MODE = 15,   /* where the re-sort runs: 0 = sort launches at each step
                                start, 1 = one workgroup at the end of the previous step
                                when some particle changed cell, 2 (default) = chosen
-                               from the measured re-sort rate.  Identical results. */
+                               from the measured number of particles that change cell
+                               per re-sort.  Identical results. */
     SPH_S_RESORT_MERGE_MAX = 16, /* particles changing cell up to which the end-of-step
                                     re-sort merges them into the previous order
                                     (0..2048, default 2048); above it, it sorts anew. */
@@ -132,8 +137,9 @@ enum sph_scalar {
                                  or 3) the contact kernel also integrates each
                                  particle (one vector component per lane) and a
                                  small pass forms the wall-force partials; 0
-                                 (default, measured faster): separate integration
-                                 kernel.  Identical results. */
+                                 (default, measured faster above 18,432
+                                 particles): separate integration kernel.
+                                 Identical results. */
     SPH_S_WALL_SUMS = 21,     /* per simulation.  0 (default, the reference,
                                  src/device.cu:2504-2505): every dynamic wall
                                  integrates wall 0's force sum; 1: wall w

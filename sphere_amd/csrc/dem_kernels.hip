@@ -1664,9 +1664,14 @@ struct CellScan {
     }
 };
 
-// Four wavefronts per SIMD (128 VGPRs): the compiler's own allocation takes
-// 131 and three; capping it spills 12 bytes per lane and measured 51.3
-// against 54.9 us on the 1e5-particle sheared bed.
+// Four wavefronts per SIMD (127 VGPRs at four lanes, no spills); at five it
+// spills 54 registers and was 4% slower.  On 1e5 sheared particles a steady
+// launch takes 23.5 us (26.6 before the prologue's scalar reads were joined),
+// on 1e6 250.  There several units are each about half busy: VALU 48%, 1,035
+// bytes of HBM traffic per particle at 4.1 TB/s, gathers of up to 64 lines an
+// instruction; shorter lists and rows (190 bytes per particle less) and one
+// round trip less measured no faster.  Below 1e4 particles it is one chain of
+// round trips and dependent FP64 operations, 11 us.
 // WG work-items per workgroup (WG / LPP particles, within one 256-particle
 // chunk).
 template <int CM, int LPP, bool FUSED, int WG>
@@ -2381,9 +2386,10 @@ __global__ __launch_bounds__(BLOCK) void k_tau_sum(const DevArrays a) {
 // next step needs no hash launch; with an adaptive grid (L[2] follows the
 // top wall, which moves after this pass) hash_next is 0.
 
-// Four wavefronts per SIMD (104 VGPRs, no spills).  Five would need 96 and
-// spill (with the per-wall partial sums), measured 5-7% slower both on 1e5
-// particles and on a 1.45e6-particle batch.
+// Four wavefronts per SIMD, no spills.  Five would need 96 VGPRs and spill (with
+// the per-wall partial sums), measured 5-7% slower both on 1e5 particles and
+// on a 1.45e6-particle batch.  Bound by memory: 765 bytes per particle, 150 us
+// on 1e6 particles (5.1 TB/s; a large copy reaches 4.8).
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_integrate(
     const DevArrays a, int hash_next) {
     __shared__ double cache[BLOCK];
@@ -3061,25 +3067,105 @@ __device__ __forceinline__ void apply_bond(const DevArrays& a, uint32_t i, uint3
     touched = true;
 }
 
+// The scan of the whole bond list for particle i by one workgroup: the bonds
+// that touch it are picked 256 at a time (eight such slices requested
+// together), their contributions staged in ascending bond id and added by one
+// work-item per component of force and torque.  Bound by that chain of
+// additions.  One work-item going through the list waited for each bond in
+// turn: 320 us a step on 13,750 particles with a tenth of their contacts bonded; this
+// takes 12.
+__device__ __forceinline__ void scan_bonds(CParams& p, const DevArrays& a, uint32_t i) {
+    constexpr uint32_t U = 8, WAVES = BLOCK / 64;
+    __shared__ unsigned long long s_mask[U][WAVES];
+    __shared__ double s_ft[6][BLOCK];
+    __shared__ uint8_t s_end[BLOCK];  // bit 0: the first end is i, bit 1: the second
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    // Work-items 0..2 add the force's components, 3..5 the torque's.
+    double* const rec = reinterpret_cast<double*>(a.out + (size_t)i * 4 +
+                                                  (tid < 3 ? OUT_F : OUT_T)) +
+                        (tid < 3 ? tid : tid - 3u);
+    double acc = tid < 6 ? *rec : 0.0;
+    bool touched = false;
+    for (uint32_t b0 = 0; b0 < p.nb0; b0 += U * BLOCK) {
+        uint32_t ok[U];
+        uint2 e[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t k = b0 + u * BLOCK + tid;
+            const uint32_t b = p.bond_base + (k < p.nb0 ? k : 0u);
+            ok[u] = k < p.nb0 ? a.bond_ok[b] : 0u;
+            e[u] = reinterpret_cast<const uint2*>(a.bonds)[b];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const unsigned long long m = __ballot(ok[u] != 0u && (e[u].x == i || e[u].y == i));
+            if (lane == 0) s_mask[u][wave] = m;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            uint32_t before = 0, n = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < WAVES; ++w) {
+                const uint32_t c = (uint32_t)__popcll(s_mask[u][w]);
+                before += w < wave ? c : 0u;
+                n += c;
+            }
+            if (n == 0) continue;  // the same for the whole workgroup
+            touched = true;
+            const unsigned long long m = s_mask[u][wave];
+            if ((m >> lane) & 1ull) {
+                const uint32_t b = p.bond_base + b0 + u * BLOCK + tid;
+                const uint32_t at = before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                const double4 f = a.bond_f[b], t = a.bond_t[b];
+                s_ft[0][at] = f.x;
+                s_ft[1][at] = f.y;
+                s_ft[2][at] = f.z;
+                s_ft[3][at] = t.x;
+                s_ft[4][at] = t.y;
+                s_ft[5][at] = t.z;
+                s_end[at] = (uint8_t)((e[u].x == i ? 1u : 0u) | (e[u].y == i ? 2u : 0u));
+            }
+            __syncthreads();
+            if (tid < 6)
+                for (uint32_t k = 0; k < n; ++k) {
+                    // (+f, -t) for the first end, (-f, +t) for the second.
+                    const double v = tid < 3 ? s_ft[tid][k] : -s_ft[tid][k];
+                    const uint32_t end = s_end[k];
+                    if (end & 1u) acc += v;
+                    if (end & 2u) acc -= v;
+                }
+            __syncthreads();
+        }
+        __syncthreads();
+    }
+    if (tid < 6 && touched) *rec = acc;
+}
+
 __global__ __launch_bounds__(BLOCK) void k_bond_gather(const DevArrays a) {
     CParams& p = chunk_params(a, blockIdx.x);
     const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i - p.base >= p.np) return;
-    const bool full = (i - p.base == p.nb0) && a.loop[p.sim].bond_retargeted != 0u;
-    if (a.tape_bond_full && i - p.base == p.nb0) a.tape_bond_full[p.sim] = full ? 1u : 0u;
-    const uint32_t b0 = full ? p.bond_base : a.badj_off[i];
-    const uint32_t b1 = full ? p.bond_base + p.nb0 : a.badj_off[i + 1];
-    if (b0 == b1) return;
-    // Force and torque of the output record (their w parts, es and ev,
-    // pass through unchanged).
-    double4* const rec = a.out + (size_t)i * 4;
-    double4 F = rec[OUT_F], T = rec[OUT_T];
-    bool touched = false;
-    for (uint32_t k = b0; k < b1; ++k) apply_bond(a, i, full ? k : a.badj[k], F, T, touched);
-    if (touched) {
-        rec[OUT_F] = F;
-        rec[OUT_T] = T;
+    // Particle nb0's workgroup scans the list together.
+    const uint32_t who = p.base + p.nb0;
+    const bool scan = p.nb0 < p.np && who / BLOCK == blockIdx.x &&
+                      a.loop[p.sim].bond_retargeted != 0u;
+    if (i - p.base < p.np) {
+        if (a.tape_bond_full && i == who) a.tape_bond_full[p.sim] = scan ? 1u : 0u;
+        const uint32_t b0 = a.badj_off[i], b1 = a.badj_off[i + 1];
+        if (b0 != b1 && !(scan && i == who)) {
+            // Force and torque of the output record (their w parts, es and
+            // ev, pass through unchanged).
+            double4* const rec = a.out + (size_t)i * 4;
+            double4 F = rec[OUT_F], T = rec[OUT_T];
+            bool touched = false;
+            for (uint32_t k = b0; k < b1; ++k) apply_bond(a, i, a.badj[k], F, T, touched);
+            if (touched) {
+                rec[OUT_F] = F;
+                rec[OUT_T] = T;
+            }
+        }
     }
+    if (scan) scan_bonds(p, a, who);
 }
 
 // Self-check of sqrt_rn_f32: the FP32 values with bit patterns in [lo, hi)

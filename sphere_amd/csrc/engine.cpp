@@ -173,7 +173,7 @@ struct sph_ctx {
     // Where a step's re-sort runs: 0 = the per-stage sort launches at the
     // step start (every step; they return at once when nothing changed),
     // 1 = one workgroup per simulation at the end of the previous step, only
-    // when needed, 2 = choose between the two from the measured rate.
+    // when needed, 2 = choose between the two from the movers per re-sort.
     int sort_mode = 2;
     bool resort_at_end = true;     // the choice for the steps being enqueued
     bool prev_walls_resorted = false;

@@ -238,3 +238,30 @@ def test_adjoint_tapes_of_successive_contexts(checkpoint):
             assert numpy.array_equal(gradient(ctx, n), want[n]), n
             assert numpy.array_equal(gradient(other, 700), want[700]), n
     engine.trim()
+
+
+# Particle nb0's scan of the bond list once bonds have broken: 256 bonds
+# exactly, one more, more than one round of 2,048, bonds it holds itself.
+@pytest.mark.parametrize("n,bonds", [(900, 256), (900, 257), (6000, 2049), (60, 7)])
+def test_many_broken_bonds(n, bonds):
+    s = cases.lattice_bed(n, 6, 0.01, 0.1, bond_frac=1.0)
+    assert len(s.bonds) >= bonds and bonds < n
+    rng = numpy.random.default_rng(n + bonds)
+    s.bonds = s.bonds[numpy.sort(rng.choice(len(s.bonds), size=bonds, replace=False))]
+    s.bonds[0] = [bonds, bonds + 1]  # a bond of particle nb0's own
+    s.nb0[0] = bonds
+    for f in ("bonds_delta_n", "bonds_omega_n"):
+        setattr(s, f, numpy.zeros(bonds))
+    for f in ("bonds_delta_t", "bonds_omega_t"):
+        setattr(s, f, numpy.zeros((bonds, 3)))
+    s.vel[:, :3] = rng.normal(0.0, 1.0, (n, 3))
+    s.sigma_b[0] = s.tau_b[0] = 1.0e7
+    image = s.tobytes()
+    ref = oracle.Oracle(image)
+    with engine.Context(image) as ctx:
+        for k in range(4):
+            ctx.step(3)
+            ref.step(3)
+            for f in ("bonds", "bonds_delta", "force", "torque", "x", "vel", "angvel"):
+                assert numpy.array_equal(ctx.get(f), ref.get(f)), (k, f)
+    assert numpy.count_nonzero(ref.get("bonds")[:, 0] == bonds) > bonds // 8
