@@ -124,10 +124,7 @@ __global__ __launch_bounds__(OV_WG) void k_ov_bounds(const double4* __restrict__
     }
 }
 
-// A uniform grid whose cells are at least the largest contact distance
-// (2 r_max, with a margin for the rounding of the cell coordinates) holds
-// every overlapping pair within adjacent cells.  The grid is coarsened until
-// it has at most ncap cells.  Positions that are not finite have no grid.
+// The extremes of all blocks, and the grid chosen from them.
 __global__ __launch_bounds__(64) void k_ov_grid(uint32_t nblocks, OverlapWork w) {
     const uint32_t lane = threadIdx.x;
     double v[8];
@@ -144,27 +141,8 @@ __global__ __launch_bounds__(64) void k_ov_grid(uint32_t nblocks, OverlapWork w)
     }
     if (lane != 0) return;
     OverlapGrid g;
-    g.use = v[7] == 1.0 ? 1 : 0;
-    double maxabs = 0.0, emax = 0.0, ext[3];
-    for (int d = 0; d < 3; ++d) {
-        maxabs = fmax(maxabs, fmax(fabs(v[d]), fabs(v[3 + d])));
-        ext[d] = v[3 + d] - v[d];
-        emax = fmax(emax, ext[d]);
-        g.lo[d] = v[d];
-        g.n[d] = 1;
-    }
-    double h = 2.0 * v[6] * (1.0 + 1e-6) + 1e-12 * maxabs;
-    if (!(h > 0.0)) h = emax > 0.0 ? emax : 1.0;
-    while (g.use) {
-        uint64_t total = 1;
-        for (int d = 0; d < 3; ++d) {
-            g.n[d] = (int)fmin(ext[d] / h, (double)(1 << 20)) + 1;
-            total *= (uint64_t)g.n[d];
-        }
-        if (total <= (uint64_t)w.ncap) break;
-        h *= 1.5;
-    }
-    g.inv_h = 1.0 / h;
+    g.total = 0;
+    choose_overlap_grid(v, w.ncap, g);
     *w.grid = g;
 }
 

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "overlap_grid.hpp"
+
 namespace sphx {
 
 // DEM::findOverlaps over one simulation's np particles (original order):
@@ -12,16 +14,6 @@ namespace sphx {
 // overlaps written from offs[i] (exclusive prefix of counts).
 hipError_t launch_overlaps(const double4* x, const double4* vel, uint32_t np, uint32_t* counts,
                            const uint64_t* offs, uint32_t* pairs, double* delta, hipStream_t s);
-
-// Uniform grid of the overlap search: cells of side 1/inv_h >= the largest
-// contact distance, n[d] cells per axis from lo[d]; key = (z n1 + y) n0 + x.
-struct OverlapGrid {
-    double lo[3];
-    double inv_h;
-    int n[3];
-    int use;                   // 0: positions not finite, no grid
-    unsigned long long total;  // overlaps found
-};
 
 constexpr uint32_t OV_SLAB = 8;      // overlaps kept per particle
 constexpr uint32_t OV_PPB = 64;      // particles per search workgroup
