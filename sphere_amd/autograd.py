@@ -70,10 +70,12 @@ class Trajectory:
     def image(self, theta, x0=None, v0=None):
         """The .bin image of the template with theta (and x0, v0) applied."""
         # The template's own arrays but for the changed ones (a decoded copy of
-        # all of them where a changed one is not as a decoded one would be).
+        # all of them where a changed one is not a 1-D array of doubles, as a
+        # decoded one would be).
         s = copy.copy(self.template)
-        fields = [f for name in self.params for f in self.ties[name]]
-        if any(getattr(getattr(s, f), "dtype", None) != numpy.float64 for f in fields):
+        changed = [getattr(s, f) for name in self.params for f in self.ties[name]]
+        if not all(isinstance(a, numpy.ndarray) and a.dtype == numpy.float64 and a.ndim == 1
+                   for a in changed):
             from .sim import sim
             s = sim().frombytes(s.tobytes())
         for name, value in zip(self.params, numpy.asarray(theta, dtype=numpy.float64)):

@@ -28,3 +28,21 @@ def test_image_of_a_trajectory(k_n, state):
         want.x[:, :3], want.vel[:, :3] = x, v
     assert got == want.tobytes()
     assert s.tobytes() == before and s.k_n.dtype == k_n.dtype
+
+
+@pytest.mark.parametrize("field,value,first", [
+    ("k_n", numpy.float64(5.0e5), 5.0e5), ("k_n", numpy.array(5.0e5), 5.0e5),
+    ("k_n", 5.0e5, 5.0e5), ("k_n", numpy.array([[5.0e5]]), 5.0e5),
+    ("k_n", numpy.array([5.0e5, 7.0]), 5.0e5),
+    ("g", numpy.array([[1.0, 2.0, -9.81]]), [1.0, 2.0, -9.81])])
+def test_image_of_a_template_with_other_shapes(field, value, first):
+    """A parameter the template holds as a number, or in an array of another
+    shape than a decoded one: its first entry changes and nothing else."""
+    s = cases.lattice_bed(130, 1, 0.01, 0.1)
+    want = sim().frombytes(s.tobytes())
+    getattr(want, field)[:] = first
+    getattr(want, field)[0] = 1.5e6
+    setattr(s, field, value)
+    t = Trajectory(s, 5, 4, params=("p",), ties={"p": (field,)})
+    assert t.image([1.5e6]) == want.tobytes()
+    assert getattr(s, field) is value
