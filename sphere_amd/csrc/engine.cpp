@@ -132,6 +132,7 @@ struct AdjHostMark {
     std::vector<double> t;
     std::vector<int64_t> iter;
     bool hash_pending, prev_walls_resorted, copies_fresh;
+    int list_lanes;  // the lists and their hit masks are among what a checkpoint holds
 };
 
 // A recorded forward pass awaiting its reverse (sph_adjoint_record).
@@ -2605,6 +2606,7 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             hm.hash_pending = c->hash_pending;
             hm.prev_walls_resorted = c->prev_walls_resorted;
             hm.copies_fresh = c->copies_fresh;
+            hm.list_lanes = c->list_lanes;
         } else {
             for (size_t k = 0; k < nsim; ++k) {
                 c->sims[k].h.t = hm.t[k];
@@ -2613,6 +2615,7 @@ static int adjoint_run(sph_ctx* c, uint64_t nsteps, const double* dL_dx, const d
             c->hash_pending = hm.hash_pending;
             c->prev_walls_resorted = hm.prev_walls_resorted;
             c->copies_fresh = hm.copies_fresh;
+            c->list_lanes = hm.list_lanes;
         }
         return SPH_OK;
     };

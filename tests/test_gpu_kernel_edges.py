@@ -265,3 +265,44 @@ def test_many_broken_bonds(n, bonds):
             for f in ("bonds", "bonds_delta", "force", "torque", "x", "vel", "angvel"):
                 assert numpy.array_equal(ctx.get(f), ref.get(f)), (k, f)
     assert numpy.count_nonzero(ref.get("bonds")[:, 0] == bonds) > bonds // 8
+
+
+# A segmented reverse pass goes back to a checkpoint whose hit masks another
+# number of lanes wrote.  Particle 0 holds particle 2 (the second entry of its
+# list: bit 4 of a mask of eight lanes) and loses it in the very step in which
+# particle 3 (the third entry: bit 4 with sixteen lanes) reaches it, the first
+# of the reverse pass.
+@pytest.mark.parametrize("lanes", [1, 4, 8, 16])
+def test_adjoint_segments_after_a_change_of_lanes(lanes):
+    r, dt, v = 0.01, 1.0e-5, 0.01
+    s = sim(np=5, sid="lanes")
+    s.radius[:] = [r, r, r, r, 0.03]
+    d = 4.5 * v * dt  # an overlap and a gap that both end after 4.5 steps
+    s.x = numpy.array([0.06, 0.03, 0.03]) + numpy.array([
+        [0.0, 0.0, 0.0], [2.02 * r, 0.0, 0.0], [0.0, 2.0 * r - d, 0.0], [0.0, 0.0, 2.0 * r + d],
+        [0.1, 0.1, 0.1]])
+    s.vel[2, 1], s.vel[3, 2] = v, -v
+    s.defaultParams(mu_s=0.5, mu_d=0.5, rho=2600.0, k_n=1.0e3, k_t=1.0e3)
+    s.g[:] = 0.0
+    s.normalBoundariesXY()
+    s.defineWorldBoundaries(L=[0.24, 0.24, 0.24])
+    s.time_dt[0], s.time_current[0], s.time_total[0], s.time_file_dt[0] = dt, 0.0, 1.0, 1.0
+    image = s.tobytes()
+    seed = numpy.random.default_rng(3).standard_normal((5, 3))
+    ref = oracle.Oracle(image)
+    held = []
+    for n in (5, 1):
+        ref.step(n)
+        held.append(set(ref.get("contacts")[0]) - {5})
+    assert held == [{2}, {3}]
+    got = []
+    for checkpoint in (0, 5):
+        with engine.Context(image) as ctx:
+            ctx.step(5)
+            ctx.set_scalar("contact_lanes", lanes)
+            ctx.set_scalar("adj_checkpoint", checkpoint)
+            g = ctx.adjoint(10, seed, seed, None)
+            got.append([g["x"], g["v"], ctx.get("contacts"), ctx.get("x")])
+    # The same steps reversed in the same order.
+    for a, b in zip(*got):
+        assert numpy.array_equal(a, b)
