@@ -306,3 +306,42 @@ def test_adjoint_segments_after_a_change_of_lanes(lanes):
     # The same steps reversed in the same order.
     for a, b in zip(*got):
         assert numpy.array_equal(a, b)
+
+
+def _contact_case(case):
+    s = {"settling": lambda: cases.settling_case(1200, 12), "crowded": cases.crowded_case,
+         "fcc": cases.fcc_case, "shear1k": lambda: cases.fixture("shear1k.bin"),
+         "bed": lambda: cases.lattice_bed(18500, 8, 0.01, 0.1)}[case.split("-")[0]]()
+    if case.endswith("hertz"):
+        s.contactmodel[0] = 3
+    return s
+
+
+# The contact pass of large contexts (four lanes, workgroups of 256, apart from
+# the integration) on small beds, where the default settings take the pass of
+# eight lanes that also integrates (another setting of the integration leaves
+# it), that default pass, and a Hertzian bed just above its limit: re-sorts,
+# a row that overflows, several rounds of contacts a wavefront, either order of
+# the workgroups.
+@pytest.mark.parametrize("form", ["four lanes", "default"])
+@pytest.mark.parametrize("case", ["settling", "settling-hertz", "crowded", "crowded-hertz", "fcc",
+                                  "fcc-hertz", "shear1k-hertz", "shear1k-xcd", "bed-hertz"])
+def test_contact_pass_of_either_form(case, form):
+    s = _contact_case(case)
+    image, steps = s.tobytes(), 10 if case == "bed-hertz" else 50
+    ref = oracle.Oracle(image)
+    with engine.Context(image) as ctx:
+        if case.endswith("xcd"):
+            ctx.set_scalar("xcd_order", 1)
+        if form == "four lanes":
+            ctx.set_scalar("integrate_lanes", 4)
+        ctx.profile(True)
+        for _ in range(4):
+            ctx.step(steps)
+            ref.step(steps)
+            for f in ("perm", "contacts", "x", "vel", "angvel", "force", "torque", "p", "es", "ev",
+                      "delta_t"):
+                assert numpy.array_equal(ctx.get(f), ref.get(f)), f
+        stages = {k: n for k, (_, n) in ctx.profile_report().items()}
+    apart = form == "four lanes" or case == "bed-hertz"
+    assert ("integrate" in stages) == apart and ("contact_integrate" in stages) != apart, stages
