@@ -536,7 +536,11 @@ void layout(sph_ctx* c) {
 constexpr size_t TAPE_KEEP = (size_t)8 << 30;
 struct TapePool {
     std::mutex mu;
-    struct Slot { void* p = nullptr; size_t bytes = 0; } slot[SCRATCH_MAX_DEVICES];
+    struct Slot {
+        void* p = nullptr;
+        size_t bytes = 0;
+        bool passed_over = false;  // a context needed far less since it was put here
+    } slot[SCRATCH_MAX_DEVICES];
     static bool known(int device) { return device >= 0 && device < SCRATCH_MAX_DEVICES; }
     size_t held(int device) {
         if (!known(device)) return 0;
@@ -544,11 +548,14 @@ struct TapePool {
         return slot[device].bytes;
     }
     // A kept buffer of at least `need` bytes (and not of many times as many),
-    // or null; one that is too small is freed.
+    // or null; one that is too small is freed, one that is far too large makes
+    // way for the next that is put here (it stays for a context that takes it
+    // before).
     void* take(int device, size_t need, size_t* bytes) {
         if (!known(device)) return nullptr;
         std::lock_guard<std::mutex> lock(mu);
         Slot& s = slot[device];
+        if (s.bytes / 8 > need) s.passed_over = true;
         if (!s.p || s.bytes / 8 > need) return nullptr;
         void* p = s.p;
         *bytes = s.bytes;
@@ -562,9 +569,10 @@ struct TapePool {
         if (known(device) && bytes <= TAPE_KEEP) {
             std::lock_guard<std::mutex> lock(mu);
             Slot& s = slot[device];
-            if (bytes > s.bytes) {
+            if (bytes > s.bytes || s.passed_over) {
                 std::swap(p, s.p);
                 s.bytes = bytes;
+                s.passed_over = false;
             }
         }
         if (p) (void)hipFree(p);

@@ -345,3 +345,28 @@ def test_contact_pass_of_either_form(case, form):
         stages = {k: n for k, (_, n) in ctx.profile_report().items()}
     apart = form == "four lanes" or case == "bed-hertz"
     assert ("integrate" in stages) == apart and ("contact_integrate" in stages) != apart, stages
+
+
+# A kept tape many times larger than the next context's is given back, and that
+# context's own is kept instead.
+def test_adjoint_tape_kept_follows_use():
+    import torch
+    small, large = (cases.lattice_bed(n, 4, 0.01, 0.1).tobytes() for n in (60, 900))
+
+    def adjoint(image, n, steps):
+        with engine.Context(image) as ctx:
+            return ctx.adjoint(steps, numpy.ones((n, 3)), None, None)["x"]
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    want = adjoint(small, 60, 7)
+    engine.trim()
+    before = free()
+    adjoint(large, 900, 300)  # 1,260 bytes a particle and step: 0.39 GB
+    assert before - free() > 0.3e9
+    for _ in range(2):
+        assert numpy.array_equal(adjoint(small, 60, 7), want)
+        assert before - free() < 0.1e9
+    engine.trim()
