@@ -2208,7 +2208,9 @@ int sph_set_scalar_sim(sph_ctx* c, int sim, int which, double v) {
             const int64_t it = (int64_t)v;
             c->hash_pending = true;
             // The sorted copies the next step reads follow the counter's
-            // parity: move them along when it changes.
+            // parity: move them along when it changes.  The last step may
+            // have re-sorted for the next one and noted under that step's
+            // parity that the lists are to be rebuilt in the new order.
             if (((it ^ c->sims[0].iter) & 1) != 0) {
                 const size_t bytes = (size_t)c->A.ntot * 32;
                 const int from = (int)(c->sims[0].iter & 1), to = from ^ 1;
@@ -2216,6 +2218,10 @@ int sph_set_scalar_sim(sph_ctx* c, int sim, int which, double v) {
                 for (auto set : sets)
                     HIPCHK(c, hipMemcpyAsync(set[to], set[from], bytes, hipMemcpyDeviceToDevice,
                                              c->stream), "copy");
+                for (size_t k = 0; k < c->sims.size(); ++k) {
+                    const int rc = set_loop_flag(c, (int)k, &DevLoop::force_rebuild);
+                    if (rc) return rc;
+                }
             }
             for (size_t k = 0; k < c->sims.size(); ++k) {
                 c->sims[k].iter = it;
