@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "dem_arrays.hpp"
+#include "dem_cells.hpp"
 #include "dem_kernels.hpp"
 #include "dem_math.hpp"
 #include "dem_scalar.hpp"
@@ -699,34 +700,6 @@ __device__ __forceinline__ void capillary_cohesion_exp(CParams& p, Acc& A, doubl
     A.F += f_c;
 }
 
-// findDistMod, src/contactsearch.cuh:12-83.  Returns the image code (see
-// CW_SHIFT_*) or -1 when the target cell lies outside the grid.
-__device__ __forceinline__ int find_dist_mod(CParams& p, int& tx, int& ty, int tz) {
-    const int nx = (int)p.num[0], ny = (int)p.num[1], nz = (int)p.num[2];
-    int code = 0;
-    if (p.periodic == 1) {
-        if (tx < 0) { tx += nx; code |= 1; }
-        if (tx >= nx) { tx -= nx; code |= 2; }
-        if (ty < 0) { ty += ny; code |= 4; }
-        if (ty >= ny) { ty -= ny; code |= 8; }
-    }
-    if (p.periodic == 2) {
-        if (tx < 0) { tx += nx; code |= 1; }
-        if (tx >= nx) { tx -= nx; code |= 2; }
-        if (ty < 0 || ty >= ny) return -1;
-    }
-    if (p.periodic > 2 || p.periodic < 1) {
-        if (tx < 0 || tx >= nx) return -1;
-        if (ty < 0 || ty >= ny) return -1;
-    }
-    if (tz < 0 || tz >= nz) return -1;
-    // A particle far outside the grid can leave tx/ty out of range after one
-    // periodic shift; the reference then reads outside cellStart.  Such a
-    // cell is skipped here.
-    if (tx < 0 || tx >= nx || ty < 0 || ty >= ny) return -1;
-    return code;
-}
-
 // The image shift of a code, exactly as findDistMod builds it from zero.
 __device__ __forceinline__ d3 shift_of(CParams& p, uint32_t code) {
     d3 s = mk3(0.0, 0.0, 0.0);
@@ -960,9 +933,9 @@ __global__ __launch_bounds__(BLOCK, CONTACT_MIN_BLOCKS) void k_contact(const Dev
     A.ev_dot = 0.0;
     A.p = 0.0;
     // src/contactsearch.cuh:352-354
-    const int gx = (int)floor((xa.x - p.origo[0]) / (p.L[0] / p.num[0]));
-    const int gy = (int)floor((xa.y - p.origo[1]) / (p.L[1] / p.num[1]));
-    const int gz = (int)floor((xa.z - p.origo[2]) / (Lz / p.num[2]));
+    const int gx = cell_coord((xa.x - p.origo[0]) / (p.L[0] / p.num[0]), (int)p.num[0]);
+    const int gy = cell_coord((xa.y - p.origo[1]) / (p.L[1] / p.num[1]), (int)p.num[1]);
+    const int gz = cell_coord((xa.z - p.origo[2]) / (Lz / p.num[2]), (int)p.num[2]);
     if constexpr (CM == 2 || CM == 3) {
         const uint4* grow = reinterpret_cast<const uint4*>(a.crow + (size_t)ia_orig * NC);
 #pragma unroll
@@ -1606,9 +1579,9 @@ struct CellScan {
     __device__ __forceinline__ CellScan(const LaneGroup<LPP>& g, CParams& p, const DevArrays& a,
                                         const double4 xa, double Lz, uint32_t* lds) {
         constexpr int R = (27 + LPP - 1) / LPP;
-        const int gx = (int)floor((xa.x - p.origo[0]) / (p.L[0] / p.num[0]));
-        const int gy = (int)floor((xa.y - p.origo[1]) / (p.L[1] / p.num[1]));
-        const int gz = (int)floor((xa.z - p.origo[2]) / (Lz / p.num[2]));
+        const int gx = cell_coord((xa.x - p.origo[0]) / (p.L[0] / p.num[0]), (int)p.num[0]);
+        const int gy = cell_coord((xa.y - p.origo[1]) / (p.L[1] / p.num[1]), (int)p.num[1]);
+        const int gz = cell_coord((xa.z - p.origo[2]) / (Lz / p.num[2]), (int)p.num[2]);
         uint32_t s[R], n[R];
 #pragma unroll
         for (int i = 0; i < R; ++i) {
