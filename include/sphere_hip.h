@@ -108,8 +108,10 @@ enum sph_scalar {
                                  contact models 2 and 3: 1, 4 (default), 8 or 16.
                                  With the default kernel settings (lanes 4,
                                  workgroups of 256, integration lanes 1, not fused)
-                                 contexts of up to 18,432 particles use 8 and
-                                 integrate in the same pass.  Results are identical
+                                 contexts of up to 18,432 particles use 8 and,
+                                 with a fixed grid height and without bonds and
+                                 wmode-3 walls, integrate in the same pass; a 4 that
+                                 is set is that default too.  Results are identical
                                  for every value. */
     SPH_S_SORT_MODE = 15,   /* where the re-sort runs: 0 = sort launches at each step
                                start, 1 = one workgroup at the end of the previous step

@@ -1638,13 +1638,15 @@ struct CellScan {
 };
 
 // Four wavefronts per SIMD (127 VGPRs at four lanes, no spills); at five it
-// spills 54 registers and was 4% slower.  On 1e5 sheared particles a steady
-// launch takes 23.5 us (26.6 before the prologue's scalar reads were joined),
-// on 1e6 250.  There several units are each about half busy: VALU 48%, 1,035
-// bytes of HBM traffic per particle at 4.1 TB/s, gathers of up to 64 lines an
-// instruction; shorter lists and rows (190 bytes per particle less) and one
-// round trip less measured no faster.  Below 1e4 particles it is one chain of
-// round trips and dependent FP64 operations, 11 us.
+// spills 54 registers and was 4% slower.  A steady launch takes 23.6 us on a
+// bed of 1e5 tiled from a settled cell (2.3 occupied slots a particle; 26.6
+// before the prologue's scalar reads were joined), 27.6 on the benchmark's
+// settled bed of 1e5 (2.95 slots), 250 on 1e6 tiled.  There several units are
+// each about half busy: VALU 48%, 1,035 bytes of HBM traffic per particle at
+// 4.1 TB/s, gathers of up to 64 lines an instruction; shorter lists and rows
+// (190 bytes per particle less) and one round trip less measured no faster.
+// Below 1e4 particles it is one chain of round trips and dependent FP64
+// operations, 11 us.
 // WG work-items per workgroup (WG / LPP particles, within one 256-particle
 // chunk).
 template <int CM, int LPP, bool FUSED, int WG>

@@ -13,7 +13,8 @@ namespace sphx {
 // has not seen in this launch; after one such pass they all hit.  Measured
 // with the contact pass's first loads ungated (no chunk map for one
 // simulation, list entries and position requested with the original index):
-// contact 13.3 -> 11.4 us on 601 particles, 26.2 -> 23.9 on 1e5; integration
+// contact 13.3 -> 11.4 us on 601 particles, 26.2 -> 23.9 on 1e5 (beds tiled from
+// settled cells); integration
 // 6.2 -> 5.8 and walls 3.3 -> 3.0 on 601.
 typedef const __attribute__((address_space(4))) void cvoid;
 template <uint32_t BYTES, uint32_t BYTES2 = 0>

@@ -121,6 +121,13 @@ struct Sim {
 // 30,000 29.4 / 26.9; a column of 4,096 15.5 / 22.1.  (Eight work-items and
 // three kernels: 601 18.0, 5,000 20.6; four work-items and two kernels: 10,000
 // 20.3 against 19.8.)
+// A step that cannot be fused (bonds, adaptive grid, wmode-3 wall) takes eight
+// work-items in its contact pass up to the same line.  Step, eight / four
+// work-items, in us, sheared beds with 2% of the contacts bonded: 503 particles
+// 28.7 / 29.2, 2,515 29.8 / 31.2, 8,048 31.3 / 33.1, 12,072 33.7 / 35.1, 16,096
+// 35.4 / 36.3, 18,108 35.9 / 36.3; with a wmode-3 wall 8,048 27.6 / 28.3, 16,096
+// 31.1 / 31.3, 18,108 31.7 / 31.6; Hertzian with bonds 8,048 30.0 / 30.9, 16,096
+// 34.7 / 34.6, 18,108 35.7 / 35.3; adaptive grid: equal at every size.
 constexpr uint32_t SMALL_NTOT = 18432;
 
 constexpr int SCRATCH_MAX_DEVICES = 64;
