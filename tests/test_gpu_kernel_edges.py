@@ -397,3 +397,29 @@ def test_counter_parity_after_a_resort(n, model):
             ref.step(1)
             for f in ("perm", "contacts", "x", "vel", "force", "p"):
                 assert numpy.array_equal(ctx.get(f), ref.get(f)), (k, f)
+
+
+# Particles of more overlaps than the search keeps (8): the first of a cluster
+# of n in which all overlap has n - 1, ordered in LDS (up to 512) or in place,
+# beside particles of few; clusters on both sides of a block of 64, and a
+# particle that touches 300 others of one small size.
+@pytest.mark.parametrize("n", [9, 10, 74, 513, 514, 700, 1500, "one"])
+def test_overlap_lists_of_many(n):
+    rng = numpy.random.default_rng(7)
+    if n == "one":
+        s = _cloud(301, 3)
+        u = rng.standard_normal((300, 3))
+        s.radius[0], s.radius[1:] = 0.2, 0.004
+        s.x[0] = 0.25
+        s.x[1:] = 0.25 + 0.201 * u / numpy.linalg.norm(u, axis=1)[:, None]
+        order = rng.permutation(301)
+        s.radius, s.x = s.radius[order], s.x[order]
+    else:
+        s = _cloud(n + 200, 3, r=(0.004, 0.006))
+        s.x[60:60 + n] = 0.25 + rng.uniform(-0.002, 0.002, (n, 3))
+    image = s.tobytes()
+    pb, db = oracle.Oracle(image).find_overlaps()
+    assert numpy.bincount(pb[:, 0]).max() >= (8 if n == "one" else n - 1)
+    with engine.Context(image) as ctx:
+        pa, da = ctx.find_overlaps()
+        assert numpy.array_equal(pa, pb) and numpy.array_equal(da, db)
