@@ -116,8 +116,8 @@ enum sph_scalar {
     SPH_S_SORT_MODE = 15,   /* where the re-sort runs: 0 = sort launches at each step
                                start, 1 = one workgroup at the end of the previous step
                                when some particle changed cell, 2 (default) = chosen
-                               from the measured number of particles that change cell
-                               per re-sort.  Identical results. */
+                               from the measured part of the order that re-sorts
+                               rewrite and how often.  Identical results. */
     SPH_S_RESORT_MERGE_MAX = 16, /* particles changing cell up to which the end-of-step
                                     re-sort merges them into the previous order
                                     (0..2048, default 2048); above it, it sorts anew. */

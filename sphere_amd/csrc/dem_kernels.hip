@@ -2539,7 +2539,8 @@ constexpr uint32_t MV_WAVE = 64;     // movers up to which each search takes a w
 // listed; with more, the whole span between the first and the last such
 // place is rewritten.  Each mover is recorded with its old and new place, so
 // that the finished step's order can be told afterwards.  Returns
-// DevLoop::resorted_last.
+// DevLoop::resorted_last; `share` receives the part that is rewritten, in
+// 1/1024 (RESORT_ANEW: sorted anew).  With `dry` nothing but that is done.
 //
 // Copying and rebuilding all places and cells in 256 work-items took 55-78 us
 // on a column of 4,096 in a wide grid and 300 us on 20,000 particles; this
@@ -2551,7 +2552,7 @@ constexpr uint32_t MV_WAVE = 64;     // movers up to which each search takes a w
 // writes the copies in the new order.
 __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp, int passes,
                                      int bits, int sorted_bits, bool fresh, uint32_t nxt,
-                                     bool& stale) {
+                                     bool dry, bool& stale, uint32_t& share) {
     __shared__ unsigned long long comp[MV_CAP];  // movers' (new key, index), ascending
     __shared__ uint32_t rk[MV_CAP];              // movers' old positions, ascending
     __shared__ uint32_t npos[MV_CAP];            // movers' new positions
@@ -2568,6 +2569,8 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
     // The radix sort orders by the low bits * passes bits of the key.
     const uint32_t kmask = bits * passes >= 32 ? 0xffffffffu : ((1u << (bits * passes)) - 1u);
     if (!(M > 0 && M <= p.mv_max && M <= MV_CAP)) {
+        share = RESORT_ANEW;
+        if (dry) return 0;
         // Sort anew, keeping the order the finished step used.
         for (uint32_t j = tid; j < N; j += WALLS_WG) {
             a.skey_bk[B + j] = a.skey[B + j];
@@ -2608,9 +2611,11 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
             comp[m] = composite(key, kmask, o);
             rk[m] = r;
             okey[m] = a.skey[B + r];
-            a.key_prev[o] = key;
-            if (sorted_bits < 32 && (key >> sorted_bits) != 0u)
-                atomicOr(&lp->error_bits, (uint32_t)DFLAG_KEY_RANGE);
+            if (!dry) {
+                a.key_prev[o] = key;
+                if (sorted_bits < 32 && (key >> sorted_bits) != 0u)
+                    atomicOr(&lp->error_bits, (uint32_t)DFLAG_KEY_RANGE);
+            }
         }
     }
     __syncthreads();
@@ -2657,11 +2662,12 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
         }
     }
     __syncthreads();
-    for (uint32_t m = tid; m < M; m += WALLS_WG) {
-        const uint32_t o = (uint32_t)(comp[m] & 0xffffffffull);
-        const uint32_t r = a.rank[o] - B;
-        rec[m] = make_uint4(o, a.skey[B + r], r, npos[m]);
-    }
+    if (!dry)
+        for (uint32_t m = tid; m < M; m += WALLS_WG) {
+            const uint32_t o = (uint32_t)(comp[m] & 0xffffffffull);
+            const uint32_t r = a.rank[o] - B;
+            rec[m] = make_uint4(o, a.skey[B + r], r, npos[m]);
+        }
     // The runs to rewrite.
     uint32_t nrun = 1;
     if (few) {
@@ -2694,6 +2700,8 @@ __device__ uint32_t resort_one_block(CParams& p, const DevArrays& a, DevLoop* lp
     }
     __syncthreads();
     const uint32_t total = roff[nrun];
+    share = (uint32_t)(((uint64_t)total * 1024u + N - 1u) / N);
+    if (dry) return 0;
     // Place t of the runs; `last` where it ends its run.
     auto place_of = [&](uint32_t t, bool& last) {
         const uint32_t k = nrun == 1 ? 0u : count_below(roff, nrun, t + 1u) - 1u;
@@ -2825,10 +2833,11 @@ __device__ __forceinline__ double wall_sum_small(CParams& p, const DevArrays& a,
 // integrateWalls + the loop advance (src/integration.cuh:344-450,
 // src/device.cu:2454-2462,2500-2538), one workgroup.  Every dynamic wall
 // integrates wall 0's force sum (src/device.cu:2504-2505).  With `resort`
-// set it first re-sorts for the next step when the integration pass found
+// 1 or 2 it first re-sorts for the next step when the integration pass found
 // particles that changed cell (the next step then launches no sort); with 2
 // it always refreshes the sorted copies (a contact pass that integrates
-// writes the arrays a stale reader would read).  With `partials` set no pass
+// writes the arrays a stale reader would read).  With -1 it only measures
+// what such a re-sort would rewrite, every sixteenth step.  With `partials` set no pass
 // before it has formed the wall-force partials nor kept the order of the rows.
 __global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resort, int partials,
                                                     int passes, int bits, int sorted_bits) {
@@ -2838,7 +2847,10 @@ __global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resor
     touch_sim(a, blockIdx.x);
     CParams& p = sim_params(a, blockIdx.x);  // one workgroup per simulation
     DevLoop* lp = a.loop + blockIdx.x;
-    if (threadIdx.x == 0) do_sort = (resort && lp->changed[step_slot(lp) ^ 1u]) ? 1u : 0u;
+    if (threadIdx.x == 0)
+        do_sort = !lp->changed[step_slot(lp) ^ 1u] ? 0u
+                  : resort > 0                     ? 1u
+                  : resort < 0 && (lp->iter & 15) == 0 && lp->nmovers ? 2u : 0u;
     __shared__ double s_fsum[MAXWALLS];
     const bool walls = p.nw > 0 && p.np > 0;
     // Work-item w integrates wall w (src/integration.cuh:344-450).  Its
@@ -2887,11 +2899,12 @@ __global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resor
     }
     __syncthreads();
     const uint32_t movers = lp->nmovers;
-    uint32_t resorted = 0;
+    uint32_t resorted = 0, share = 0;
     bool stale = false;
-    if (do_sort)
+    const uint32_t sorting = do_sort;
+    if (sorting)
         resorted = resort_one_block(p, a, lp, passes, bits, sorted_bits, resort == 2, slot ^ 1u,
-                                    stale);
+                                    sorting == 2u, stale, share);
     if (mine) {
         const uint32_t wi = p.wall_base + w;
         w_mvfd.z = s_fsum[p.wall_sums ? w : 0u];  // 0.0 + partial[0] + partial[1] + ...
@@ -2905,13 +2918,16 @@ __global__ __launch_bounds__(WALLS_WG) void k_walls(const DevArrays a, int resor
         a.w_acc[wi] = acc;
     }
     if (threadIdx.x != 0) return;
-    if (do_sort) lp->sorts = sorts + 1u;
+    if (sorting == 1u) lp->sorts = sorts + 1u;
     lp->resorted_last = resorted;
     if (resorted == RESORTED_MERGE) lp->nmv_last = movers;
-    if (movers) lp->moved += movers;
+    if (sorting) {
+        lp->shifted += share;
+        lp->measured += 1u;
+    }
     // The next step's contact pass maps its rows to the new order and reads
     // the state through perm.
-    lp->order_changed = do_sort;
+    lp->order_changed = sorting == 1u ? 1u : 0u;
     lp->copies_stale = stale ? 1u : 0u;
     if (p.adaptive == 1 && walls) lp->grid_Lz = grid_top;
     if (t_now >= 10.0 && t_now < 15.0 && vstate == 1) lp->velocity_state = 2;

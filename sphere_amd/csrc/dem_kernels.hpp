@@ -54,10 +54,11 @@ hipError_t launch_integrate(const DevArrays& a, int hash_next, hipStream_t s);
 // height, no wmode-3 wall.
 hipError_t launch_integrate_q(const DevArrays& a, hipStream_t s);
 // Per simulation: serial sum of the partials + integrateWalls + loop advance
-// (src/integration.cuh:344-450, src/device.cu:2500-2538).  With resort != 0
+// (src/integration.cuh:344-450, src/device.cu:2500-2538).  With resort 1 or 2
 // it also re-sorts the simulation for the next step, in one workgroup, when
 // the integration pass (launched with hash_next) found a cell change; with 2
-// the sorted copies follow.  With partials != 0 it forms the partials itself.
+// the sorted copies follow; with -1 it measures now and then what that would
+// rewrite.  With partials != 0 it forms the partials itself.
 hipError_t launch_check_sqrt32(unsigned long long* bad, uint64_t lo, uint64_t hi, hipStream_t s);
 hipError_t launch_walls(const DevArrays& a, int resort, int partials, int passes, int bits,
                         int sorted_bits, hipStream_t s);

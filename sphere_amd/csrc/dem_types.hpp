@@ -140,13 +140,17 @@ struct DevLoop {
     uint32_t copies_stale;      // the sorted copies are in the previous order (read
                                 // the original-index arrays through perm instead)
     uint32_t nmv_last;          // records of the last merge (DevArrays::mv_last)
-    uint32_t moved;             // particles that changed cell so far (diagnostic)
-    uint32_t pad1;
+    uint32_t shifted;           // places that re-sorts rewrite, summed over the measured
+                                // ones, in 1/1024 of the simulation (RESORT_ANEW: a sort)
+    uint32_t measured;          // re-sorts measured so far
 };
 
 // DevLoop::resorted_last: how the previous order is kept.
 constexpr uint32_t RESORTED_FULL = 1u;
 constexpr uint32_t RESORTED_MERGE = 2u;
+// DevLoop::shifted of a re-sort that sorts anew: it costs the workgroup about as
+// much as rewriting every place twice in small totals (up to six times beyond).
+constexpr uint32_t RESORT_ANEW = 2048u;
 
 // Batch-wide state.
 struct DevGlobal {

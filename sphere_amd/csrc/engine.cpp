@@ -181,7 +181,7 @@ struct sph_ctx {
     // Where a step's re-sort runs: 0 = the per-stage sort launches at the
     // step start (every step; they return at once when nothing changed),
     // 1 = one workgroup per simulation at the end of the previous step, only
-    // when needed, 2 = choose between the two from the movers per re-sort.
+    // when needed, 2 = choose between the two from what re-sorts rewrite.
     int sort_mode = 2;
     bool resort_at_end = true;     // the choice for the steps being enqueued
     bool prev_walls_resorted = false;
@@ -196,7 +196,7 @@ struct sph_ctx {
     bool sample_pending = false;
     int64_t sample_iter0 = 0;
     uint64_t sample_sorts0 = 0;
-    uint32_t sample_moved0 = 0;
+    uint32_t sample_shifted0 = 0, sample_measured0 = 0;
     // Steady-state step chunks replayed from captured HIP graphs (0 = off):
     // one graph per (chunk length, re-sort placement, contact lanes).
     int graph_steps = 0;
@@ -1077,61 +1077,6 @@ void prof_collect(sph_ctx* c) {
     ps.pending.clear();
 }
 
-// Re-sort placement for the steps about to be enqueued.  In automatic mode
-// the choice follows the particles that changed cell per re-sort over the
-// previous sph_step call, read from an asynchronous copy of the loop counters
-// (no synchronisation).  The end-of-step workgroup rewrites only what the
-// movers shift; the sort launches cost 16-20 us a step even when they return
-// at once and sort everything when they do not.  Collapsing gases, us a step,
-// end of step / launches: 5,000 particles 40 / 70 (83% of the steps re-sort),
-// 100,000 112 / 186 (98%), 1,000,000 940 / 1,651 (100%, a few movers each).
-// With more movers what they shift grows, the sooner against a whole sort the
-// smaller the simulation: 133 / 191 at 25 movers and 275 / 191 at 125 of
-// 100,000, 390 / 488 at 75 of 300,000, 1,356 / 1,652 at 250 of 1,000,000.  Up
-// to SMALL_NP particles rewriting everything in one workgroup still costs
-// less than the launches (20,000: 75 / 88).
-constexpr double MOVERS_PER_SQRT_NP = 0.27, MOVERS_SMALL = 1024.0;
-constexpr uint32_t SMALL_NP = 32768;
-
-void choose_sort_placement(sph_ctx* c) {
-    if (c->sort_mode != 2) {
-        c->resort_at_end = c->sort_mode == 1;
-        return;
-    }
-    // A batch re-sorts each simulation in its own workgroup, in parallel,
-    // which beats a batch-wide sort whenever any simulation changes.
-    if (c->sims.size() > 1) {
-        c->resort_at_end = true;
-        return;
-    }
-    if (!c->sample_pending || !c->loop_sample) return;
-    if (hipEventQuery(c->sample_ev) != hipSuccess) return;
-    c->sample_pending = false;
-    const DevLoop& L = c->loop_sample[0];
-    const uint32_t sorts = L.sorts - (uint32_t)c->sample_sorts0;
-    const uint32_t moved = L.moved - c->sample_moved0;
-    const uint32_t np = c->sims[0].h.np;
-    const double limit = np > SMALL_NP ? MOVERS_PER_SQRT_NP * sqrt((double)np) : MOVERS_SMALL;
-    if (L.iter - c->sample_iter0 >= 20)
-        c->resort_at_end = (double)moved <= limit * (double)std::max(sorts, 1u);
-    c->sample_iter0 = L.iter;
-    c->sample_sorts0 = L.sorts;
-    c->sample_moved0 = L.moved;
-}
-
-void sample_loop(sph_ctx* c) {
-    if (c->sort_mode != 2 || c->sims.size() > 1 || !c->loop_sample || c->sample_pending) return;
-    if (hipMemcpyAsync(c->loop_sample, c->A.loop, sizeof(DevLoop), hipMemcpyDeviceToHost,
-                       c->stream) != hipSuccess ||
-        hipEventRecord(c->sample_ev, c->stream) != hipSuccess) {
-        (void)hipGetLastError();
-        return;
-    }
-    c->sample_pending = true;
-}
-
-int set_loop_flag(sph_ctx* c, int sim, uint32_t DevLoop::*flag);
-
 // How a step's kernels run.
 struct StepForm {
     int lanes;      // work-items per particle in the contact pass
@@ -1155,6 +1100,66 @@ StepForm step_form(const sph_ctx* c) {
     }
     return f;
 }
+
+// Re-sort placement for the steps about to be enqueued.  In automatic mode
+// the choice follows what a re-sort rewrites (DevLoop::shifted) over the
+// previous sph_step call, read from an asynchronous copy of the loop counters
+// (no synchronisation).  The end-of-step workgroup pays for each place that
+// the movers shift: 2.7 ns where the copies stay stale, 9 ns where they follow
+// (the two-kernel step); the sort launches sort everything, and cost a step
+// of 18 us and more when there is nothing to sort.  Gases (a few movers a step
+// in every direction) and falling lattices (whole layers shift), us a step, the
+// part rewritten, end of step / launches: 15,000 particles 4% 30 / 64, 17%
+// 43 / 66, 39% 81 / 69; 40,000 6% 49 / 98, 21% 75 / 100, 51% 128 / 99; 100,000
+// 4% 81 / 148, 11% 103 / 149, 39% 179 / 151, 60% 312 / 185; 200,000 14%
+// 191 / 252, 45% 417 / 256; 1,000,000 9% 883 / 1,318, 21% 1,203 / 1,320, 67%
+// 3,784 / 1,346.  The movers alone do not tell it: 49 of 40,000 rewrite 21% in
+// a gas and 51% in a lattice.
+void choose_sort_placement(sph_ctx* c) {
+    if (c->sort_mode != 2) {
+        c->resort_at_end = c->sort_mode == 1;
+        return;
+    }
+    // A batch re-sorts each simulation in its own workgroup, in parallel,
+    // which beats a batch-wide sort whenever any simulation changes.
+    if (c->sims.size() > 1) {
+        c->resort_at_end = true;
+        return;
+    }
+    if (!c->sample_pending || !c->loop_sample) return;
+    if (hipEventQuery(c->sample_ev) != hipSuccess) return;
+    c->sample_pending = false;
+    const DevLoop& L = c->loop_sample[0];
+    const double steps = (double)(L.iter - c->sample_iter0);
+    const double sorts = (double)(L.sorts - (uint32_t)c->sample_sorts0);
+    const uint32_t shifted = L.shifted - c->sample_shifted0;
+    const uint32_t measured = L.measured - c->sample_measured0;
+    if (steps >= 20.0) {
+        const double np = c->sims[0].h.np;
+        const double places = measured ? np * shifted / 1024.0 / measured : np;
+        // What a re-sort at the end of the step costs more than the launches.
+        const double more = step_form(c).fused ? 9.0e-3 * (places - 4200.0)
+                                               : 2.7e-3 * (places - (4000.0 + 0.23 * np));
+        c->resort_at_end = sorts * more <= (steps - sorts) * 18.0;
+    }
+    c->sample_iter0 = L.iter;
+    c->sample_sorts0 = L.sorts;
+    c->sample_shifted0 = L.shifted;
+    c->sample_measured0 = L.measured;
+}
+
+void sample_loop(sph_ctx* c) {
+    if (c->sort_mode != 2 || c->sims.size() > 1 || !c->loop_sample || c->sample_pending) return;
+    if (hipMemcpyAsync(c->loop_sample, c->A.loop, sizeof(DevLoop), hipMemcpyDeviceToHost,
+                       c->stream) != hipSuccess ||
+        hipEventRecord(c->sample_ev, c->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    c->sample_pending = true;
+}
+
+int set_loop_flag(sph_ctx* c, int sim, uint32_t DevLoop::*flag);
 
 int enqueue_step(sph_ctx* c) {
     const DevArrays& A = c->A;
@@ -1237,8 +1242,10 @@ int enqueue_step(sph_ctx* c) {
     }
     const bool resort = hash_in_integrate && c->resort_at_end;
     pr.begin("walls");
-    HIPCHK(c, launch_walls(A, !resort ? 0 : form.fused ? 2 : 1, fused && form.partials ? 1 : 0,
-                           c->passes, c->radix_bits, c->sorted_bits, s), "walls");
+    const int place = resort ? (form.fused ? 2 : 1)
+                             : hash_in_integrate && c->sort_mode == 2 ? -1 : 0;
+    HIPCHK(c, launch_walls(A, place, fused && form.partials ? 1 : 0, c->passes, c->radix_bits,
+                           c->sorted_bits, s), "walls");
     pr.end();
     c->copies_fresh = !resort || form.fused;
     c->prev_walls_resorted = resort;

@@ -423,3 +423,32 @@ def test_overlap_lists_of_many(n):
     with engine.Context(image) as ctx:
         pa, da = ctx.find_overlaps()
         assert numpy.array_equal(pa, pb) and numpy.array_equal(da, db)
+
+
+# The automatic re-sort placement: a falling lattice, whose movers are few but
+# shift whole layers of the order at every step, is sorted by the launches; a
+# bed whose movers shift little is re-sorted by the walls kernel.  The launches
+# measure what the other placement would rewrite, and change nothing.
+@pytest.mark.parametrize("n,speed,launched", [(60000, 0.0, True), (40000, 0.05, False)])
+def test_resort_placement_follows_what_is_rewritten(n, speed, launched):
+    rng = numpy.random.default_rng(n)
+    s = cases.lattice_bed(n, 4, 0.01, 0.1)
+    if not launched:
+        s.radius *= 0.4
+        s.g[:] = 0.0
+        s.vel[:, :3] = rng.normal(0.0, speed, (n, 3))
+        s.fixvel[:] = 0.0
+    image = s.tobytes()
+    fields = ("perm", "cellid", "contacts", "x", "vel", "force")
+    with engine.Context(image) as ctx, engine.Context(image) as other:
+        other.set_scalar("sort_mode", 0 if not launched else 1)
+        for _ in range(8):
+            ctx.step(100)
+            other.step(100)
+        ctx.profile(True)
+        ctx.step(20)
+        other.step(20)
+        assert ("sort" in ctx.profile_report()) == launched
+        assert ctx.scalar("sorts") > 100
+        for f in fields:
+            assert numpy.array_equal(ctx.get(f), other.get(f)), f
