@@ -1841,48 +1841,43 @@ int sph_run(sph_ctx* c, const char* out_dir, const char* sid) {
     return SPH_OK;
 }
 
-// The order (global keys, batch indices) the last step of simulation `sim`
-// used, when that step ended by re-sorting for the next one.
-static int previous_order(sph_ctx* c, int sim, const DevLoop& L, std::vector<uint32_t>& key,
-                          std::vector<uint32_t>& perm) {
+// One array (of global keys, or of batch indices: `keys`) of the order the last
+// step of simulation `sim` used, when that step ended by re-sorting for the
+// next one, into dst (np words).
+static int previous_order(sph_ctx* c, int sim, const DevLoop& L, bool keys, uint32_t* dst) {
     const Sim& S = c->sims[sim];
     const size_t np = S.h.np, b0 = S.P.base;
-    const bool full = L.resorted_last == RESORTED_FULL;
-    key.resize(np);
-    perm.resize(np);
-    int rc = d2h(c, key.data(), (full ? c->A.skey_bk : c->A.skey) + b0, np * 4);
-    if (!rc) rc = d2h(c, perm.data(), (full ? c->A.perm_bk : c->A.perm) + b0, np * 4);
-    if (rc || full) return rc;
+    if (L.resorted_last == RESORTED_FULL)
+        return d2h(c, dst, (keys ? c->A.skey_bk : c->A.perm_bk) + b0, np * 4);
     // Undo the merge: take the movers out of their new places (ascending in
     // the records) and put them back at their old ones.
+    std::vector<uint32_t> now(np);
     std::vector<uint4> mv(L.nmv_last);
-    rc = d2h(c, mv.data(), c->A.mv_last + (size_t)sim * MV_CAP, mv.size() * sizeof(uint4));
+    int rc = d2h(c, now.data(), (keys ? c->A.skey : c->A.perm) + b0, np * 4);
+    if (!rc)
+        rc = d2h(c, mv.data(), c->A.mv_last + (size_t)sim * MV_CAP, mv.size() * sizeof(uint4));
     if (rc) return rc;
-    std::vector<uint32_t> k0, p0;
-    k0.reserve(np);
-    p0.reserve(np);
-    size_t e = 0;
-    for (size_t j = 0; j < np; ++j) {
-        if (e < mv.size() && mv[e].w == j) {
-            ++e;
-            continue;
-        }
-        k0.push_back(key[j]);
-        p0.push_back(perm[j]);
+    // (A mover is a particle, and the padding lies behind all of them.)
+    for (const uint4& m : mv)
+        if (m.z >= np || m.w >= np) return fail(c, SPH_E_DEVICE, "bad record of a re-sort");
+    uint32_t* end = now.data();
+    size_t at = 0;
+    for (const uint4& m : mv) {
+        memmove(end, now.data() + at, (m.w - at) * 4);
+        end += m.w - at;
+        at = (size_t)m.w + 1;
     }
+    memmove(end, now.data() + at, (np - at) * 4);
     std::sort(mv.begin(), mv.end(), [](const uint4& x, const uint4& y) { return x.z < y.z; });
-    size_t n = 0, d = 0;
-    for (size_t i = 0; i < np; ++i) {
-        if (d < mv.size() && mv[d].z == i) {
-            key[i] = mv[d].y;
-            perm[i] = mv[d].x;
-            ++d;
-        } else {
-            key[i] = k0[n];
-            perm[i] = p0[n];
-            ++n;
-        }
+    const uint32_t* rest = now.data();
+    at = 0;
+    for (const uint4& m : mv) {
+        memcpy(dst + at, rest, (m.z - at) * 4);
+        rest += m.z - at;
+        dst[m.z] = keys ? m.y : m.x;
+        at = (size_t)m.z + 1;
     }
+    memcpy(dst + at, rest, (np - at) * 4);
     return SPH_OK;
 }
 
@@ -1983,23 +1978,25 @@ int sph_get_field_sim(sph_ctx* c, int sim, int f, void* dst, size_t bytes) {
                     if (!range || w[i] != 0xffffffffu) w[i] -= base;
                 return SPH_OK;
             }
-            std::vector<uint32_t> key, perm;
-            rc = previous_order(c, sim, L, key, perm);
+            if (f == SPH_F_CELLID || f == SPH_F_PERM) {
+                const uint32_t base = f == SPH_F_CELLID ? S.P.cell_base : (uint32_t)b0;
+                rc = previous_order(c, sim, L, f == SPH_F_CELLID, w);
+                for (size_t i = 0; !rc && i < np; ++i) w[i] -= base;
+                return rc;
+            }
+            // The ranges of the order's keys (the ends of empty cells are not
+            // meaningful).
+            std::vector<uint32_t> key(np);
+            rc = previous_order(c, sim, L, true, key.data());
             if (rc) return rc;
-            if (f == SPH_F_CELLID)
-                for (size_t i = 0; i < np; ++i) w[i] = key[i] - S.P.cell_base;
-            if (f == SPH_F_PERM)
-                for (size_t i = 0; i < np; ++i) w[i] = perm[i] - (uint32_t)b0;
-            if (f == SPH_F_CELLSTART || f == SPH_F_CELLEND) {
-                // The ranges of the order's keys (the ends of empty cells
-                // are not meaningful).
-                for (size_t i = 0; i < S.P.ncells; ++i) w[i] = 0xffffffffu;
-                for (size_t i = 0; i < np; ++i) {
-                    const uint32_t k = key[i] - S.P.cell_base;
-                    if (k >= S.P.ncells) continue;
-                    if (f == SPH_F_CELLEND) w[k] = (uint32_t)i + 1u;
-                    else if (w[k] == 0xffffffffu) w[k] = (uint32_t)i;
-                }
+            memset(w, 0xff, bytes);
+            for (size_t i = 0; i < np;) {
+                const uint32_t k = key[i];
+                size_t e = i + 1;
+                while (e < np && key[e] == k) ++e;
+                if (k - S.P.cell_base < S.P.ncells)
+                    w[k - S.P.cell_base] = (uint32_t)(f == SPH_F_CELLEND ? e : i);
+                i = e;
             }
             return SPH_OK;
         }
